@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void k_write_tris(uint32_t n, const uint32_t* 
     plane[p] = plane_u[t];
     TriRest r;
     r.sv = sv_u[t]; r.ev = ev_u[t];
-    r.meta = make_uint2(t, bytes[t]); r.pad = make_uint2(0u, 0u);
+    r.meta = make_uint2(t, bytes[t]); r.axes = srlnp_axes_code((int)bytes[t]); r.pad = 0u;
     rest[p] = r;
     plo[p] = blo_u[t]; phi[p] = bhi_u[t];
 }
@@ -309,11 +309,12 @@ __global__ void k_ray_queue_reset(unsigned long long* q) { if (threadIdx.x == 0)
 template <int STACK>
 __global__ __launch_bounds__(256) void k_trace_closest(ColliderView c, const float4* __restrict__ ro, const float4* __restrict__ rd,
                                                        uint32_t n, int4* __restrict__ hits, uint8_t* __restrict__ front,
-                                                       uint32_t* __restrict__ overflow, unsigned long long* __restrict__ queue)
+                                                       unsigned long long* __restrict__ queue)
 {
     __shared__ int32_t stk[STACK * 256];
     const uint32_t lane = threadIdx.x & 63u;
-    bool busy = false, ok = true;
+    const LaneStack ls(stk + threadIdx.x, 256);
+    bool busy = false;
     bool done = false;              // the queue is empty (wave-uniform)
     uint32_t ray = 0;
     TraceState S;
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(256) void k_trace_closest(ColliderView c, const flo
             if (!busy && q0 < n && rank < n - q0) {
                 ray = (uint32_t)q0 + rank;
                 const float4 a = ro[ray], b = rd[ray];
-                if (trace_begin(S, c, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w)) busy = true;
+                if (trace_begin(S, c, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, ls)) busy = true;
                 else {
                     hits[ray] = make_int4(-1, 0, 0, 0);
                     if (front) front[ray] = 0;
@@ -341,13 +342,13 @@ __global__ __launch_bounds__(256) void k_trace_closest(ColliderView c, const flo
         if (!bm) break;             // queue empty and nothing in flight
         if (!busy) continue;
         const uint32_t yield_at = done ? 0u : 64u - kRefill;
-        if (!trace_resume<STACK>(S, NoFilter(), c, stk + threadIdx.x, 256, yield_at, ok)) continue;
+        if (!trace_resume<STACK>(S, NoFilter(), c, ls, yield_at)) continue;
         busy = false;
-        hits[ray] = S.bi >= 0 ? make_int4(S.bi, __float_as_int(S.best), __float_as_int(S.bu), __float_as_int(S.bv))
-                              : make_int4(-1, 0, 0, 0);
-        if (front) front[ray] = (S.bi >= 0 && S.bf) ? 1 : 0;
+        TraceResult r;
+        trace_finish(S, c, r);
+        hits[ray] = r.tri >= 0 ? make_int4(r.tri, __float_as_int(r.t), __float_as_int(r.u), __float_as_int(r.v)) : make_int4(-1, 0, 0, 0);
+        if (front) front[ray] = (r.tri >= 0 && r.front) ? 1 : 0;
     }
-    if (!ok && overflow) atomicOr(overflow, 1u);
 }
 
 template <int STACK>
@@ -368,15 +369,14 @@ __global__ __launch_bounds__(256) void k_trace_stats(ColliderView c, const float
 template <int STACK>
 __global__ __launch_bounds__(256) void k_trace_full(ColliderView c, const float4* __restrict__ ro, const float4* __restrict__ rd,
                                                     uint32_t n, int4* __restrict__ hits, float4* __restrict__ planes,
-                                                    uint8_t* __restrict__ front, uint32_t* __restrict__ overflow)
+                                                    uint8_t* __restrict__ front)
 {
     __shared__ int32_t stk[STACK * 256];
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const float4 a = ro[i], b = rd[i];
     TraceResult r; uint32_t nv = 0, nt = 0;
-    bool ok = trace_closest<STACK, false>(NoFilter(), c, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, stk + threadIdx.x, 256, r, nv, nt);
-    if (!ok) atomicOr(overflow, 1u);
+    trace_closest<STACK, false>(NoFilter(), c, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, stk + threadIdx.x, 256, r, nv, nt);
     if (r.tri >= 0) {
         hits[i] = make_int4(r.tri, __float_as_int(r.t), __float_as_int(r.u), __float_as_int(r.v));
         planes[i] = c.plane[r.slot];
@@ -694,6 +694,34 @@ static int read_tree_file(const char* path, const uint8_t mesh_hash[20], uint32_
     return LSG_OK;
 }
 
+// whether a stored 4-wide tree is one the traversal can walk: parents before their children
+// (so no cycles), refs within the tree and the triangles, and never more stack entries
+// than stated -- the traversal does not check its stack
+static bool tree4_walkable(const Node4* nodes, uint32_t n4, int32_t root4, uint32_t nvalid, uint32_t stack_need)
+{
+    auto leaf_ok = [&](int32_t r) { return (uint64_t)leaf_start(r) + leaf_count(r) <= nvalid; };
+    if (root4 < 0) return n4 == 0 && leaf_ok(root4);
+    if (!n4) return !nvalid;
+    if (root4 != 0) return false;
+    std::vector<uint32_t> held(n4, 0);                // entries on the stack when a node is visited, at most
+    for (uint32_t i = 0; i < n4; i++) {
+        int32_t r[4];
+        memcpy(r, &nodes[i].q[6], sizeof r);
+        uint32_t m = 0;
+        for (int32_t c : r) {
+            if (c == kNoChild) continue;
+            m++;
+            if (c < 0 ? !leaf_ok(c) : ((uint32_t)c <= i || (uint32_t)c >= n4)) return false;
+        }
+        if (!m) return false;
+        const uint32_t h = held[i] + m - 1;
+        if (h > stack_need) return false;
+        for (int32_t c : r)
+            if (c >= 0 && c != kNoChild && held[c] < h) held[c] = h;
+    }
+    return true;
+}
+
 static int load_from_file(const float* verts, uint32_t nv, const uint32_t* idx, uint32_t nt, const uint8_t hash[20], const char* path,
                           uint32_t want_leaf, uint32_t want_flags, lsg_collider** out)
 {
@@ -710,6 +738,8 @@ static int load_from_file(const float* verts, uint32_t nv, const uint32_t* idx, 
         if (order[i] >= nt) return fail(LSG_ERR_INVALID, "tree file %s: leaf order names triangle %u", path, order[i]);
     const Node* nodes = (const Node*)(payload.data() + 4ull * h.nvalid);
     const Node4* nodes4 = (const Node4*)(payload.data() + 4ull * h.nvalid + sizeof(Node) * (uint64_t)h.nnodes);
+    if (!tree4_walkable(nodes4, h.nnodes4, h.root4, h.nvalid, h.stack_need))
+        return fail(LSG_ERR_INVALID, "tree file %s: its 4-wide tree has refs out of range or needs more stack than stated", path);
     lsg_collider* c = new (std::nothrow) lsg_collider;
     if (!c) return fail(LSG_ERR_OOM, "lsg_collider_load: host allocation failed");
     if ((st = load_tree(c->impl, verts, nv, idx, nt, h, order, nodes, nodes4))) { free_impl(c->impl); delete c; return st; }
@@ -902,9 +932,8 @@ int lsg_collider_intersect_device(const lsg_collider* c, const void* ro, const v
     if (!c || (!n)) return c ? LSG_OK : fail(LSG_ERR_INVALID, "lsg_collider_intersect_device: null collider");
     if (!ro || !rd || !hits) return fail(LSG_ERR_INVALID, "lsg_collider_intersect_device: null buffer");
     const ColliderImpl& C = c->impl;
-    int stack = stack_size_for_depth(C.depth);
+    const int stack = traversal_stack(C);
     if (!stack) return fail(LSG_ERR_LIMIT, "tree too deep");
-    uint32_t* d_over = nullptr;   // stack >= depth+1 by construction; the kernel guard only prevents overrun
     hipStream_t s = (hipStream_t)stream;
     // a counter of this collider's ring (launches in flight on one collider take different
     // ones), zeroed on the launch's stream; waves enough to fill every CU at 4 per SIMD
@@ -921,9 +950,9 @@ int lsg_collider_intersect_device(const lsg_collider* c, const void* ro, const v
     const unsigned resident = (unsigned)cus * (unsigned)(stack <= 32 ? per32 : per64);
     const unsigned nb = std::max(1u, std::min(blocks(n, 256u * 4u), resident));
     if (stack <= 32)
-        k_trace_closest<32><<<nb, 256, 0, s>>>(C.view(), (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, d_over, q);
+        k_trace_closest<32><<<nb, 256, 0, s>>>(C.view(), (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, q);
     else
-        k_trace_closest<64><<<nb, 256, 0, s>>>(C.view(), (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, d_over, q);
+        k_trace_closest<64><<<nb, 256, 0, s>>>(C.view(), (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, q);
     LSG_HIP(hipGetLastError());
     return LSG_OK;
 }
@@ -936,7 +965,7 @@ int lsg_collider_trace_stats(const lsg_collider* c, const void* ro, const void* 
     LSG_HIP(hipMalloc(&d_cnt, 16));
     LSG_HIP(hipMemset(d_cnt, 0, 16));
     if (n) {
-        if (stack_size_for_depth(C.depth) <= 32)
+        if (traversal_stack(C) <= 32)
             k_trace_stats<32><<<blocks(n), 256>>>(C.view(), (const float4*)ro, (const float4*)rd, n, d_cnt);
         else
             k_trace_stats<64><<<blocks(n), 256>>>(C.view(), (const float4*)ro, (const float4*)rd, n, d_cnt);
@@ -966,29 +995,26 @@ int lsg_collider_intersect_rrrays(const lsg_collider* c, void* rays, uint32_t n,
         ho[i] = make_float4(o[0], o[1], o[2], mn);
         hd[i] = make_float4(d[0], d[1], d[2], mx);
     }
-    float4 *d_o = nullptr, *d_d = nullptr, *d_pl = nullptr; int4* d_h = nullptr; uint8_t* d_f = nullptr; uint32_t* d_over = nullptr;
-    auto cleanup = [&]() { dfree(d_o); dfree(d_d); dfree(d_pl); dfree(d_h); dfree(d_f); dfree(d_over); };
+    float4 *d_o = nullptr, *d_d = nullptr, *d_pl = nullptr; int4* d_h = nullptr; uint8_t* d_f = nullptr;
+    auto cleanup = [&]() { dfree(d_o); dfree(d_d); dfree(d_pl); dfree(d_h); dfree(d_f); };
     int st;
 #define CK(x) do { if ((st = (x))) { cleanup(); return st; } } while (0)
 #define CKH(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { cleanup(); return hip_fail(e_, #x, __LINE__); } } while (0)
-    CK(dalloc(&d_o, n)); CK(dalloc(&d_d, n)); CK(dalloc(&d_pl, n)); CK(dalloc(&d_h, n)); CK(dalloc(&d_f, n)); CK(dalloc(&d_over, 1));
+    CK(dalloc(&d_o, n)); CK(dalloc(&d_d, n)); CK(dalloc(&d_pl, n)); CK(dalloc(&d_h, n)); CK(dalloc(&d_f, n));
     CKH(hipMemcpy(d_o, ho.data(), 16 * (size_t)n, hipMemcpyHostToDevice));
     CKH(hipMemcpy(d_d, hd.data(), 16 * (size_t)n, hipMemcpyHostToDevice));
-    CKH(hipMemset(d_over, 0, 4));
-    if (stack_size_for_depth(C.depth) <= 32)
-        k_trace_full<32><<<blocks(n), 256>>>(C.view(), d_o, d_d, n, d_h, d_pl, d_f, d_over);
+    if (traversal_stack(C) <= 32)
+        k_trace_full<32><<<blocks(n), 256>>>(C.view(), d_o, d_d, n, d_h, d_pl, d_f);
     else
-        k_trace_full<64><<<blocks(n), 256>>>(C.view(), d_o, d_d, n, d_h, d_pl, d_f, d_over);
+        k_trace_full<64><<<blocks(n), 256>>>(C.view(), d_o, d_d, n, d_h, d_pl, d_f);
     CKH(hipGetLastError());
-    std::vector<int4> hh(n); std::vector<float4> hp(n); std::vector<uint8_t> hf(n); uint32_t over = 0;
+    std::vector<int4> hh(n); std::vector<float4> hp(n); std::vector<uint8_t> hf(n);
     CKH(hipMemcpy(hh.data(), d_h, 16 * (size_t)n, hipMemcpyDeviceToHost));
     CKH(hipMemcpy(hp.data(), d_pl, 16 * (size_t)n, hipMemcpyDeviceToHost));
     CKH(hipMemcpy(hf.data(), d_f, n, hipMemcpyDeviceToHost));
-    CKH(hipMemcpy(&over, d_over, 4, hipMemcpyDeviceToHost));
     cleanup();
 #undef CK
 #undef CKH
-    if (over) return fail(LSG_ERR_LIMIT, "traversal stack overflow");
     uint32_t hitsn = 0;
     for (uint32_t i = 0; i < n; i++) {
         uint8_t* r = R + (size_t)i * LSG_RRRAY_SIZE;

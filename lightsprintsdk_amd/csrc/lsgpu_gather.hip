@@ -132,9 +132,13 @@ struct GatherFilterT {
     {
         const uint32_t* si = idx + 3 * (size_t)shooter;
         const uint32_t* hi = idx + 3 * (size_t)tri;
+        // (rolled: unrolled, its eighteen coordinates in flight set the register peak of every
+        // traversal, for a test that only hits within 1000 rayLengthMin reach)
+#pragma unroll 1
         for (int i = 0; i < 3; i++) {
             const float* hv = verts + 3 * (size_t)hi[i];
             bool eq = false;
+#pragma unroll 1
             for (int k = 0; k < 3; k++) {
                 const float* sv = verts + 3 * (size_t)si[k];
                 eq |= (hv[0] == sv[0]) & (hv[1] == sv[1]) & (hv[2] == sv[2]);
@@ -184,6 +188,19 @@ __device__ inline GatherFilterT<(FEAT & kFeatMats) != 0> gather_filter(const Gat
         f.qinterp = mode == 0 ? 0u : A.quality / 10;
     }
     return f;
+}
+
+// light li, which every lane of a batch shades at once: read through the constant address
+// space, so that it sits in scalar registers during the shadow ray
+__device__ inline lsg_light light_at(const GatherArgs& A, uint32_t li)
+{
+    typedef const __attribute__((address_space(4))) uint32_t* cptr;
+    const cptr w = (cptr)(uintptr_t)A.lights + li * (sizeof(lsg_light) / 4);
+    uint32_t t[sizeof(lsg_light) / 4];
+    for (uint32_t k = 0; k < sizeof(lsg_light) / 4; k++) t[k] = w[k];
+    lsg_light L;
+    __builtin_memcpy(&L, t, sizeof L);
+    return L;
 }
 
 // The shooter of subtexel j: seeded jitter -> origin o on the subtexel's triangle tri,
@@ -422,7 +439,7 @@ __device__ inline float4 hit_exitance(const SceneView& S, int tri, bool front, c
     float u = 0.f, v = 0.f;
     if (ind || point) {
         const TriRest* tr = S.col.rest + S.slot[tri];
-        srlnp_test(tr->sv, tr->ev, (int)tr->meta.y, o, d, t, u, v);
+        srlnp_hit(tr->sv, tr->ev, tr->axes, o, d, t, u, v);
     }
     const float w = 1 - u - v;
     float ix = 0.f, iy = 0.f, iz = 0.f, ax = 0.f, ay = 0.f, az = 0.f;
@@ -748,7 +765,7 @@ __device__ void gather_texel(const GatherArgs& A, uint32_t ti, uint32_t wlane, i
                 }
                 auto flt = gather_filter<FEAT>(A, tri, near_t, 1, rug_below);
                 for (uint32_t li = 0; li < nl; li++) {
-                    const lsg_light L = A.lights[li];
+                    const lsg_light L = light_at(A, li);
                     float dx, dy, dz;
                     if (L.type == 1) { dx = -L.direction[0]; dy = -L.direction[1]; dz = -L.direction[2]; }
                     else { dx = L.position[0] - o.x; dy = L.position[1] - o.y; dz = L.position[2] - o.z; }
@@ -831,7 +848,7 @@ __device__ void gather_texel(const GatherArgs& A, uint32_t ti, uint32_t wlane, i
             const float3 d = make_float3(nx * cosa + tx * x + bx * y, ny * cosa + ty * x + by * y, nz * cosa + tz * x + bz * y);
             TraceResult r;
             uint32_t nv_ = 0, nt_ = 0;
-            trace_closest<STACK, STATS>(flt, A.sc.col, o, d, A.tmin, A.locality, mystk, stride, r, nv_, nt_);
+            trace_closest<STACK, STATS, decltype(flt)>(flt, A.sc.col, o, d, A.tmin, A.locality, mystk, stride, r, nv_, nt_);
             if (STATS) { stH[0]++; stH[1] += nv_; stH[2] += nt_; }
             // a hit reads the exitance of the side it sees; a ray that leaves the scene
             // returns environment * multiplier, or nothing (pathtracer.cpp:156-173)
@@ -1088,7 +1105,7 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
                 shooter_cached(A, ts, sj, key, shooter_base + s, subc, o, nx, ny, nz, tri);
                 auto flt = gather_filter<FEAT>(A, tri, near_t, 1, rug_below);
                 for (uint32_t li = 0; li < nl; li++) {
-                    const lsg_light L = A.lights[li];
+                    const lsg_light L = light_at(A, li);
                     float dx, dy, dz;
                     if (L.type == 1) { dx = -L.direction[0]; dy = -L.direction[1]; dz = -L.direction[2]; }
                     else { dx = L.position[0] - o.x; dy = L.position[1] - o.y; dz = L.position[2] - o.z; }
@@ -1101,8 +1118,7 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
                     if (L.cast_shadows) {
                         TraceResult r;
                         uint32_t nv_ = 0, nt_ = 0;
-                        // min/max visit: this kernel keeps a hemisphere ray's state alongside
-                        trace_closest<STACK, false, decltype(flt), false, false>(flt, A.sc.col, o, make_float3(dx, dy, dz), A.tmin, dsz, mystk, stride, r, nv_, nt_);
+                        trace_closest<STACK, false, decltype(flt), false>(flt, A.sc.col, o, make_float3(dx, dy, dz), A.tmin, dsz, mystk, stride, r, nv_, nt_);
                         blocked = r.tri >= 0; bt = r.t;
                     }
                     if (!blocked) {
@@ -1133,7 +1149,8 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
             perm = perm_prepare(pscr, f0, n, lane, filler);
         }
         uint32_t next = 0;                         // next shooter to hand out (wave-uniform)
-        bool busy = false, ok = true;
+        bool busy = false;
+        const LaneStack ls(mystk, stride);
         uint32_t stri = 0;                         // the lane's shooter triangle
         TraceState S;
         for (;;) {
@@ -1223,7 +1240,7 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
                     const float cosa = sqrtf(1 - dist);                          // gather.cpp:125-126
                     const float3 d = make_float3(nx * cosa + tx * x + bx * y, ny * cosa + ty * x + by * y, nz * cosa + tz * x + bz * y);
                     stri = tri;
-                    if (trace_begin(S, A.sc.col, o, d, A.tmin, A.locality)) busy = true;
+                    if (trace_begin(S, A.sc.col, o, d, A.tmin, A.locality, ls)) busy = true;
                     else {
                         // the ray leaves the scene box: environment or nothing (pathtracer.cpp:156-173)
                         if constexpr ((FEAT & kFeatEnv) != 0) {
@@ -1239,12 +1256,14 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
                 const bool refill = next < n && qtail - qhead < 64u;
                 const uint32_t yield_at = refill ? 64u - kGatherRefill : 0u;
                 auto flt = gather_filter<FEAT>(A, stri, near_t, 0, rug_below);
-                if (trace_resume<STACK>(S, flt, A.sc.col, mystk, stride, yield_at, ok)) {
+                if (trace_resume<STACK>(S, flt, A.sc.col, ls, yield_at)) {
                     busy = false;
                     // a hit reads the exitance of the side it sees; a ray that leaves the
                     // scene returns environment * multiplier, or nothing
-                    if (S.bi >= 0) {
-                        const float4 e = hit_exitance<(FEAT & kFeatMats) != 0>(A.sc, S.bi, S.bf, S.o, S.d, S.best, A.quality);
+                    TraceResult r;
+                    trace_finish(S, A.sc.col, r);
+                    if (r.tri >= 0) {
+                        const float4 e = hit_exitance<(FEAT & kFeatMats) != 0>(A.sc, r.tri, r.front, S.o, S.d, S.best, A.quality);
                         hr += e.x; hg += e.y; hb += e.z;
                     } else if constexpr ((FEAT & kFeatEnv) != 0) {
                         const float4 v = env_at(A.sc, S.d);
@@ -1254,7 +1273,8 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
                 }
             }
             // a full light batch runs once no hemisphere ray is in flight
-            if (!__any(busy) && qtail - qhead >= 64u) { light_batch(64u); qhead += 64u; }
+            // (no lane's ray state is live across it: cleared, so that it takes no registers there)
+            if (!__any(busy) && qtail - qhead >= 64u) { light_batch(64u); qhead += 64u; S = TraceState(); }
         }
         while (qtail != qhead) {
             const uint32_t cnt = min(64u, qtail - qhead);
@@ -1347,9 +1367,7 @@ __device__ void gather_texel_lane(const GatherArgs& A, uint32_t ti, int32_t* stk
                 auto flt = gather_filter<FEAT>(A, tri, near_t, 0, rug_below);
                 TraceResult r;
                 uint32_t nv_ = 0, nt_ = 0;
-                // min/max visit: measured faster here (the near/far form raised this kernel
-                // from 109 to 122 VGPRs and the 10M-triangle city's cheap gathers slowed)
-                trace_closest<STACK, false, decltype(flt), true, false>(flt, A.sc.col, o, d, A.tmin, A.locality, stk, stride, r, nv_, nt_);
+                trace_closest<STACK, false, decltype(flt)>(flt, A.sc.col, o, d, A.tmin, A.locality, stk, stride, r, nv_, nt_);
                 if (r.tri >= 0) {
                     const float4 e = hit_exitance<(FEAT & kFeatMats) != 0>(A.sc, r.tri, r.front, o, d, r.t, A.quality);
                     hr += e.x; hg += e.y; hb += e.z;
@@ -1362,7 +1380,7 @@ __device__ void gather_texel_lane(const GatherArgs& A, uint32_t ti, int32_t* stk
             if (doL) {
                 auto flt = gather_filter<FEAT>(A, tri, near_t, 1, rug_below);
                 for (uint32_t li = 0; li < nl; li++) {
-                    const lsg_light L = A.lights[li];
+                    const lsg_light L = light_at(A, li);
                     float dx, dy, dz;
                     if (L.type == 1) { dx = -L.direction[0]; dy = -L.direction[1]; dz = -L.direction[2]; }
                     else { dx = L.position[0] - o.x; dy = L.position[1] - o.y; dz = L.position[2] - o.z; }
@@ -1375,7 +1393,7 @@ __device__ void gather_texel_lane(const GatherArgs& A, uint32_t ti, int32_t* stk
                     if (L.cast_shadows) {
                         TraceResult r;
                         uint32_t nv_ = 0, nt_ = 0;
-                        trace_closest<STACK, false, decltype(flt), false, false>(flt, A.sc.col, o, make_float3(dx, dy, dz), A.tmin, dsz, stk, stride, r, nv_, nt_);
+                        trace_closest<STACK, false, decltype(flt), false>(flt, A.sc.col, o, make_float3(dx, dy, dz), A.tmin, dsz, stk, stride, r, nv_, nt_);
                         blocked = r.tri >= 0; bt = r.t;
                     }
                     if (!blocked) {
@@ -1566,7 +1584,7 @@ int gather_args(lsg_scene* s, const lsg_texel* texels, uint32_t ntexels, const l
                 const lsg_gather_params* p, float* out_rgba, GatherArgs& A, int& stack)
 {
     const ColliderImpl& C = s->impl.col->impl;
-    stack = stack_size_for_depth(C.depth);
+    stack = traversal_stack(C);
     if (!stack) return fail(LSG_ERR_LIMIT, "tree too deep");
     if (!(p->ray_length_min >= 0) || !(p->rug_distance > 0) || !(p->locality > 0))
         return fail(LSG_ERR_INVALID, "gather: ray_length_min >= 0, rug_distance > 0 and locality > 0 required");

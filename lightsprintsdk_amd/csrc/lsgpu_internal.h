@@ -85,25 +85,35 @@ __device__ inline float plane_distance(const float4 n, const float3 o, const flo
     return -ndoto / ndotdir;
 }
 
-// intersect_triangleSRLNP (IntersectBspFast.cpp:189-252) at distance t already in range.
-__device__ inline bool srlnp_test(const float4 sv, const float4 ev, int byte, const float3 o, const float3 d,
-                                  float t, float& u, float& v)
+// intersectByte's projection axes as a test reads them: bits 0-1 = x (y is the axis after
+// it), bits 2-3 = z, bit 4 = degenerate (never hit), so a test selects components without
+// the byte's division by 3
+__host__ __device__ inline uint32_t srlnp_axes_code(int byte)
 {
-    float px = o.x + d.x * t, py = o.y + d.y * t, pz = o.z + d.z * t;   // IntersectLinear.cpp:40-45
     int x, y, z;
     srlnp_axes(byte, x, y, z);
-    float pX = sel3(px, py, pz, x), pY = sel3(px, py, pz, y), pZ = sel3(px, py, pz, z);
+    return (uint32_t)x | (uint32_t)z << 2 | (byte > 8 ? 16u : 0u);
+}
+
+// intersect_triangleSRLNP (IntersectBspFast.cpp:189-252) at distance t already in range.
+__device__ inline bool srlnp_hit(const float4 sv, const float4 ev, uint32_t axes, const float3 o, const float3 d, float t, float& u,
+                                 float& v)
+{
+    const float px = o.x + d.x * t, py = o.y + d.y * t, pz = o.z + d.z * t;   // IntersectLinear.cpp:40-45
+    const uint32_t x = axes & 3u, z = (axes >> 2) & 3u;
+    const bool x0 = x == 0u, x1 = x == 1u;
+    const float pX = x0 ? px : (x1 ? py : pz), pY = x0 ? py : (x1 ? pz : px);
+    const float pZ = z == 0u ? px : (z == 1u ? py : pz);
     v = ((pY - sv.y) * ev.x - (pX - sv.x) * ev.y) * sv.w;
-    if (v < 0 || v > 1) return false;
     u = (pZ - sv.z - ev.z * v) * ev.w;
-    if (u < 0 || u + v > 1) return false;
-    return byte <= 8;
+    return !((v < 0) | (v > 1) | (u < 0) | (u + v > 1) | (axes >= 16u));
 }
 
 // ---- device-side collider view ---------------------------------------------------------
-// The rest of a triangle's test record in leaf order, 48 bytes: projected edge data and
-// (original index, intersectByte), read together once a ray passes the plane test.
-struct alignas(16) TriRest { float4 sv, ev; uint2 meta; uint2 pad; };
+// The rest of a triangle's test record in leaf order, 48 bytes: projected edge data,
+// (original index, intersectByte) and the byte's axes code, read together once a ray
+// passes the plane test.
+struct alignas(16) TriRest { float4 sv, ev; uint2 meta; uint32_t axes, pad; };
 
 struct ColliderView {
     const Node* nodes;
@@ -144,6 +154,14 @@ struct ColliderImpl {
 };
 
 int stack_size_for_depth(uint32_t depth);   // 0 when too deep
+// the traversal kernels' stack (32 or 64 entries, 0 = too deep) for a built tree.  The
+// 32-entry kernels address nodes and triangle records by 32-bit byte offsets, so a tree
+// whose arrays pass 4 GB takes the 64-entry ones.
+inline int traversal_stack(const ColliderImpl& C)
+{
+    const int st = stack_size_for_depth(C.depth);
+    return st == 32 && (C.nnodes4 > (1u << 25) || C.nvalid > (1u << 26)) ? 64 : st;
+}
 
 // ---- device-wide primitives (lsgpu_prim.hip) --------------------------------------------
 // words of scratch scan_exclusive_u32 needs for n values

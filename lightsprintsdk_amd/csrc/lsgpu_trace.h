@@ -25,131 +25,74 @@ struct NoFilter {
     __device__ float clamp(float best) const { return best; }
 };
 
-// One BVH4 node: the four child-box slab tests, then the children that are hit, nearest
-// first.  noi = -o * idir per ray, so each plane distance is one fma: (b - o) * idir =
-// b * idir - o * idir.  The fused form differs from the two-step one by about |o * idir|
+constexpr int32_t kDone = 0x7fffffff;          // never a node index: the ray is finished
+constexpr uint32_t kNoSlot = 0xffffffffu;
+
+// One lane's traversal stack: a column of a workgroup's LDS array, successive entries
+// `step` bytes apart.  top is the LDS byte address of the next free entry.
+typedef __attribute__((address_space(3))) int32_t lds_int;
+struct LaneStack {
+    uint32_t base, first, step;
+    // stk: this lane's first entry; a wave's lanes own 64 consecutive columns or part of them,
+    // so an address below `first` (scalar) is a first entry, whichever lane asks
+    __device__ LaneStack(int32_t* stk, int stride)
+        : base((uint32_t)(uintptr_t)(lds_int*)stk), step(4u * (uint32_t)stride)
+    {
+        first = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + 252u;
+    }
+    // an entry that stays only where keep: written in any case (the slot at top is free by
+    // the stack bound), so no branch
+    __device__ void push_if(uint32_t& top, int32_t r, bool keep) const
+    {
+        *(lds_int*)(uintptr_t)top = r;
+        top += keep ? step : 0u;
+    }
+    __device__ int32_t pop(uint32_t& top) const
+    {
+        if (top <= first) return kDone;
+        top -= step;
+        return *(lds_int*)(uintptr_t)top;
+    }
+};
+
+// Element i of an array.  Trees with the 32-entry stack keep every array below 4 GB
+// (traversal_stack), so their loads take the array's scalar base plus a 32-bit offset,
+// without 64-bit address arithmetic per load.
+template <bool WIDE, class T> __device__ inline T load_at(const void* base, uint32_t i, uint32_t size, uint32_t off)
+{
+    if constexpr (WIDE) return *(const T*)((const char*)base + (size_t)i * size + off);
+    else return *(const T*)((const char*)base + ((size == 48u ? (i + 2u * i) << 4 : i * size) + off));
+}
+
+// (distance, child ref) pairs as one 64-bit float: the distance's bits are the high word, so
+// the doubles order as the distances do (never a NaN: the high word is at most that of
+// binary32 infinity, a finite double; binary64 keeps denormals) and v_min_f64 / v_max_f64,
+// issued at the binary32 rate, move both words of a comparator in two instructions
+// instead of a compare and four selects.
+__device__ inline double pair(float k, int32_t r) { return __hiloint2double(__float_as_int(k), r); }
+__device__ inline void pair_sort(double& a, double& b)
+{
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo; b = hi;
+}
+__device__ inline bool pair_hit(double p) { return __int_as_float(__double2hiint(p)) < __builtin_huge_valf(); }
+
+// max / min of three and of two without the quieting of signalling NaNs that fmaxf's
+// lowering adds for values it cannot trace (box planes and distances are never one)
+__device__ inline float vmax3(float a, float b, float c) { float r; asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
+__device__ inline float vmin3(float a, float b, float c) { float r; asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
+__device__ inline float vmax(float a, float b) { float r; asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ inline float vmin(float a, float b) { float r; asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+
+// what a ray's box tests need: noi = -o * idir, so each plane distance is one fma: (b - o) *
+// idir = b * idir - o * idir.  The fused form differs from the two-step one by about |o * idir|
 // ulp, i.e. |o| * 6e-8 in distance, while every child box is inflated by DELTA_BSP =
 // max|coordinate| * 1e-5; culling stays conservative and the hit, decided only by the
-// triangle test, is unchanged.  The nearest child is returned as the next ref, the
-// others go on the stack farthest first.  No child hit: the next ref is popped.  The
-// tree is collapsed so that the stack never holds more than STACK-1 entries.
-__device__ inline void cswap(float& ka, int32_t& ra, float& kb, int32_t& rb)
-{
-    const bool sw = kb < ka;
-    const float k = sw ? kb : ka; kb = sw ? ka : kb; ka = k;
-    const int32_t r = sw ? rb : ra; rb = sw ? ra : rb; ra = r;
-}
-
-template <int STACK, class Pop, bool ORDERED = true>
-__device__ inline int32_t visit4(const Node4* __restrict__ nodes, int32_t ref, const float3 noi, const float3 idir, float tlo,
-                                 float thi, int32_t* stk, int stride, int& sp, bool& ok, Pop pop)
-{
-    const Node4* np = nodes + ref;
-    float4 tn, tf;
-    // the node's seven 16-byte loads are issued together, before any use: left to itself
-    // the scheduler issues four, waits for them, then the other three (two memory
-    // round trips per node visit)
-    const float4 n0 = np->q[0], n1 = np->q[1], n2 = np->q[2], n3 = np->q[3], n4 = np->q[4], n5 = np->q[5], n6 = np->q[6];
-    __builtin_amdgcn_sched_barrier(0);
-    {
-        const float4 l = n0, h = n1;
-        float a, b;
-        a = __fmaf_rn(l.x, idir.x, noi.x); b = __fmaf_rn(h.x, idir.x, noi.x); tn.x = fminf(a, b); tf.x = fmaxf(a, b);
-        a = __fmaf_rn(l.y, idir.x, noi.x); b = __fmaf_rn(h.y, idir.x, noi.x); tn.y = fminf(a, b); tf.y = fmaxf(a, b);
-        a = __fmaf_rn(l.z, idir.x, noi.x); b = __fmaf_rn(h.z, idir.x, noi.x); tn.z = fminf(a, b); tf.z = fmaxf(a, b);
-        a = __fmaf_rn(l.w, idir.x, noi.x); b = __fmaf_rn(h.w, idir.x, noi.x); tn.w = fminf(a, b); tf.w = fmaxf(a, b);
-    }
-    {
-        const float4 l = n2, h = n3;
-        float a, b;
-        a = __fmaf_rn(l.x, idir.y, noi.y); b = __fmaf_rn(h.x, idir.y, noi.y); tn.x = fmaxf(tn.x, fminf(a, b)); tf.x = fminf(tf.x, fmaxf(a, b));
-        a = __fmaf_rn(l.y, idir.y, noi.y); b = __fmaf_rn(h.y, idir.y, noi.y); tn.y = fmaxf(tn.y, fminf(a, b)); tf.y = fminf(tf.y, fmaxf(a, b));
-        a = __fmaf_rn(l.z, idir.y, noi.y); b = __fmaf_rn(h.z, idir.y, noi.y); tn.z = fmaxf(tn.z, fminf(a, b)); tf.z = fminf(tf.z, fmaxf(a, b));
-        a = __fmaf_rn(l.w, idir.y, noi.y); b = __fmaf_rn(h.w, idir.y, noi.y); tn.w = fmaxf(tn.w, fminf(a, b)); tf.w = fminf(tf.w, fmaxf(a, b));
-    }
-    {
-        const float4 l = n4, h = n5;
-        float a, b;
-        a = __fmaf_rn(l.x, idir.z, noi.z); b = __fmaf_rn(h.x, idir.z, noi.z); tn.x = fmaxf(tn.x, fminf(a, b)); tf.x = fminf(tf.x, fmaxf(a, b));
-        a = __fmaf_rn(l.y, idir.z, noi.z); b = __fmaf_rn(h.y, idir.z, noi.z); tn.y = fmaxf(tn.y, fminf(a, b)); tf.y = fminf(tf.y, fmaxf(a, b));
-        a = __fmaf_rn(l.z, idir.z, noi.z); b = __fmaf_rn(h.z, idir.z, noi.z); tn.z = fmaxf(tn.z, fminf(a, b)); tf.z = fminf(tf.z, fmaxf(a, b));
-        a = __fmaf_rn(l.w, idir.z, noi.z); b = __fmaf_rn(h.w, idir.z, noi.z); tn.w = fmaxf(tn.w, fminf(a, b)); tf.w = fminf(tf.w, fmaxf(a, b));
-    }
-    const float4 rq = n6;
-    int32_t r0 = __float_as_int(rq.x), r1 = __float_as_int(rq.y), r2 = __float_as_int(rq.z), r3 = __float_as_int(rq.w);
-    constexpr float kInf = __builtin_huge_valf();
-    float k0 = fmaxf(tn.x, tlo), k1 = fmaxf(tn.y, tlo), k2 = fmaxf(tn.z, tlo), k3 = fmaxf(tn.w, tlo);
-    k0 = (r0 != kNoChild && k0 <= fminf(tf.x, thi)) ? k0 : kInf;
-    k1 = (r1 != kNoChild && k1 <= fminf(tf.y, thi)) ? k1 : kInf;
-    k2 = (r2 != kNoChild && k2 <= fminf(tf.z, thi)) ? k2 : kInf;
-    k3 = (r3 != kNoChild && k3 <= fminf(tf.w, thi)) ? k3 : kInf;
-    auto push = [&](int32_t r) { if (sp < STACK) stk[(sp++) * stride] = r; else ok = false; };
-    if constexpr (!ORDERED) {
-        // any order: continue with the last hit child in slot order, push the others
-        int32_t nxt = 0;
-        bool have = false;
-        auto take = [&](float k, int32_t r) { if (k < kInf) { if (have) push(nxt); nxt = r; have = true; } };
-        take(k0, r0); take(k1, r1); take(k2, r2); take(k3, r3);
-        return have ? nxt : pop();
-    }
-    cswap(k0, r0, k1, r1); cswap(k2, r2, k3, r3); cswap(k0, r0, k2, r2); cswap(k1, r1, k3, r3); cswap(k1, r1, k2, r2);
-    if (k3 < kInf) push(r3);
-    if (k2 < kInf) push(r2);
-    if (k1 < kInf) push(r1);
-    return k0 < kInf ? r0 : pop();
-}
-
-// visit4 with each child's entry and exit distances from its near and far planes only
-// (same values, about 20 fewer VALU operations per visit, a dozen more registers)
-template <int STACK, class Pop, bool ORDERED = true>
-__device__ inline int32_t visit4_nf(const Node4* __restrict__ nodes, int32_t ref, const float3 noi, const float3 idir, float tlo,
-                                 float thi, int32_t* stk, int stride, int& sp, bool& ok, Pop pop)
-{
-    const Node4* np = nodes + ref;
-    // near and far planes by the signs of the ray direction: lo planes sit at byte
-    // offsets 0/32/64 of the node and hi planes 16 bytes after them, so per axis the lane
-    // loads its near plane first and the far one at the other offset.  near <= far per
-    // axis (fma is monotonic and idir never 0), so these are the min/max of the two plane
-    // distances without computing both; the hoisted offsets cost two adds per visit.
-    const uint32_t ox = idir.x < 0.f ? 16u : 0u, oy = idir.y < 0.f ? 48u : 32u, oz = idir.z < 0.f ? 80u : 64u;
-    const char* nb = (const char*)np;
-    // the node's seven 16-byte loads are issued together, before any use: left to itself
-    // the scheduler issues four, waits for them, then the other three (two memory
-    // round trips per node visit)
-    const float4 nx = *(const float4*)(nb + ox), fx = *(const float4*)(nb + (ox ^ 16u));
-    const float4 ny = *(const float4*)(nb + oy), fy = *(const float4*)(nb + (oy ^ 16u));
-    const float4 nz = *(const float4*)(nb + oz), fz = *(const float4*)(nb + (oz ^ 16u));
-    const float4 n6 = np->q[6];
-    __builtin_amdgcn_sched_barrier(0);
-    auto enter = [&](float x, float y, float z) {
-        return fmaxf(fmaxf(__fmaf_rn(x, idir.x, noi.x), __fmaf_rn(y, idir.y, noi.y)), fmaxf(__fmaf_rn(z, idir.z, noi.z), tlo));
-    };
-    auto leave = [&](float x, float y, float z) {
-        return fminf(fminf(__fmaf_rn(x, idir.x, noi.x), __fmaf_rn(y, idir.y, noi.y)), fminf(__fmaf_rn(z, idir.z, noi.z), thi));
-    };
-    const float4 rq = n6;
-    int32_t r0 = __float_as_int(rq.x), r1 = __float_as_int(rq.y), r2 = __float_as_int(rq.z), r3 = __float_as_int(rq.w);
-    constexpr float kInf = __builtin_huge_valf();
-    float k0 = enter(nx.x, ny.x, nz.x), k1 = enter(nx.y, ny.y, nz.y), k2 = enter(nx.z, ny.z, nz.z), k3 = enter(nx.w, ny.w, nz.w);
-    k0 = (r0 != kNoChild && k0 <= leave(fx.x, fy.x, fz.x)) ? k0 : kInf;
-    k1 = (r1 != kNoChild && k1 <= leave(fx.y, fy.y, fz.y)) ? k1 : kInf;
-    k2 = (r2 != kNoChild && k2 <= leave(fx.z, fy.z, fz.z)) ? k2 : kInf;
-    k3 = (r3 != kNoChild && k3 <= leave(fx.w, fy.w, fz.w)) ? k3 : kInf;
-    auto push = [&](int32_t r) { if (sp < STACK) stk[(sp++) * stride] = r; else ok = false; };
-    if constexpr (!ORDERED) {
-        // any order: continue with the last hit child in slot order, push the others
-        int32_t nxt = 0;
-        bool have = false;
-        auto take = [&](float k, int32_t r) { if (k < kInf) { if (have) push(nxt); nxt = r; have = true; } };
-        take(k0, r0); take(k1, r1); take(k2, r2); take(k3, r3);
-        return have ? nxt : pop();
-    }
-    cswap(k0, r0, k1, r1); cswap(k2, r2, k3, r3); cswap(k0, r0, k2, r2); cswap(k1, r1, k3, r3); cswap(k1, r1, k2, r2);
-    if (k3 < kInf) push(r3);
-    if (k2 < kInf) push(r2);
-    if (k1 < kInf) push(r1);
-    return k0 < kInf ? r0 : pop();
-}
+// triangle test, is unchanged.  near: byte offsets of the
+// axes' near planes in a node, a byte each.
+struct RayBox { float3 idir, noi; uint32_t near; };
 
 __device__ inline float3 safe_inv(float3 d)
 {
@@ -159,10 +102,102 @@ __device__ inline float3 safe_inv(float3 d)
     return make_float3(1.0f / x, 1.0f / y, 1.0f / z);
 }
 
-// Closest accepted hit of one ray.  stk = this lane's first stack slot (LDS),
-// successive slots `stride` ints apart.  Returns false on stack overflow (cannot
-// happen when STACK > tree depth, which the host guarantees).
+__device__ inline RayBox ray_box(const float3 o, const float3 d)
+{
+    RayBox r;
+    r.idir = safe_inv(d);
+    r.noi = make_float3(-o.x * r.idir.x, -o.y * r.idir.y, -o.z * r.idir.z);
+    r.near = (r.idir.x < 0.f ? 16u : 0u) | (r.idir.y < 0.f ? 48u : 32u) << 8 | (r.idir.z < 0.f ? 80u : 64u) << 16;
+    return r;
+}
+
+// One BVH4 node: the four child-box slab tests, then the children that are hit.  The
+// nearest child is returned as the next ref, the others go on the stack farthest first
+// (ORDERED; else any order).  No child hit: the next ref is popped.  The tree is collapsed
+// so that the stack never holds more than STACK-1 entries.
 //
+// Per axis the lane loads its near plane (lo or hi by the direction's sign) and the far
+// one, 16 bytes apart: near <= far (fma is monotonic and idir never 0), so entry and exit
+// are a max3 / min3 of three fmas per child without a min/max pair per axis.
+//
+// Bound by VALU issue together with the L1's tag lookups (a lookup per distinct node and
+// load; SQ and TA counters of a 1024-ray gather over 50k triangles: VALU 78% of issue, TA
+// busy 86%).  Straight-line tests, sorting (distance, ref) pairs as doubles, branch-free
+// pushes and 32-bit offsets issue 39.7e9 instead of 49.7e9 wave instructions per such gather:
+// 89.6 -> 84.9 ms, 1M random rays against 100k triangles 0.718 -> 0.638 ms, a sun-and-sky
+// gather over 132k triangles 27.9 -> 24.3 ms.
+template <bool WIDE, bool ORDERED>
+__device__ inline int32_t visit4(const Node4* __restrict__ nodes, int32_t ref, const RayBox& R, float tlo, float thi,
+                                 const LaneStack& stk, uint32_t& top)
+{
+    const uint32_t n = (uint32_t)ref, ax = R.near & 255u, ay = (R.near >> 8) & 255u, az = R.near >> 16;
+    // the node's seven 16-byte loads are issued together, before any use: left to itself
+    // the scheduler issues four, waits for them, then the other three (two memory
+    // round trips per node visit)
+    const float4 nx = load_at<WIDE, float4>(nodes, n, 128u, ax), fx = load_at<WIDE, float4>(nodes, n, 128u, ax ^ 16u);
+    const float4 ny = load_at<WIDE, float4>(nodes, n, 128u, ay), fy = load_at<WIDE, float4>(nodes, n, 128u, ay ^ 16u);
+    const float4 nz = load_at<WIDE, float4>(nodes, n, 128u, az), fz = load_at<WIDE, float4>(nodes, n, 128u, az ^ 16u);
+    const int4 r = load_at<WIDE, int4>(nodes, n, 128u, 96u);
+    __builtin_amdgcn_sched_barrier(0);
+    auto enter = [&](float x, float y, float z) {
+        return vmax3(__fmaf_rn(x, R.idir.x, R.noi.x), __fmaf_rn(y, R.idir.y, R.noi.y), vmax(__fmaf_rn(z, R.idir.z, R.noi.z), tlo));
+    };
+    auto leave = [&](float x, float y, float z) {
+        return vmin3(__fmaf_rn(x, R.idir.x, R.noi.x), __fmaf_rn(y, R.idir.y, R.noi.y), vmin(__fmaf_rn(z, R.idir.z, R.noi.z), thi));
+    };
+    const float k0 = enter(nx.x, ny.x, nz.x), k1 = enter(nx.y, ny.y, nz.y), k2 = enter(nx.z, ny.z, nz.z), k3 = enter(nx.w, ny.w, nz.w);
+    // (bitwise, so that the tests stay straight-line code)
+    const bool h0 = (r.x != kNoChild) & (k0 <= leave(fx.x, fy.x, fz.x)), h1 = (r.y != kNoChild) & (k1 <= leave(fx.y, fy.y, fz.y));
+    const bool h2 = (r.z != kNoChild) & (k2 <= leave(fx.z, fy.z, fz.z)), h3 = (r.w != kNoChild) & (k3 <= leave(fx.w, fy.w, fz.w));
+    if constexpr (!ORDERED) {
+        // any order: continue with the last hit child in slot order, push the others
+        int32_t nxt = h0 ? r.x : kDone;
+        stk.push_if(top, nxt, h1 & h0);
+        bool have = h0 | h1;
+        nxt = h1 ? r.y : nxt;
+        stk.push_if(top, nxt, h2 & have);
+        have = have | h2;
+        nxt = h2 ? r.z : nxt;
+        stk.push_if(top, nxt, h3 & have);
+        nxt = h3 ? r.w : nxt;
+        return nxt != kDone ? nxt : stk.pop(top);
+    }
+    constexpr float kInf = __builtin_huge_valf();
+    double p0 = pair(h0 ? k0 : kInf, r.x), p1 = pair(h1 ? k1 : kInf, r.y), p2 = pair(h2 ? k2 : kInf, r.z), p3 = pair(h3 ? k3 : kInf, r.w);
+    pair_sort(p0, p1); pair_sort(p2, p3); pair_sort(p0, p2); pair_sort(p1, p3); pair_sort(p1, p2);
+    stk.push_if(top, __double2loint(p3), pair_hit(p3));
+    stk.push_if(top, __double2loint(p2), pair_hit(p2));
+    stk.push_if(top, __double2loint(p1), pair_hit(p1));
+    return pair_hit(p0) ? __double2loint(p0) : stk.pop(top);
+}
+
+// Closest accepted hit of one ray, resumable: trace_begin sets a ray up, trace_resume runs
+// it until it is finished (returns true) or until no more than `yield_at` lanes of the
+// wave are still tracing (returns false, state kept), trace_finish gives its hit.  The
+// state keeps the best hit's leaf-order slot and distance; triangle, side and hitPoint2d
+// are recomputed from the slot's record once per ray, bit-identical to the test's.
+struct TraceState {
+    float3 o, d;
+    RayBox box;
+    float lo, best, bound;
+    int32_t ref, leaf;
+    uint32_t slot, top;
+};
+
+// false when the ray misses the scene box (then it is finished, no hit)
+__device__ inline bool trace_begin(TraceState& S, const ColliderView& c, const float3 o, const float3 d, float rmin, float rmax,
+                                   const LaneStack& stk)
+{
+    float lo, hi;
+    S.slot = kNoSlot;
+    if (!c.nvalid || !ref_box_intersect(c.bmin, c.bmax, o, d, rmin, rmax, lo, hi)) return false;
+    S.o = o; S.d = d;
+    S.box = ray_box(o, d);
+    S.lo = lo; S.best = hi; S.bound = hi;
+    S.ref = c.root4; S.leaf = 0; S.top = stk.base;
+    return true;
+}
+
 // Loop shape: "while-while" with speculative traversal (Aila & Laine, HPG 2009).
 // Lanes descend inner nodes; a lane that reaches a leaf parks it and keeps
 // descending, until every lane of the wave holds a parked leaf; then the wave tests
@@ -173,138 +208,83 @@ __device__ inline float3 safe_inv(float3 d)
 // asks whether a blocker lies below rugDistance and, if not, whether any blocker lies in
 // range; after the first hit its range shrinks below rugDistance and the search there is
 // exhaustive, so the answer does not depend on the order, and the sort is saved.
-// NF: visit4_nf (fewer operations) or visit4 (fewer registers, for callers near the
-// register cap).
-template <int STACK, bool STATS, class Filter, bool ORDERED = true, bool NF = true>
-__device__ inline bool trace_closest(const Filter& flt, const ColliderView& c, const float3 o, const float3 d,
-                                     float rmin, float rmax, int32_t* stk, int stride, TraceResult& res,
-                                     uint32_t& nvis, uint32_t& ntest)
+template <int STACK, bool STATS, class Filter, bool ORDERED, bool YIELD>
+__device__ inline bool trace_run(TraceState& S, const Filter& flt, const ColliderView& c, const LaneStack& stk, uint32_t yield_at,
+                                 uint32_t& nvis, uint32_t& ntest)
 {
-    constexpr int32_t kDone = 0x7fffffff;          // never a node index
-    res.tri = -1;
-    float lo, hi;
-    if (!c.nvalid || !ref_box_intersect(c.bmin, c.bmax, o, d, rmin, rmax, lo, hi)) return true;
-    const float3 idir = safe_inv(d);
-    const float3 noi = make_float3(-o.x * idir.x, -o.y * idir.y, -o.z * idir.z);
-    float best = hi, bound = hi;
-    int bi = -1; float bu = 0.f, bv = 0.f; bool bf = false; uint32_t bslot = 0;
-    int32_t ref = c.root4;         // next node: >= 0 inner, < 0 leaf, kDone finished
-    int32_t leaf = 0;              // parked leaf (< 0) or none (0)
-    int sp = 0;
-    bool ok = true;
-    auto pop = [&]() -> int32_t { return sp ? stk[(--sp) * stride] : kDone; };
-    while (ref != kDone || leaf < 0) {
+    constexpr bool WIDE = STACK > 32;
+    while (S.ref != kDone || S.leaf < 0) {
+        if (YIELD && (uint32_t)__popcll(__ballot(1)) <= yield_at) return false;     // enough lanes are free
         // inner nodes, parking the first leaf met
-        while (ref >= 0 && ref != kDone) {
+        while (S.ref >= 0 && S.ref != kDone) {
             if (STATS) nvis++;
-            if constexpr (NF) ref = visit4_nf<STACK, decltype(pop), ORDERED>(c.nodes4, ref, noi, idir, lo, bound, stk, stride, sp, ok, pop);
-            else ref = visit4<STACK, decltype(pop), ORDERED>(c.nodes4, ref, noi, idir, lo, bound, stk, stride, sp, ok, pop);
-            if (ref < 0 && leaf == 0) { leaf = ref; ref = pop(); }
-            if (!__any(leaf == 0)) break;                // every active lane holds a leaf
+            S.ref = visit4<WIDE, ORDERED>(c.nodes4, S.ref, S.box, S.lo, S.bound, stk, S.top);
+            if (S.ref < 0 && S.leaf == 0) { S.leaf = S.ref; S.ref = stk.pop(S.top); }
+            if (!__any(S.leaf == 0)) break;              // every active lane holds a leaf
         }
         // a leaf reached outside the loop above (the root itself, or a leaf next on
         // the stack while none was parked) is parked here, so every pass progresses
-        if (leaf == 0 && ref < 0) { leaf = ref; ref = pop(); }
+        if (S.leaf == 0 && S.ref < 0) { S.leaf = S.ref; S.ref = stk.pop(S.top); }
         // triangles of the parked leaf, then of leaves met directly on the stack
-        while (leaf < 0) {
-            const uint32_t st = leaf_start(leaf), cnt = leaf_count(leaf);
-            bool stop = false;
-            for (uint32_t k = 0; k < cnt; k++) {
-                const uint32_t p = st + k;
+        while (S.leaf < 0) {
+            const uint32_t st = leaf_start(S.leaf), end = st + leaf_count(S.leaf);
+            S.leaf = 0;
+            for (uint32_t p = st; p < end; p++) {
                 if (STATS) ntest++;
-                const float4 pl = c.plane[p];
+                const float4 pl = load_at<WIDE, float4>(c.plane, p, 16u, 0u);
                 float ndd;
-                const float t = plane_distance(pl, o, d, ndd);
-                if (!(t >= lo && t <= bound)) continue;
-                const TriRest* tr = c.rest + p;
-                const uint2 mt = tr->meta;
-                if (!(bi < 0 || t < best || (int)mt.x < bi)) continue;
+                const float t = plane_distance(pl, S.o, S.d, ndd);
+                if (!(t >= S.lo && t <= S.bound)) continue;
+                // the whole record in one round trip
+                const float4 sv = load_at<WIDE, float4>(c.rest, p, 48u, 0u), ev = load_at<WIDE, float4>(c.rest, p, 48u, 16u);
+                const uint4 mt = load_at<WIDE, uint4>(c.rest, p, 48u, 32u);
+                __builtin_amdgcn_sched_barrier(0);
                 float u, v;
-                if (!srlnp_test(tr->sv, tr->ev, (int)mt.y, o, d, t, u, v)) continue;
-                const bool fr = ndd < 0;
-                if (!flt.accept(mt.x, fr, t, u, v)) continue;
-                best = t; bi = (int)mt.x; bu = u; bv = v; bf = fr; bslot = p;
-                bound = flt.clamp(best);
-                if (flt.done(t)) { stop = true; break; }
+                if (!srlnp_hit(sv, ev, mt.z, S.o, S.d, t, u, v)) continue;
+                // a tie goes to the lower triangle index
+                if (t == S.best && S.slot != kNoSlot && mt.x >= load_at<WIDE, uint32_t>(c.rest, S.slot, 48u, 32u)) continue;
+                if (!flt.accept(mt.x, ndd < 0, t, u, v)) continue;
+                S.best = t; S.slot = p;
+                S.bound = flt.clamp(t);
+                if (flt.done(t)) { S.ref = kDone; break; }
             }
-            if (stop) { ref = kDone; leaf = 0; break; }
-            leaf = 0;
-            if (ref < 0) { leaf = ref; ref = pop(); }
+            if (S.ref < 0) { S.leaf = S.ref; S.ref = stk.pop(S.top); }
         }
     }
-    if (bi >= 0) { res.tri = bi; res.t = best; res.u = bu; res.v = bv; res.front = bf; res.slot = bslot; }
-    return ok;
-}
-
-// ---- resumable form ---------------------------------------------------------------------
-// The same traversal with its state kept by the caller, so a lane can leave the loop
-// before its ray is finished and continue later: trace_begin sets a ray up,
-// trace_resume runs it until it is finished (returns true) or until no more than
-// `yield_at` lanes of the wave are still tracing (returns false, state kept).  Used by
-// the closest-hit kernel to refill lanes whose rays have finished.
-struct TraceState {
-    float3 o, d, idir, noi;
-    float lo, best, bound, bu, bv;
-    int32_t ref, leaf, bi;
-    int sp;
-    bool bf;
-};
-
-// false when the ray misses the scene box (then it is finished, no hit)
-__device__ inline bool trace_begin(TraceState& S, const ColliderView& c, const float3 o, const float3 d, float rmin, float rmax)
-{
-    float lo, hi;
-    S.bi = -1;
-    if (!c.nvalid || !ref_box_intersect(c.bmin, c.bmax, o, d, rmin, rmax, lo, hi)) return false;
-    S.o = o; S.d = d;
-    S.idir = safe_inv(d);
-    S.noi = make_float3(-o.x * S.idir.x, -o.y * S.idir.y, -o.z * S.idir.z);
-    S.lo = lo; S.best = hi; S.bound = hi;
-    S.bu = 0.f; S.bv = 0.f; S.bf = false;
-    S.ref = c.root4; S.leaf = 0; S.sp = 0;
     return true;
 }
 
 template <int STACK, class Filter>
-__device__ inline bool trace_resume(TraceState& S, const Filter& flt, const ColliderView& c, int32_t* stk, int stride,
-                                    uint32_t yield_at, bool& ok)
+__device__ inline bool trace_resume(TraceState& S, const Filter& flt, const ColliderView& c, const LaneStack& stk, uint32_t yield_at)
 {
-    constexpr int32_t kDone = 0x7fffffff;
-    auto pop = [&]() -> int32_t { return S.sp ? stk[(--S.sp) * stride] : kDone; };
-    while (S.ref != kDone || S.leaf < 0) {
-        if ((uint32_t)__popcll(__ballot(1)) <= yield_at) return false;     // enough lanes are free
-        while (S.ref >= 0 && S.ref != kDone) {
-            S.ref = visit4<STACK>(c.nodes4, S.ref, S.noi, S.idir, S.lo, S.bound, stk, stride, S.sp, ok, pop);
-            if (S.ref < 0 && S.leaf == 0) { S.leaf = S.ref; S.ref = pop(); }
-            if (!__any(S.leaf == 0)) break;
-        }
-        if (S.leaf == 0 && S.ref < 0) { S.leaf = S.ref; S.ref = pop(); }
-        while (S.leaf < 0) {
-            const uint32_t st = leaf_start(S.leaf), cnt = leaf_count(S.leaf);
-            bool stop = false;
-            for (uint32_t k = 0; k < cnt; k++) {
-                const uint32_t p = st + k;
-                const float4 pl = c.plane[p];
-                float ndd;
-                const float t = plane_distance(pl, S.o, S.d, ndd);
-                if (!(t >= S.lo && t <= S.bound)) continue;
-                const TriRest* tr = c.rest + p;
-                const uint2 mt = tr->meta;
-                if (!(S.bi < 0 || t < S.best || (int)mt.x < S.bi)) continue;
-                float u, v;
-                if (!srlnp_test(tr->sv, tr->ev, (int)mt.y, S.o, S.d, t, u, v)) continue;
-                const bool fr = ndd < 0;
-                if (!flt.accept(mt.x, fr, t, u, v)) continue;
-                S.best = t; S.bi = (int)mt.x; S.bu = u; S.bv = v; S.bf = fr;
-                S.bound = flt.clamp(S.best);
-                if (flt.done(t)) { stop = true; break; }
-            }
-            if (stop) { S.ref = kDone; S.leaf = 0; break; }
-            S.leaf = 0;
-            if (S.ref < 0) { S.leaf = S.ref; S.ref = pop(); }
-        }
-    }
-    return true;
+    uint32_t a = 0, b = 0;
+    return trace_run<STACK, false, Filter, true, true>(S, flt, c, stk, yield_at, a, b);
+}
+
+// the hit of a finished ray (tri -1: none)
+__device__ inline void trace_finish(const TraceState& S, const ColliderView& c, TraceResult& res)
+{
+    res.tri = -1; res.slot = S.slot;
+    if (S.slot == kNoSlot) return;
+    const float4 pl = c.plane[S.slot];
+    const TriRest* tr = c.rest + S.slot;
+    res.tri = (int)tr->meta.x;
+    res.t = S.best;
+    res.front = S.d.x * pl.x + S.d.y * pl.y + S.d.z * pl.z < 0;
+    srlnp_hit(tr->sv, tr->ev, tr->axes, S.o, S.d, S.best, res.u, res.v);
+}
+
+// the whole ray at once
+template <int STACK, bool STATS, class Filter, bool ORDERED = true>
+__device__ inline void trace_closest(const Filter& flt, const ColliderView& c, const float3 o, const float3 d, float rmin, float rmax,
+                                     int32_t* stk, int stride, TraceResult& res, uint32_t& nvis, uint32_t& ntest)
+{
+    TraceState S;
+    const LaneStack ls(stk, stride);
+    res.tri = -1;
+    if (!trace_begin(S, c, o, d, rmin, rmax, ls)) return;
+    trace_run<STACK, STATS, Filter, ORDERED, false>(S, flt, c, ls, 0u, nvis, ntest);
+    trace_finish(S, c, res);
 }
 
 } // namespace lsg

@@ -94,6 +94,48 @@ def test_gpu_cache_refuses_other_mesh_and_damage(gpu, tmp_path):
         col.close()
 
 
+def _payload_sum(p):
+    """The tree files' payload checksum."""
+    mask, prime = (1 << 64) - 1, 0x100000001b3
+    h = [0xcbf29ce484222325, 0x84222325cbf29ce4, 0x9e3779b97f4a7c15, 0xc2b2ae3d27d4eb4f]
+    n = len(p) // 32 * 32
+    for k, w in enumerate(np.frombuffer(p[:n], "<u8").tolist()):
+        h[k & 3] = (h[k & 3] ^ w) * prime & mask
+    r = h[0] ^ (h[1] * 3 & mask) ^ (h[2] * 5 & mask) ^ (h[3] * 7 & mask)
+    for b in p[n:]:
+        r = (r ^ b) * prime & mask
+    return (r ^ len(p)) * prime & mask
+
+
+@pytest.mark.parametrize("what", ["sound", "cycle", "node_past_end", "leaf_past_end"])
+def test_gpu_cache_walks_the_stored_tree(gpu, tmp_path, what):
+    """A file whose checksum is right but whose 4-wide tree could lead the traversal out of
+    its arrays is refused before it reaches the GPU."""
+    from lightsprintsdk_amd import native as N
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = S.icosphere(8, seed=2)
+    a = RRCollider.create(V, I)
+    path = str(tmp_path / "t.lsgbvh")
+    a.save(path)
+    n4 = a.info().num_nodes4
+    a.close()
+    raw = bytearray(open(path, "rb").read())
+    head = 8 + 4 + 4 + 20 + 4 + 8          # magic, version, header bytes, mesh hash, padding, then past the checksum
+    head_bytes = int.from_bytes(raw[12:16], "little")
+    refs = len(raw) - 128 * n4 + 96        # child refs of the 4-wide root
+    assert _payload_sum(bytes(raw[head_bytes:])) == int.from_bytes(raw[head - 8:head], "little")
+    bad = dict(sound=None, cycle=0, node_past_end=n4, leaf_past_end=-(1 << 31) | (len(I) << 4))[what]
+    if bad is not None:
+        raw[refs:refs + 4] = int(bad & 0xFFFFFFFF).to_bytes(4, "little")
+    raw[head - 8:head] = _payload_sum(bytes(raw[head_bytes:])).to_bytes(8, "little")
+    open(path, "wb").write(raw)
+    if bad is None:
+        RRCollider.load(V, I, path).close()
+        return
+    with pytest.raises(N.LsgError, match="4-wide tree"):
+        RRCollider.load(V, I, path)
+
+
 def test_gpu_cache_small_trees_and_star(gpu, tmp_path):
     from lightsprintsdk_amd.collider import RRCollider
     v = np.float32([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]])

@@ -234,3 +234,38 @@ def test_gpu_bvh4_stack_bound(gpu, oracle, scene):
     g, gf = c.intersect_batch(R)
     o = oracle.intersect_linear_srlnp(V, I, R)
     np.testing.assert_array_equal(g["tri"], o["tri"])
+
+
+@pytest.mark.parametrize("copies", [40, 300])
+def test_gpu_deep_tree_64_entry_stack(gpu, oracle, copies):
+    """A tree deeper than 31 (triangles at single-bit Morton codes, then many in one Morton
+    cell) takes the kernels with the 64-entry stack and 64-bit addresses: hits of the device
+    and the RRRay batch equal the oracle's."""
+    from lightsprintsdk_amd.collider import RRCollider, make_rrrays
+    rng = np.random.default_rng(copies)
+    c = [np.zeros(3), np.full(3, 1023.9)]
+    for bit in range(10):
+        for axis in range(3):
+            p = np.zeros(3)
+            p[axis] = 2.0 ** bit + 0.5
+            c.append(p)
+    c += [rng.uniform(0, 0.7, 3) for _ in range(copies)]
+    V = (np.repeat(np.array(c), 3, 0) + rng.uniform(0, 0.25, (3 * len(c), 3))).astype(np.float32)
+    I = np.arange(len(V), dtype=np.uint32).reshape(-1, 3)
+    col = RRCollider.create(V, I, leaf_size=1, lbvh_only=True)
+    inf = col.info()
+    assert 32 < inf.depth + 1 <= 64 and inf.stack_need <= 63
+    aim = V[I].mean(1)[rng.integers(0, len(I), 6000)]
+    R = scenes.random_rays(V, 6000, seed=9)
+    d = aim - R[:, 0:3]
+    R[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    o = oracle.intersect_linear_srlnp(V, I, R)
+    assert (o["tri"] >= 0).mean() > 0.5
+    g, _ = col.intersect_batch(R)
+    for f in ("tri", "t", "u", "v"):
+        m = slice(None) if f == "tri" else o["tri"] >= 0
+        np.testing.assert_array_equal(g[f][m], o[f][m])
+    rr = make_rrrays(R)
+    mask = col.intersect_rrrays(rr)
+    np.testing.assert_array_equal(mask.astype(bool), o["tri"] >= 0)
+    np.testing.assert_array_equal(rr["hitTriangle"][mask > 0], o["tri"][mask > 0].astype(np.uint32))
