@@ -569,8 +569,14 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
         return fail(LSG_ERR_LIMIT, "BVH depth %u exceeds the traversal stack (63)", C.depth);
     if (C.root < 0 || !C.nnodes) {
         C.root4 = C.root; C.nnodes4 = 0; C.stack_need = 0;
-        if ((st = dalloc(&C.d_nodes4, 1, &C.bytes))) return st;
-    } else if ((st = collapse4_device(C, (uint32_t)stack_size_for_depth(C.depth) - 1))) return st;
+        if ((st = pack4_device(C, nullptr))) return st;
+    } else {
+        Node4* n4 = nullptr;
+        if ((st = collapse4_device(C, (uint32_t)stack_size_for_depth(C.depth) - 1, &n4))) return st;
+        st = pack4_device(C, n4);
+        dfree(n4);                         // waits for the packing kernel
+        if (st) return st;
+    }
     C.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return LSG_OK;
 }
@@ -625,8 +631,9 @@ static int load_tree(ColliderImpl& C, const float* verts, uint32_t nv, const uin
     LSG_HIP(hipMemcpy(C.d_idx, idx, 12 * (size_t)nt, hipMemcpyHostToDevice));
     uint32_t *d_keys = nullptr, *d_vals = nullptr, *d_bytes = nullptr, *d_nvalid = nullptr, *d_order = nullptr;
     float4 *d_plane_u = nullptr, *d_sv_u = nullptr, *d_ev_u = nullptr, *d_blo_u = nullptr, *d_bhi_u = nullptr, *d_plo = nullptr, *d_phi = nullptr;
+    Node4* d_n4 = nullptr;
     auto cleanup = [&]() {
-        dfree(d_keys); dfree(d_vals); dfree(d_bytes); dfree(d_nvalid); dfree(d_order);
+        dfree(d_keys); dfree(d_vals); dfree(d_bytes); dfree(d_nvalid); dfree(d_order); dfree(d_n4);
         dfree(d_plane_u); dfree(d_sv_u); dfree(d_ev_u); dfree(d_blo_u); dfree(d_bhi_u); dfree(d_plo); dfree(d_phi);
     };
 #define CK(x) do { if ((st = (x))) { cleanup(); return st; } } while (0)
@@ -657,8 +664,9 @@ static int load_tree(ColliderImpl& C, const float* verts, uint32_t nv, const uin
     CK(dalloc(&C.d_nodes, C.nnodes ? C.nnodes : 1, &C.bytes));
     if (C.nnodes) CKH(hipMemcpy(C.d_nodes, nodes, sizeof(Node) * (size_t)C.nnodes, hipMemcpyHostToDevice));
     C.nnodes4 = h.nnodes4; C.root4 = h.root4; C.stack_need = h.stack_need;
-    CK(dalloc(&C.d_nodes4, C.nnodes4 ? C.nnodes4 : 1, &C.bytes));
-    if (C.nnodes4) CKH(hipMemcpy(C.d_nodes4, nodes4, sizeof(Node4) * (size_t)C.nnodes4, hipMemcpyHostToDevice));
+    CK(dalloc(&d_n4, C.nnodes4));
+    if (C.nnodes4) CKH(hipMemcpy(d_n4, nodes4, sizeof(Node4) * (size_t)C.nnodes4, hipMemcpyHostToDevice));
+    CK(pack4_device(C, d_n4));
     CKH(hipDeviceSynchronize());
     cleanup();
 #undef CK
@@ -768,9 +776,18 @@ static int save_to_file(const lsg_collider* c, const char* path, uint32_t flags,
         for (uint32_t i = 0; i < C.nvalid; i++) order[i] = m[i].meta.x;
     }
     if (C.nnodes) LSG_HIP(hipMemcpy(payload.data() + 4ull * C.nvalid, C.d_nodes, sizeof(Node) * (size_t)C.nnodes, hipMemcpyDeviceToHost));
-    if (C.nnodes4)
-        LSG_HIP(hipMemcpy(payload.data() + 4ull * C.nvalid + sizeof(Node) * (size_t)C.nnodes, C.d_nodes4, sizeof(Node4) * (size_t)C.nnodes4,
-                          hipMemcpyDeviceToHost));
+    if (C.nnodes4) {
+        // the file holds the 4-wide tree in binary32, which the collapse gives again
+        ColliderImpl again = C;
+        Node4* n4 = nullptr;
+        if (int st = collapse4_device(again, (uint32_t)stack_size_for_depth(C.depth) - 1, &n4)) return st;
+        const hipError_t e = again.nnodes4 == C.nnodes4
+                                 ? hipMemcpy(payload.data() + 4ull * C.nvalid + sizeof(Node) * (size_t)C.nnodes, n4,
+                                             sizeof(Node4) * (size_t)C.nnodes4, hipMemcpyDeviceToHost)
+                                 : hipErrorUnknown;
+        dfree(n4);
+        if (e != hipSuccess) return hip_fail(e, "4-wide tree", __LINE__);
+    }
     // the mesh hash from the device copy of the mesh
     std::vector<float> v(3 * (size_t)C.nverts);
     std::vector<uint32_t> ix(3 * (size_t)C.ntri);

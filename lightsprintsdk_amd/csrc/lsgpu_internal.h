@@ -29,13 +29,27 @@ bool device_ready();   // a gfx950 device is present and selected
 // count = (ref&15)+1 triangles in leaf order.
 struct alignas(16) Node { float4 q0, q1, q2, q3; };
 
-// BVH4 node, 128 bytes (one cache line), collapsed from the BVH2 above and used by
-// every GPU traversal:
+// BVH4 node, 128 bytes, collapsed from the BVH2 above (what tree files hold):
 //   q[0] = lo.x of children 0..3   q[1] = hi.x   q[2] = lo.y   q[3] = hi.y
 //   q[4] = lo.z                    q[5] = hi.z   q[6] = child refs (int bits)
 // Refs as in the BVH2 (>= 0 inner BVH4 node, < 0 leaf); kNoChild marks an unused slot.
 struct alignas(128) Node4 { float4 q[8]; };
 constexpr int32_t kNoChild = 0x7ffffffe;
+
+// The BVH4 node as every GPU traversal reads it, one cache line, five 16-byte loads.  The
+// child planes are binary16 distances from the node's origin, in units of the tree's power-
+// of-two scale, rounded outwards (lo down, hi up): the boxes only grow, so culling stays
+// conservative, and v_fma_mix reads them at no cost.  Each axis holds lo[4] hi[4] lo[4]: a ray
+// going up loads 16 bytes from the first lo (near, far planes), one going down from hi.
+struct alignas(128) NodeT {
+    uint16_t x[12], y[12];     // bytes 0 and 24
+    int32_t ref[4];            // byte 48
+    uint16_t z[12];            // byte 64
+    uint16_t pad0[4];
+    float org[4];              // byte 96: origin, scaled
+    uint32_t pad1[4];
+};
+static_assert(sizeof(NodeT) == 128, "a node is one cache line");
 
 // Triangle in leaf order, 48 bytes + 8 bytes meta (TriangleSRLNP,
 // IntersectBspFast.h:33-49, with the projection-selected components pre-picked):
@@ -117,7 +131,8 @@ struct alignas(16) TriRest { float4 sv, ev; uint2 meta; uint32_t axes, pad; };
 
 struct ColliderView {
     const Node* nodes;
-    const Node4* nodes4;
+    const NodeT* nodes4;
+    float unscale;         // 1 / the nodes' scale
     int32_t root4;
     const float4* plane; const TriRest* rest;
     int32_t root;
@@ -129,7 +144,8 @@ struct ColliderImpl {
     uint32_t ntri = 0, nverts = 0, nvalid = 0, nnodes = 0, depth = 0, leaf = 4;
     uint32_t nnodes4 = 0, stack_need = 0;   // BVH4 nodes; worst-case traversal stack entries
     int32_t root4 = 0;
-    Node4* d_nodes4 = nullptr;
+    NodeT* d_nodes4 = nullptr;
+    float scale = 1.f;            // the nodes' power-of-two scale (node_scale)
     int32_t root = 0;
     float bmin[3], bmax[3], margin = 0;
     float* d_verts = nullptr; uint32_t* d_idx = nullptr;
@@ -145,7 +161,7 @@ struct ColliderImpl {
     {
         ColliderView v;
         v.nodes = d_nodes; v.plane = d_plane; v.rest = d_rest;
-        v.nodes4 = d_nodes4; v.root4 = root4;
+        v.nodes4 = d_nodes4; v.root4 = root4; v.unscale = 1.f / scale;
         v.root = root; v.nvalid = nvalid;
         v.bmin = make_float3(bmin[0], bmin[1], bmin[2]);
         v.bmax = make_float3(bmax[0], bmax[1], bmax[2]);
@@ -182,9 +198,12 @@ std::string cache_file_name(const uint8_t hash[20], uint32_t version, const char
 // two leaves, else an LSG_ERR_* code
 int sah_rebuild_device(const int* d_first, const int* d_last, const int* d_split, int nprim, uint32_t leafmax, const Node* d_nodes,
                        Node** out_nodes, uint32_t* out_count, uint32_t* out_depth);
-// The BVH4 of C's BVH2 on the GPU (lsgpu_sah.hip): C.d_nodes4, nnodes4, root4, stack_need
+// The BVH4 of C's BVH2 on the GPU (lsgpu_sah.hip): C.nnodes4, root4, stack_need and the nodes
+// (device, the caller's to free)
 struct ColliderImpl;
-int collapse4_device(ColliderImpl& C, uint32_t budget);
+int collapse4_device(ColliderImpl& C, uint32_t budget, Node4** nodes4);
+// C.d_nodes4 and C.scale from the BVH4 nodes (device) of C's tree; C.bytes counts them
+int pack4_device(ColliderImpl& C, const Node4* nodes4);
 // SAH rebuild of a BVH2's inner nodes over its leaves (lsgpu_sah.cpp): 0 = rebuilt,
 // 1 = fewer than two leaves, 2 = malformed tree
 int sah_rebuild(const float* nodes, uint32_t nnodes, int32_t root, float* out, uint32_t* out_nodes, int32_t* out_root,

@@ -13,6 +13,8 @@
 // Tasks of 2^15 leaves or more (the top levels) take the same steps across the chip:
 // many workgroups bin, one lane splits, a scan of left/right flags partitions.
 #include "lsgpu_internal.h"
+#include <algorithm>
+#include <cmath>
 #include <vector>
 
 namespace lsg {
@@ -477,6 +479,53 @@ __global__ __launch_bounds__(256) void k_c4_link(const C4Work* __restrict__ work
     }
 }
 
+// binary16 bits of the largest value <= x (DOWN) or the smallest >= x; beyond the range that is
+// the largest finite value or infinity, whichever side is asked for
+template <bool DOWN> __device__ inline uint16_t half_towards(double x)
+{
+    const float f = DOWN ? __double2float_rd(x) : __double2float_ru(x);
+    const _Float16 h = (_Float16)f;
+    uint16_t b;
+    __builtin_memcpy(&b, &h, 2);
+    if (DOWN ? (float)h <= f : (float)h >= f) return b;
+    // one step of the ordered bits: away from zero when the value must grow in size
+    if ((b & 0x7fffu) == 0u) return DOWN ? 0x8001u : 0x0001u;
+    const bool neg = (b & 0x8000u) != 0u;
+    return (uint16_t)(neg == DOWN ? b + 1u : b - 1u);
+}
+
+// Node4 -> NodeT: the origin is the middle of the node's box, so that the planes' distances
+// from it are at most half its size (binary16 keeps 11 bits of them)
+__global__ __launch_bounds__(256) void k_c4_pack(const Node4* __restrict__ in, uint32_t n, float scale, NodeT* __restrict__ out)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const Node4 nd = in[i];
+    const float* f = (const float*)nd.q;
+    const int32_t* ref = (const int32_t*)&nd.q[6];
+    NodeT o;
+    for (int k = 0; k < 4; k++) { o.ref[k] = ref[k]; o.pad0[k] = 0; o.pad1[k] = 0; }
+    o.org[3] = 0.f;
+    for (int a = 0; a < 3; a++) {
+        const float* lo = f + 8 * a;
+        const float* hi = lo + 4;
+        float mn = 0.f, mx = 0.f;
+        bool any = false;
+        for (int k = 0; k < 4; k++)
+            if (ref[k] != kNoChild) { mn = any ? fminf(mn, lo[k]) : lo[k]; mx = any ? fmaxf(mx, hi[k]) : hi[k]; any = true; }
+        const float org = (0.5f * mn + 0.5f * mx) * scale;
+        o.org[a] = org;
+        uint16_t* q = a == 0 ? o.x : (a == 1 ? o.y : o.z);
+        for (int k = 0; k < 4; k++) {
+            const bool have = ref[k] != kNoChild;
+            const uint16_t l = have ? half_towards<true>((double)lo[k] * (double)scale - (double)org) : (uint16_t)0;
+            const uint16_t h = have ? half_towards<false>((double)hi[k] * (double)scale - (double)org) : (uint16_t)0;
+            q[k] = l; q[4 + k] = h; q[8 + k] = l;
+        }
+    }
+    out[i] = o;
+}
+
 inline void sfree(void* p) { if (p) (void)hipFree(p); }
 
 } // namespace
@@ -591,9 +640,10 @@ int sah_rebuild_device(const int* d_first, const int* d_last, const int* d_split
 // The BVH4 of a BVH2 (nodes, nn, root >= 0) on the GPU, breadth first: heights bottom-up
 // (one launch per level),
 // then one level of BVH4 nodes per launch, slots in level order.  budget = the traversal
-// stack entries minus one.  Sets C.d_nodes4, C.nnodes4, C.root4 = 0, C.stack_need.
-int collapse4_device(ColliderImpl& C, uint32_t budget)
+// stack entries minus one.  Sets C.nnodes4, C.root4 = 0, C.stack_need.
+int collapse4_device(ColliderImpl& C, uint32_t budget, Node4** nodes4)
 {
+    *nodes4 = nullptr;
     const uint32_t nn = C.nnodes;
     uint32_t *H = nullptr, *cnt = nullptr, *prefix = nullptr, *pnext = nullptr, *tmp = nullptr, *total = nullptr,
              *need = nullptr;
@@ -648,15 +698,28 @@ int collapse4_device(ColliderImpl& C, uint32_t budget)
     }
     uint32_t sn = 0;
     SK(hipMemcpy(&sn, need, 4, hipMemcpyDeviceToHost));
-    Node4* exact = nullptr;
-    SK(hipMalloc(&exact, sizeof(Node4) * (size_t)n4));
-    SK(hipMemcpy(exact, out, sizeof(Node4) * (size_t)n4, hipMemcpyDeviceToDevice));
     cleanup();
-    sfree(out);
 #undef SK
-    C.d_nodes4 = exact;
-    C.bytes += sizeof(Node4) * (uint64_t)n4;
+    *nodes4 = out;
     C.nnodes4 = n4; C.root4 = 0; C.stack_need = sn;
+    return LSG_OK;
+}
+
+int pack4_device(ColliderImpl& C, const Node4* nodes4)
+{
+    // the scene's size becomes 2^13 to 2^14: a plane's distance from its node's origin is far
+    // from binary16's limit, and the boxes' inflation (1e-5 of the largest coordinate) far
+    // above its smallest steps
+    float ext = 0.f;
+    for (int a = 0; a < 3; a++) ext = std::max(ext, C.bmax[a] - C.bmin[a]);
+    int e = 0;
+    if (ext > 0.f && std::isfinite(ext)) (void)std::frexp(ext, &e);
+    C.scale = std::ldexp(1.f, std::min(100, std::max(-100, 14 - e)));
+    const size_t n = C.nnodes4 ? C.nnodes4 : 1;
+    LSG_HIP(hipMalloc(&C.d_nodes4, sizeof(NodeT) * n));
+    C.bytes += sizeof(NodeT) * n;
+    if (C.nnodes4) k_c4_pack<<<(C.nnodes4 + 255) / 256, 256>>>(nodes4, C.nnodes4, C.scale, C.d_nodes4);
+    LSG_HIP(hipGetLastError());
     return LSG_OK;
 }
 

@@ -64,6 +64,8 @@ template <bool WIDE, class T> __device__ inline T load_at(const void* base, uint
     else return *(const T*)((const char*)base + ((size == 48u ? (i + 2u * i) << 4 : i * size) + off));
 }
 
+typedef _Float16 half8 __attribute__((ext_vector_type(8), aligned(8)));
+
 // (distance, child ref) pairs as one 64-bit float: the distance's bits are the high word, so
 // the doubles order as the distances do (never a NaN: the high word is at most that of
 // binary32 infinity, a finite double; binary64 keeps denormals) and v_min_f64 / v_max_f64,
@@ -86,12 +88,13 @@ __device__ inline float vmin3(float a, float b, float c) { float r; asm("v_min3_
 __device__ inline float vmax(float a, float b) { float r; asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
 __device__ inline float vmin(float a, float b) { float r; asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
 
-// what a ray's box tests need: noi = -o * idir, so each plane distance is one fma: (b - o) *
-// idir = b * idir - o * idir.  The fused form differs from the two-step one by about |o * idir|
-// ulp, i.e. |o| * 6e-8 in distance, while every child box is inflated by DELTA_BSP =
-// max|coordinate| * 1e-5; culling stays conservative and the hit, decided only by the
-// triangle test, is unchanged.  near: byte offsets of the
-// axes' near planes in a node, a byte each.
+// what a ray's box tests need.  idir is the inverse direction divided by the nodes' scale, noi
+// = -o * inverse direction: with c = origin * idir + noi per node and axis, a plane's
+// distance along the ray is one fma, distance from the origin * idir + c.  That differs from
+// (plane - o) * inverse direction by a few ulp of |o * inverse direction|, i.e. |o| * 2e-7 in
+// distance, while every child box is inflated by DELTA_BSP = max|coordinate| * 1e-5; culling
+// stays conservative and the hit, decided only by the triangle test, is unchanged.  near:
+// byte offsets of the axes' near planes in a node, a byte each.
 struct RayBox { float3 idir, noi; uint32_t near; };
 
 __device__ inline float3 safe_inv(float3 d)
@@ -102,12 +105,14 @@ __device__ inline float3 safe_inv(float3 d)
     return make_float3(1.0f / x, 1.0f / y, 1.0f / z);
 }
 
-__device__ inline RayBox ray_box(const float3 o, const float3 d)
+__device__ inline RayBox ray_box(const float3 o, const float3 d, float unscale)
 {
     RayBox r;
     r.idir = safe_inv(d);
     r.noi = make_float3(-o.x * r.idir.x, -o.y * r.idir.y, -o.z * r.idir.z);
-    r.near = (r.idir.x < 0.f ? 16u : 0u) | (r.idir.y < 0.f ? 48u : 32u) << 8 | (r.idir.z < 0.f ? 80u : 64u) << 16;
+    r.idir.x *= unscale; r.idir.y *= unscale; r.idir.z *= unscale;
+    // (by the inverse: -0 has a negative one)
+    r.near = (r.idir.x < 0.f ? 8u : 0u) | (r.idir.y < 0.f ? 32u : 24u) << 8 | (r.idir.z < 0.f ? 72u : 64u) << 16;
     return r;
 }
 
@@ -116,39 +121,41 @@ __device__ inline RayBox ray_box(const float3 o, const float3 d)
 // (ORDERED; else any order).  No child hit: the next ref is popped.  The tree is collapsed
 // so that the stack never holds more than STACK-1 entries.
 //
-// Per axis the lane loads its near plane (lo or hi by the direction's sign) and the far
-// one, 16 bytes apart: near <= far (fma is monotonic and idir never 0), so entry and exit
-// are a max3 / min3 of three fmas per child without a min/max pair per axis.
+// Per axis one load brings the near planes (lo or hi by the direction's sign), then the far
+// ones: near <= far (fma is monotonic), so entry and exit are a max3 / min3 of three fmas
+// per child without a min/max pair per axis.
 //
-// Bound by VALU issue together with the L1's tag lookups (a lookup per distinct node and
-// load; SQ and TA counters of a 1024-ray gather over 50k triangles: VALU 78% of issue, TA
-// busy 86%).  Straight-line tests, sorting (distance, ref) pairs as doubles, branch-free
-// pushes and 32-bit offsets issue 39.7e9 instead of 49.7e9 wave instructions per such gather:
-// 89.6 -> 84.9 ms, 1M random rays against 100k triangles 0.718 -> 0.638 ms, a sun-and-sky
-// gather over 132k triangles 27.9 -> 24.3 ms.
+// Bound by VALU issue.  SQ and TA counters of a 1024-ray gather over 50k triangles (751k
+// texels), seven binary32 loads a visit -> these five binary16 ones: time 84.9 -> 71.0 ms, VALU
+// 78% -> 94% of issue, L1 tag lookups (one per distinct node and load) 46.7e9 -> 35.1e9, TA
+// busy 86% -> 79%; sun-and-sky bake over 132k triangles 24.2 -> 22.3 ms.  1M random rays
+// against 100k triangles, bound by latency at 20% active lanes, stay at 0.638 ms.
+// Straight-line tests, pairs sorted as doubles, branch-free pushes and 32-bit offsets had
+// taken the gather's wave instructions from 49.7e9 to 39.7e9 (89.6 -> 84.9 ms).
 template <bool WIDE, bool ORDERED>
-__device__ inline int32_t visit4(const Node4* __restrict__ nodes, int32_t ref, const RayBox& R, float tlo, float thi,
+__device__ inline int32_t visit4(const NodeT* __restrict__ nodes, int32_t ref, const RayBox& R, float tlo, float thi,
                                  const LaneStack& stk, uint32_t& top)
 {
-    const uint32_t n = (uint32_t)ref, ax = R.near & 255u, ay = (R.near >> 8) & 255u, az = R.near >> 16;
-    // the node's seven 16-byte loads are issued together, before any use: left to itself
-    // the scheduler issues four, waits for them, then the other three (two memory
-    // round trips per node visit)
-    const float4 nx = load_at<WIDE, float4>(nodes, n, 128u, ax), fx = load_at<WIDE, float4>(nodes, n, 128u, ax ^ 16u);
-    const float4 ny = load_at<WIDE, float4>(nodes, n, 128u, ay), fy = load_at<WIDE, float4>(nodes, n, 128u, ay ^ 16u);
-    const float4 nz = load_at<WIDE, float4>(nodes, n, 128u, az), fz = load_at<WIDE, float4>(nodes, n, 128u, az ^ 16u);
-    const int4 r = load_at<WIDE, int4>(nodes, n, 128u, 96u);
+    const uint32_t n = (uint32_t)ref;
+    // the node's five 16-byte loads are issued together, before any use (left to itself the
+    // scheduler issues some, waits for them, then the others)
+    const half8 x = load_at<WIDE, half8>(nodes, n, 128u, R.near & 255u), y = load_at<WIDE, half8>(nodes, n, 128u, (R.near >> 8) & 255u);
+    const half8 z = load_at<WIDE, half8>(nodes, n, 128u, R.near >> 16);
+    const float4 org = load_at<WIDE, float4>(nodes, n, 128u, 96u);
+    const int4 r = load_at<WIDE, int4>(nodes, n, 128u, 48u);
     __builtin_amdgcn_sched_barrier(0);
-    auto enter = [&](float x, float y, float z) {
-        return vmax3(__fmaf_rn(x, R.idir.x, R.noi.x), __fmaf_rn(y, R.idir.y, R.noi.y), vmax(__fmaf_rn(z, R.idir.z, R.noi.z), tlo));
+    const float cx = __fmaf_rn(org.x, R.idir.x, R.noi.x), cy = __fmaf_rn(org.y, R.idir.y, R.noi.y), cz = __fmaf_rn(org.z, R.idir.z, R.noi.z);
+    auto enter = [&](int k) {
+        return vmax3(__fmaf_rn((float)x[k], R.idir.x, cx), __fmaf_rn((float)y[k], R.idir.y, cy), vmax(__fmaf_rn((float)z[k], R.idir.z, cz), tlo));
     };
-    auto leave = [&](float x, float y, float z) {
-        return vmin3(__fmaf_rn(x, R.idir.x, R.noi.x), __fmaf_rn(y, R.idir.y, R.noi.y), vmin(__fmaf_rn(z, R.idir.z, R.noi.z), thi));
+    auto leave = [&](int k) {
+        return vmin3(__fmaf_rn((float)x[4 + k], R.idir.x, cx), __fmaf_rn((float)y[4 + k], R.idir.y, cy),
+                     vmin(__fmaf_rn((float)z[4 + k], R.idir.z, cz), thi));
     };
-    const float k0 = enter(nx.x, ny.x, nz.x), k1 = enter(nx.y, ny.y, nz.y), k2 = enter(nx.z, ny.z, nz.z), k3 = enter(nx.w, ny.w, nz.w);
+    const float k0 = enter(0), k1 = enter(1), k2 = enter(2), k3 = enter(3);
     // (bitwise, so that the tests stay straight-line code)
-    const bool h0 = (r.x != kNoChild) & (k0 <= leave(fx.x, fy.x, fz.x)), h1 = (r.y != kNoChild) & (k1 <= leave(fx.y, fy.y, fz.y));
-    const bool h2 = (r.z != kNoChild) & (k2 <= leave(fx.z, fy.z, fz.z)), h3 = (r.w != kNoChild) & (k3 <= leave(fx.w, fy.w, fz.w));
+    const bool h0 = (r.x != kNoChild) & (k0 <= leave(0)), h1 = (r.y != kNoChild) & (k1 <= leave(1));
+    const bool h2 = (r.z != kNoChild) & (k2 <= leave(2)), h3 = (r.w != kNoChild) & (k3 <= leave(3));
     if constexpr (!ORDERED) {
         // any order: continue with the last hit child in slot order, push the others
         int32_t nxt = h0 ? r.x : kDone;
@@ -192,7 +199,7 @@ __device__ inline bool trace_begin(TraceState& S, const ColliderView& c, const f
     S.slot = kNoSlot;
     if (!c.nvalid || !ref_box_intersect(c.bmin, c.bmax, o, d, rmin, rmax, lo, hi)) return false;
     S.o = o; S.d = d;
-    S.box = ray_box(o, d);
+    S.box = ray_box(o, d, c.unscale);
     S.lo = lo; S.best = hi; S.bound = hi;
     S.ref = c.root4; S.leaf = 0; S.top = stk.base;
     return true;

@@ -269,3 +269,22 @@ def test_gpu_deep_tree_64_entry_stack(gpu, oracle, copies):
     mask = col.intersect_rrrays(rr)
     np.testing.assert_array_equal(mask.astype(bool), o["tri"] >= 0)
     np.testing.assert_array_equal(rr["hitTriangle"][mask > 0], o["tri"][mask > 0].astype(np.uint32))
+
+
+@pytest.mark.parametrize("scale,offset", [(1e-7, 0.0), (1e-3, 5.0), (1.0, 300.0), (3e4, 0.0), (1e8, 0.0)])
+def test_gpu_node_boxes_at_any_scale(gpu, oracle, scale, offset):
+    """The traversal's nodes hold child boxes as binary16 distances rounded outwards: no hit is
+    culled, in small and large scenes, far from the origin, along the axes and from the
+    surface itself."""
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = scenes.icosphere(14, seed=6)
+    V = (V.astype(np.float64) * scale + offset * np.array([1.0, -2.0, 0.5])).astype(np.float32)
+    R = scenes.random_rays(V, 9000, seed=12)
+    axis = np.eye(3, dtype=np.float32)
+    R[:3000, 4:7] = np.where(np.arange(3000)[:, None] % 2, 1, -1).astype(np.float32) * axis[np.arange(3000) % 3]
+    R[3000:4500, 0:3] = V[I[np.arange(1500) % len(I)]].mean(1)       # from triangles' middles
+    col = RRCollider.create(V, I)
+    g, gf = col.intersect_batch(R)
+    o = oracle.intersect_linear_srlnp(V, I, R)
+    assert (o["tri"] >= 0).mean() > 0.2
+    _same_hits(g, gf, o, o)
