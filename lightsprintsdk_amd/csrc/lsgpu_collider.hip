@@ -295,13 +295,23 @@ __global__ __launch_bounds__(256) void k_write_tris(uint32_t n, const uint32_t* 
 // ---------------------------------------------------------------------------------------
 // traversal
 
-// Closest hit of a device ray batch.  The waves of a launch take rays from one queue (a
-// counter in device memory): whenever kRefill of a wave's lanes are free, the wave takes that
-// many consecutive rays with one atomic add and hands them to the free lanes in lane order,
-// while the other lanes keep tracing (trace_resume yields and keeps their state).  No wave
-// idles while rays remain, whichever rays turn out long.  Rays that miss the scene box are
-// finished at once.
-constexpr uint32_t kRefill = 24;
+// Closest hit of a device ray batch.  Batches of at most one ray per resident lane are
+// spread over the chip: every wave takes per_wave rays at once, so few that they reach 4 waves
+// per SIMD first (kSpread waves per CU) and then fill the waves' lanes.  Larger ones: the
+// waves take rays from one queue (a counter in device memory): whenever kRefill of a wave's
+// lanes are free, the wave takes that many consecutive rays with one atomic add and hands them
+// to the free lanes in lane order, while the other lanes keep tracing (trace_resume yields
+// and keeps their state).  Rays that miss the scene box are finished at once.
+//
+// Bound by the longest rays' chain of dependent loads in small batches (a ray of 81 visits
+// and 69 tests alone takes 66 us) and by divergence in large ones (VALU 60% of issue, 20% of
+// the lanes active; sorted rays run no faster, the lengths scatter within any cell).
+// Displaced icosphere, random rays, 4 rays per lane in a quarter of the waves -> this spread,
+// with a leaf's triangles read together (EAGER): 4,096 rays / 2,880 triangles 107 -> 31 us,
+// 50k / 100k triangles 391 -> 129 us, 200k 425 -> 202 us.  1M / 100k triangles (queue), refill
+// at 24 / 32 / 40 / 48 / 64 free lanes: 600 / 547 / 496 / 511 / 630 us (636 before).
+constexpr uint32_t kRefill = 40;
+constexpr uint32_t kMinPerWave = 4, kSpread = 16;
 constexpr uint32_t kRayQueues = 256;      // counters per collider: launches in flight at once
 
 __global__ void k_ray_queue_reset(unsigned long long* q) { if (threadIdx.x == 0) *q = 0ull; }
@@ -309,7 +319,8 @@ __global__ void k_ray_queue_reset(unsigned long long* q) { if (threadIdx.x == 0)
 template <int STACK>
 __global__ __launch_bounds__(256) void k_trace_closest(ColliderView c, const float4* __restrict__ ro, const float4* __restrict__ rd,
                                                        uint32_t n, int4* __restrict__ hits, uint8_t* __restrict__ front,
-                                                       unsigned long long* __restrict__ queue)
+                                                       float4* __restrict__ planes, unsigned long long* __restrict__ queue,
+                                                       uint32_t per_wave)
 {
     __shared__ int32_t stk[STACK * 256];
     const uint32_t lane = threadIdx.x & 63u;
@@ -323,10 +334,16 @@ __global__ __launch_bounds__(256) void k_trace_closest(ColliderView c, const flo
         const uint32_t nfree = 64u - (uint32_t)__popcll(bm);
         if (!done && (nfree >= kRefill || !bm)) {
             unsigned long long q0 = 0;
-            if (lane == 0) q0 = atomicAdd(queue, (unsigned long long)nfree);
-            q0 = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(q0 >> 32)) << 32)
-                 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)q0);
-            if (q0 >= n || n - q0 <= nfree) done = true;
+            if (per_wave) {
+                q0 = (unsigned long long)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4u + (threadIdx.x >> 6))) * per_wave;
+                n = (uint32_t)min((unsigned long long)n, q0 + per_wave);
+                done = true;
+            } else {
+                if (lane == 0) q0 = atomicAdd(queue, (unsigned long long)nfree);
+                q0 = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(q0 >> 32)) << 32)
+                     | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)q0);
+                if (q0 >= n || n - q0 <= nfree) done = true;
+            }
             const uint32_t rank = (uint32_t)__popcll(~bm & (lane ? (~0ull >> (64 - lane)) : 0ull));   // free lanes below
             if (!busy && q0 < n && rank < n - q0) {
                 ray = (uint32_t)q0 + rank;
@@ -342,12 +359,13 @@ __global__ __launch_bounds__(256) void k_trace_closest(ColliderView c, const flo
         if (!bm) break;             // queue empty and nothing in flight
         if (!busy) continue;
         const uint32_t yield_at = done ? 0u : 64u - kRefill;
-        if (!trace_resume<STACK>(S, NoFilter(), c, ls, yield_at)) continue;
+        if (!trace_resume<STACK, true>(S, NoFilter(), c, ls, yield_at)) continue;
         busy = false;
         TraceResult r;
         trace_finish(S, c, r);
         hits[ray] = r.tri >= 0 ? make_int4(r.tri, __float_as_int(r.t), __float_as_int(r.u), __float_as_int(r.v)) : make_int4(-1, 0, 0, 0);
         if (front) front[ray] = (r.tri >= 0 && r.front) ? 1 : 0;
+        if (planes && r.tri >= 0) planes[ray] = c.plane[r.slot];
     }
 }
 
@@ -363,28 +381,6 @@ __global__ __launch_bounds__(256) void k_trace_stats(ColliderView c, const float
     trace_closest<STACK, true>(NoFilter(), c, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, stk + threadIdx.x, 256, r, nv, nt);
     atomicAdd(&counters[0], (unsigned long long)nv);
     atomicAdd(&counters[1], (unsigned long long)nt);
-}
-
-// RRRay-shaped results for lsg_collider_intersect_rrrays: (tri,t,u,v) + plane of the hit.
-template <int STACK>
-__global__ __launch_bounds__(256) void k_trace_full(ColliderView c, const float4* __restrict__ ro, const float4* __restrict__ rd,
-                                                    uint32_t n, int4* __restrict__ hits, float4* __restrict__ planes,
-                                                    uint8_t* __restrict__ front)
-{
-    __shared__ int32_t stk[STACK * 256];
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float4 a = ro[i], b = rd[i];
-    TraceResult r; uint32_t nv = 0, nt = 0;
-    trace_closest<STACK, false>(NoFilter(), c, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, stk + threadIdx.x, 256, r, nv, nt);
-    if (r.tri >= 0) {
-        hits[i] = make_int4(r.tri, __float_as_int(r.t), __float_as_int(r.u), __float_as_int(r.v));
-        planes[i] = c.plane[r.slot];
-        front[i] = r.front ? 1 : 0;
-    } else {
-        hits[i] = make_int4(-1, 0, 0, 0);
-        front[i] = 0;
-    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -406,6 +402,43 @@ static void free_impl(ColliderImpl& c)
 }
 
 static inline unsigned blocks(uint64_t n, unsigned per = 256) { return (unsigned)((n + per - 1) / per); }
+
+// closest hits of n rays (planes: optional, the hits' planes)
+static void launch_trace(const ColliderImpl& C, int stack, const float4* ro, const float4* rd, uint32_t n, int4* hits, uint8_t* front,
+                         float4* planes, hipStream_t s)
+{
+    // resident blocks on the chip as the kernels' registers and LDS allow, queried once
+    struct Shape {
+        int cus = 256, per32 = 4, per64 = 2;
+        Shape()
+        {
+            int v = 0;
+            if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, 0) == hipSuccess && v > 0) cus = v;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_trace_closest<32>, 256, 0) == hipSuccess && v > 0) per32 = v;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_trace_closest<64>, 256, 0) == hipSuccess && v > 0) per64 = v;
+        }
+    };
+    static const Shape shape;
+    const uint32_t cus = (uint32_t)shape.cus;
+    const unsigned resident = cus * (unsigned)(stack <= 32 ? shape.per32 : shape.per64);
+    unsigned nb = resident;
+    uint32_t per_wave = 0;
+    unsigned long long* q = nullptr;
+    if (n <= resident * 256u) {
+        // every ray has a lane of its own: each wave takes its rays at once
+        per_wave = std::min(64u, std::max(kMinPerWave, (uint32_t)(((uint64_t)n + cus * kSpread - 1) / (cus * kSpread))));
+        nb = blocks((n + per_wave - 1) / per_wave, 4);
+    } else {
+        // a counter of this collider's ring (launches in flight on one collider take different
+        // ones), zeroed on the launch's stream
+        q = C.d_queue + (__atomic_fetch_add(&C.queue_next, 1u, __ATOMIC_RELAXED) % kRayQueues);
+        k_ray_queue_reset<<<1, 64, 0, s>>>(q);
+    }
+    if (stack <= 32)
+        k_trace_closest<32><<<nb, 256, 0, s>>>(C.view(), ro, rd, n, hits, front, planes, q, per_wave);
+    else
+        k_trace_closest<64><<<nb, 256, 0, s>>>(C.view(), ro, rd, n, hits, front, planes, q, per_wave);
+}
 
 // BVH2 -> BVH4, on the host after the GPU build.  Every BVH4 node starts from one BVH2
 // node's two children and opens the inner child of largest surface area, up to four
@@ -951,25 +984,7 @@ int lsg_collider_intersect_device(const lsg_collider* c, const void* ro, const v
     const ColliderImpl& C = c->impl;
     const int stack = traversal_stack(C);
     if (!stack) return fail(LSG_ERR_LIMIT, "tree too deep");
-    hipStream_t s = (hipStream_t)stream;
-    // a counter of this collider's ring (launches in flight on one collider take different
-    // ones), zeroed on the launch's stream; waves enough to fill every CU at 4 per SIMD
-    unsigned long long* q = C.d_queue + (__atomic_fetch_add(&C.queue_next, 1u, __ATOMIC_RELAXED) % kRayQueues);
-    k_ray_queue_reset<<<1, 64, 0, s>>>(q);
-    // resident blocks per CU as the kernel's registers and LDS allow, queried once
-    static int cus = 0, per32 = 0, per64 = 0;
-    if (!cus) {
-        int v = 0;
-        cus = (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, 0) == hipSuccess && v > 0) ? v : 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per32, k_trace_closest<32>, 256, 0) != hipSuccess || per32 < 1) per32 = 4;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per64, k_trace_closest<64>, 256, 0) != hipSuccess || per64 < 1) per64 = 2;
-    }
-    const unsigned resident = (unsigned)cus * (unsigned)(stack <= 32 ? per32 : per64);
-    const unsigned nb = std::max(1u, std::min(blocks(n, 256u * 4u), resident));
-    if (stack <= 32)
-        k_trace_closest<32><<<nb, 256, 0, s>>>(C.view(), (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, q);
-    else
-        k_trace_closest<64><<<nb, 256, 0, s>>>(C.view(), (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, q);
+    launch_trace(C, stack, (const float4*)ro, (const float4*)rd, n, (int4*)hits, (uint8_t*)front, nullptr, (hipStream_t)stream);
     LSG_HIP(hipGetLastError());
     return LSG_OK;
 }
@@ -1020,10 +1035,7 @@ int lsg_collider_intersect_rrrays(const lsg_collider* c, void* rays, uint32_t n,
     CK(dalloc(&d_o, n)); CK(dalloc(&d_d, n)); CK(dalloc(&d_pl, n)); CK(dalloc(&d_h, n)); CK(dalloc(&d_f, n));
     CKH(hipMemcpy(d_o, ho.data(), 16 * (size_t)n, hipMemcpyHostToDevice));
     CKH(hipMemcpy(d_d, hd.data(), 16 * (size_t)n, hipMemcpyHostToDevice));
-    if (traversal_stack(C) <= 32)
-        k_trace_full<32><<<blocks(n), 256>>>(C.view(), d_o, d_d, n, d_h, d_pl, d_f);
-    else
-        k_trace_full<64><<<blocks(n), 256>>>(C.view(), d_o, d_d, n, d_h, d_pl, d_f);
+    launch_trace(C, traversal_stack(C), d_o, d_d, n, d_h, d_f, d_pl, nullptr);
     CKH(hipGetLastError());
     std::vector<int4> hh(n); std::vector<float4> hp(n); std::vector<uint8_t> hf(n);
     CKH(hipMemcpy(hh.data(), d_h, 16 * (size_t)n, hipMemcpyDeviceToHost));

@@ -1256,7 +1256,7 @@ __device__ void gather_texel_refill(const GatherArgs& A, uint32_t ti, uint32_t l
                 const bool refill = next < n && qtail - qhead < 64u;
                 const uint32_t yield_at = refill ? 64u - kGatherRefill : 0u;
                 auto flt = gather_filter<FEAT>(A, stri, near_t, 0, rug_below);
-                if (trace_resume<STACK>(S, flt, A.sc.col, ls, yield_at)) {
+                if (trace_resume<STACK, false>(S, flt, A.sc.col, ls, yield_at)) {
                     busy = false;
                     // a hit reads the exitance of the side it sees; a ray that leaves the
                     // scene returns environment * multiplier, or nothing

@@ -205,6 +205,31 @@ __device__ inline bool trace_begin(TraceState& S, const ColliderView& c, const f
     return true;
 }
 
+// One triangle against the ray: slot p with plane pl and record (sv, ev, mt) (all zero where
+// the caller has not read it: LATE reads it here, once the plane test passes).
+template <bool WIDE, bool LATE, class Filter>
+__device__ inline void test_triangle(TraceState& S, const Filter& flt, const ColliderView& c, uint32_t p, const float4 pl, float4 sv,
+                                     float4 ev, uint4 mt)
+{
+    float ndd;
+    const float t = plane_distance(pl, S.o, S.d, ndd);
+    if (!(t >= S.lo && t <= S.bound)) return;
+    if constexpr (LATE) {
+        // the whole record in one round trip
+        sv = load_at<WIDE, float4>(c.rest, p, 48u, 0u); ev = load_at<WIDE, float4>(c.rest, p, 48u, 16u);
+        mt = load_at<WIDE, uint4>(c.rest, p, 48u, 32u);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    float u, v;
+    if (!srlnp_hit(sv, ev, mt.z, S.o, S.d, t, u, v)) return;
+    // a tie goes to the lower triangle index
+    if (t == S.best && S.slot != kNoSlot && mt.x >= load_at<WIDE, uint32_t>(c.rest, S.slot, 48u, 32u)) return;
+    if (!flt.accept(mt.x, ndd < 0, t, u, v)) return;
+    S.best = t; S.slot = p;
+    S.bound = flt.clamp(t);
+    if (flt.done(t)) S.ref = kDone;
+}
+
 // Loop shape: "while-while" with speculative traversal (Aila & Laine, HPG 2009).
 // Lanes descend inner nodes; a lane that reaches a leaf parks it and keeps
 // descending, until every lane of the wave holds a parked leaf; then the wave tests
@@ -215,7 +240,9 @@ __device__ inline bool trace_begin(TraceState& S, const ColliderView& c, const f
 // asks whether a blocker lies below rugDistance and, if not, whether any blocker lies in
 // range; after the first hit its range shrinks below rugDistance and the search there is
 // exhaustive, so the answer does not depend on the order, and the sort is saved.
-template <int STACK, bool STATS, class Filter, bool ORDERED, bool YIELD>
+// EAGER (scattered rays, bound by latency): a leaf's triangles are read two at a time with
+// plane and record together, one memory round trip instead of four.
+template <int STACK, bool STATS, class Filter, bool ORDERED, bool YIELD, bool EAGER>
 __device__ inline bool trace_run(TraceState& S, const Filter& flt, const ColliderView& c, const LaneStack& stk, uint32_t yield_at,
                                  uint32_t& nvis, uint32_t& ntest)
 {
@@ -236,24 +263,25 @@ __device__ inline bool trace_run(TraceState& S, const Filter& flt, const Collide
         while (S.leaf < 0) {
             const uint32_t st = leaf_start(S.leaf), end = st + leaf_count(S.leaf);
             S.leaf = 0;
-            for (uint32_t p = st; p < end; p++) {
-                if (STATS) ntest++;
-                const float4 pl = load_at<WIDE, float4>(c.plane, p, 16u, 0u);
-                float ndd;
-                const float t = plane_distance(pl, S.o, S.d, ndd);
-                if (!(t >= S.lo && t <= S.bound)) continue;
-                // the whole record in one round trip
-                const float4 sv = load_at<WIDE, float4>(c.rest, p, 48u, 0u), ev = load_at<WIDE, float4>(c.rest, p, 48u, 16u);
-                const uint4 mt = load_at<WIDE, uint4>(c.rest, p, 48u, 32u);
-                __builtin_amdgcn_sched_barrier(0);
-                float u, v;
-                if (!srlnp_hit(sv, ev, mt.z, S.o, S.d, t, u, v)) continue;
-                // a tie goes to the lower triangle index
-                if (t == S.best && S.slot != kNoSlot && mt.x >= load_at<WIDE, uint32_t>(c.rest, S.slot, 48u, 32u)) continue;
-                if (!flt.accept(mt.x, ndd < 0, t, u, v)) continue;
-                S.best = t; S.slot = p;
-                S.bound = flt.clamp(t);
-                if (flt.done(t)) { S.ref = kDone; break; }
+            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+            if constexpr (EAGER) {
+                for (uint32_t p = st; p < end; p += 2) {
+                    const uint32_t q = min(p + 1, end - 1);
+                    const float4 pl0 = load_at<WIDE, float4>(c.plane, p, 16u, 0u), pl1 = load_at<WIDE, float4>(c.plane, q, 16u, 0u);
+                    const float4 sv0 = load_at<WIDE, float4>(c.rest, p, 48u, 0u), ev0 = load_at<WIDE, float4>(c.rest, p, 48u, 16u);
+                    const float4 sv1 = load_at<WIDE, float4>(c.rest, q, 48u, 0u), ev1 = load_at<WIDE, float4>(c.rest, q, 48u, 16u);
+                    const uint4 mt0 = load_at<WIDE, uint4>(c.rest, p, 48u, 32u), mt1 = load_at<WIDE, uint4>(c.rest, q, 48u, 32u);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (STATS) ntest += q - p + 1;
+                    test_triangle<WIDE, false>(S, flt, c, p, pl0, sv0, ev0, mt0);
+                    if (q != p) test_triangle<WIDE, false>(S, flt, c, q, pl1, sv1, ev1, mt1);
+                }
+            } else {
+                for (uint32_t p = st; p < end; p++) {
+                    if (STATS) ntest++;
+                    test_triangle<WIDE, true>(S, flt, c, p, load_at<WIDE, float4>(c.plane, p, 16u, 0u), zero, zero, make_uint4(0u, 0u, 0u, 0u));
+                    if (S.ref == kDone && flt.done(S.best)) break;
+                }
             }
             if (S.ref < 0) { S.leaf = S.ref; S.ref = stk.pop(S.top); }
         }
@@ -261,11 +289,11 @@ __device__ inline bool trace_run(TraceState& S, const Filter& flt, const Collide
     return true;
 }
 
-template <int STACK, class Filter>
+template <int STACK, bool EAGER, class Filter>
 __device__ inline bool trace_resume(TraceState& S, const Filter& flt, const ColliderView& c, const LaneStack& stk, uint32_t yield_at)
 {
     uint32_t a = 0, b = 0;
-    return trace_run<STACK, false, Filter, true, true>(S, flt, c, stk, yield_at, a, b);
+    return trace_run<STACK, false, Filter, true, true, EAGER>(S, flt, c, stk, yield_at, a, b);
 }
 
 // the hit of a finished ray (tri -1: none)
@@ -282,7 +310,7 @@ __device__ inline void trace_finish(const TraceState& S, const ColliderView& c, 
 }
 
 // the whole ray at once
-template <int STACK, bool STATS, class Filter, bool ORDERED = true>
+template <int STACK, bool STATS, class Filter, bool ORDERED = true, bool EAGER = false>
 __device__ inline void trace_closest(const Filter& flt, const ColliderView& c, const float3 o, const float3 d, float rmin, float rmax,
                                      int32_t* stk, int stride, TraceResult& res, uint32_t& nvis, uint32_t& ntest)
 {
@@ -290,7 +318,7 @@ __device__ inline void trace_closest(const Filter& flt, const ColliderView& c, c
     const LaneStack ls(stk, stride);
     res.tri = -1;
     if (!trace_begin(S, c, o, d, rmin, rmax, ls)) return;
-    trace_run<STACK, STATS, Filter, ORDERED, false>(S, flt, c, ls, 0u, nvis, ntest);
+    trace_run<STACK, STATS, Filter, ORDERED, false, EAGER>(S, flt, c, ls, 0u, nvis, ntest);
     trace_finish(S, c, res);
 }
 

@@ -288,3 +288,27 @@ def test_gpu_node_boxes_at_any_scale(gpu, oracle, scale, offset):
     o = oracle.intersect_linear_srlnp(V, I, R)
     assert (o["tri"] >= 0).mean() > 0.2
     _same_hits(g, gf, o, o)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 63, 257, 16385, 16389, 262145, 400_001])
+def test_gpu_batch_sizes(gpu, oracle, n):
+    """Every launch shape of a device batch (rays spread over few lanes of many waves, full waves,
+    the ray queue) answers each ray once, as the oracle does; rays past the batch are untouched."""
+    from lightsprintsdk_amd.collider import RRCollider, DeviceRays
+    V, I = scenes.icosphere(6, seed=3)
+    base = scenes.random_rays(V, 4093, seed=8)
+    o = oracle.intersect_linear_srlnp(V, I, base)
+    pick = np.arange(n + 5) % len(base)
+    col = RRCollider.create(V, I)
+    rays = DeviceRays(base[pick])
+    rays.hits.upload(np.full((n + 5, 4), 7, np.int32))
+    rays.n = n
+    for _ in range(2):
+        col.intersect_device(rays)
+    rays.n = n + 5
+    g, gf = rays.download_hits()
+    ref = o[pick[:n]]
+    np.testing.assert_array_equal(g["tri"][:n], ref["tri"])
+    m = ref["tri"] >= 0
+    np.testing.assert_array_equal(g["t"][:n][m], ref["t"][m])
+    np.testing.assert_array_equal(g.view(np.int32).reshape(-1, 4)[n:], 7)
