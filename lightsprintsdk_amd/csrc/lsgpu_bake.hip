@@ -272,9 +272,10 @@ int lsg_bake_create(lsg_scene* scene, const lsg_bake_object* objects, uint32_t n
     AL(B.d_emit, 12 * (size_t)B.ntri); UP(B.d_emit, emittance, 12 * (size_t)B.ntri);
 #undef AL
 #undef UP
-    int st = maps_upload(B.maps.data(), B.nmaps, &B.d_maps, &B.ftotal);
+    uint32_t tiles = 0;
+    int st = maps_upload(B.maps.data(), B.nmaps, &B.d_maps, &B.ftotal, &tiles);
     if (st) return bail(st);
-    if ((st = scratch_alloc(B.S, B.ftotal))) return bail(st);
+    if ((st = scratch_alloc(B.S, B.ftotal, tiles))) return bail(st);
     int dev = 0;
     (void)hipGetDevice(&dev);
     hipDeviceProp_t prop;

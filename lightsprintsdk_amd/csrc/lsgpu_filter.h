@@ -9,15 +9,21 @@ struct FilterMap {
     uint32_t base;       // float4 slot of texel (0,0) in the RGBA buffer
     uint32_t out_base;   // RGBF texel slot of texel (0,0) in the output buffer
     uint32_t width, height;
+    uint32_t tfirst;     // first lightmapGrow tile of this map in the batch's tile numbering
 };
+
+// lightmapGrow works on tiles of kTile x kTile texels (row-major per map)
+constexpr uint32_t kTile = 32;
+inline uint32_t map_tiles(uint32_t width, uint32_t height) { return ((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile); }
 
 struct FilterScratch {
     float4* a = nullptr; float4* b = nullptr; float4* c = nullptr;
     uint8_t* flags = nullptr;
-    uint32_t* changed = nullptr;   // [0] last step changed; [1..3] frontier sizes; [4..19] step log
-    uint32_t* front[2] = {nullptr, nullptr};   // lightmapGrow frontiers (texel indices)
-    uint32_t* mark = nullptr;      // step + 1 at which a texel was queued in a frontier, 0 = never
-    uint32_t* host_log = nullptr;  // pinned: two chunks of frontier sizes read by the host
+    uint32_t* changed = nullptr;   // [0] last step changed; [1] last step that filled a texel (wrap: [1..3] frontier sizes, [4..19] step log)
+    uint32_t* front[2] = {nullptr, nullptr};   // lightmapGrow: tile states in [0]; with wrap the frontiers (texel indices)
+    uint32_t* mark = nullptr;      // step at which a texel was filled; with wrap step + 1 at which it was queued, 0 = never
+    uint32_t tiles = 0;            // lightmapGrow tiles of the batch (at most one per texel)
+    uint32_t* host_log = nullptr;  // pinned: two chunks of step logs read by the host
     hipEvent_t ev[2] = {nullptr, nullptr};
 };
 
@@ -44,12 +50,12 @@ struct SeamStore {
 int seams_set(SeamStore& S, uint32_t nmaps, const lsg_unwrap_seam* seams, const uint32_t* begin);
 void seams_free(SeamStore& S);
 
-int maps_upload(const lsg_lightmap* maps, uint32_t nmaps, FilterMap** d_maps, uint32_t* total);
-int scratch_alloc(FilterScratch& S, uint32_t total);
+int maps_upload(const lsg_lightmap* maps, uint32_t nmaps, FilterMap** d_maps, uint32_t* total, uint32_t* tiles);
+int scratch_alloc(FilterScratch& S, uint32_t total, uint32_t tiles);
 void scratch_free(FilterScratch& S);
-// fixed_steps < 0: lightmapGrow iterates until a step changes nothing (host checks
-// every 16 steps, one chunk behind the GPU); fixed_steps >= 0: exactly that many steps, no host sync (graph
-// capture), S.changed[0] = whether the last step still changed a texel.
+// fixed_steps < 0: lightmapGrow iterates until a step changes nothing (the host checks
+// one chunk of launches behind the GPU); fixed_steps >= 0: exactly that many steps, no host sync (graph
+// capture), S.changed[0] = whether the last step still changed a texel and more were allowed.
 int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* rgba, float* rgbf,
                const lsg_filter_params& fp, FilterScratch& S, hipStream_t s, bool rgba_out,
                int fixed_steps, uint32_t* steps_used, const SeamSet* seams = nullptr);

@@ -24,6 +24,8 @@ enum { QUADRANT_X0Y0 = 1, QUADRANT_X1Y0 = 2, QUADRANT_X0Y1 = 4, QUADRANT_X1Y1 = 
 
 __device__ inline uint32_t to_flags(float a) { return (uint32_t)(a * 255 + 0.5f); }  // FLOAT_TO_TEXELFLAGS
 
+constexpr uint32_t kEmpty = 0xffffffffu;    // mark of a texel lightmapGrow has not filled
+
 // map lookup: texel t -> (map index) by binary search over the prefix of texel counts
 __device__ inline uint32_t find_map(const FilterMap* maps, uint32_t nmaps, uint32_t t)
 {
@@ -116,7 +118,8 @@ __global__ __launch_bounds__(256) void k_smooth_finish(const FilterMap* __restri
 }
 
 __global__ __launch_bounds__(256) void k_grow_bilinear(const FilterMap* __restrict__ maps, uint32_t nmaps, uint32_t total,
-                                                       const float4* __restrict__ rgba, float4* __restrict__ out, int wrap)
+                                                       const float4* __restrict__ rgba, float4* __restrict__ out,
+                                                       uint32_t* __restrict__ mark, int wrap)
 {
     const uint32_t t = blockIdx.x * 256 + threadIdx.x;
     if (t >= total) return;
@@ -143,9 +146,189 @@ __global__ __launch_bounds__(256) void k_grow_bilinear(const FilterMap* __restri
         if (sum.w != 0) c = make_float4(sum.x / sum.w, sum.y / sum.w, sum.z / sum.w, 0.001f);
     }
     out[t] = c;
+    if (mark) mark[t] = c.w > 0 ? 0u : kEmpty;     // lightmapGrow's start state (RRBuffer.cpp:889-893)
 }
 
-// lightmapGrow init (RRBuffer.cpp:889-893)
+// lightmapGrow on tiles.  The reference's step (RRBuffer.cpp:897-947) fills every empty texel
+// that has a filled neighbour in the previous state with 1.6 x the 4 edge neighbours + the 4
+// corner neighbours, divided by their weights, so what a texel becomes depends only on
+// texels within s of it s steps earlier.  A workgroup takes a tile of 32 x 32 texels with a
+// halo of 16 into LDS (64 x 64 texels, one 64-bit word per row says which are filled), runs up
+// to 16 steps there -- the texels whose state is still exact shrink by one per step on every
+// side, the tile's own stay exact -- and writes the tile's new texels with the step that
+// filled them (mark).  Another tile's texels filled in this launch carry a mark above `base`
+// and count as empty, whether or not they have arrived, so tiles need no order.  info:
+// bit 0 = the tile has filled texels, bit 1 = empty ones; a tile with nothing to fill, or with
+// nothing filled around it, is passed over.
+//
+// In a step every wave keeps the words of all 64 rows (lane = row), so each finds the whole
+// step's texels from registers, lists those of its own 8 columns and fills them 64 at a time: the
+// eight 16-byte LDS reads per texel bound a step, and a row of a wave each would
+// read 4 to 10 times as often for the few texels a row has.  A texel's w is the step that
+// filled it, so what this step writes is not yet seen by it: one barrier per step.
+//
+// One launch does what 16 launches over a frontier list did (each a few hundred to a few
+// thousand texels: 8 to 16 us of launch and latency).  5 maps of 1013 x 731, 96 steps: 1.54 ms +
+// 0.26 ms to seed the list -> 0.55 ms (8 launches of 68 us; reading the marks with their
+// halos alone takes 12 us); a light-layer call of 9 maps of 97^2, five chains: 5.6 -> 2.9 ms.  256
+// threads a tile: 0.72 ms, 1024: 0.58 ms (two workgroups per CU either way, by LDS).
+constexpr uint32_t kHalo = 16, kRegion = 64, kTileSteps = 16, kTileThreads = 512, kTileWaves = kTileThreads / 64;
+constexpr uint32_t kStrip = kRegion / kTileWaves;       // columns of a wave
+constexpr uint32_t kValPitch = kRegion + 1;             // odd: a column's texels lie in different banks
+constexpr float kNever = 1e9f;
+
+__device__ inline uint64_t row_above(uint64_t v)        // the word of lane - 1 (0 for lane 0)
+{
+    return (uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, 0x138, 0xf, 0xf, true) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), 0x138, 0xf, 0xf, true) << 32;
+}
+__device__ inline uint64_t row_below(uint64_t v)        // the word of lane + 1 (0 for lane 63)
+{
+    return (uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, 0x130, 0xf, 0xf, true) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), 0x130, 0xf, 0xf, true) << 32;
+}
+
+__global__ __launch_bounds__(kTileThreads) void k_grow_tiles(const FilterMap* __restrict__ maps, uint32_t nmaps, uint32_t ntiles,
+                                                             float4* __restrict__ img, uint32_t* __restrict__ mark, uint32_t* __restrict__ info,
+                                                             uint32_t base, uint32_t nsteps, uint32_t* __restrict__ last_step)
+{
+    __shared__ float4 val[kRegion * kValPitch];         // w = step that filled the texel (0 before this launch, kNever = empty)
+    __shared__ uint64_t fill0[kRegion], empty0[kRegion];
+    __shared__ uint16_t list[kTileWaves][kRegion * kStrip];
+    __shared__ uint64_t todo[kTileWaves];
+    __shared__ uint32_t tmap[kTileThreads];
+    __shared__ uint32_t block_last;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+    uint32_t last = 0;                                  // the last step in which this thread filled a texel
+    if (tid == 0) block_last = 0;
+    for (uint64_t batch = blockIdx.x; batch < ntiles; batch += (uint64_t)gridDim.x * kTileThreads) {
+        // which of this workgroup's next tiles have work: one thread looks at each
+        const uint64_t t64 = batch + (uint64_t)tid * gridDim.x;
+        bool work = false;
+        uint32_t mi = 0;
+        if (t64 < ntiles) {
+            const uint32_t t = (uint32_t)t64;
+            uint32_t lo = 0, hi = nmaps;
+            while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (maps[mid].tfirst <= t) lo = mid; else hi = mid; }
+            mi = lo;
+            work = base == 0;
+            if (!work && (info[t] & 2u)) {
+                const int tw = (int)((maps[mi].width + kTile - 1) / kTile), th = (int)((maps[mi].height + kTile - 1) / kTile);
+                const int k = (int)(t - maps[mi].tfirst), x = k % tw, y = k / tw;
+                for (int j = max(y - 1, 0); j <= min(y + 1, th - 1); j++)
+                    for (int i = max(x - 1, 0); i <= min(x + 1, tw - 1); i++) work = work || (info[maps[mi].tfirst + (uint32_t)(j * tw + i)] & 1u);
+            }
+        }
+        tmap[tid] = mi;
+        const uint64_t wm = __ballot(work);
+        if (lane == 0) todo[wave] = wm;
+        __syncthreads();
+        for (uint32_t word = 0; word < kTileWaves; word++)
+            for (uint64_t rest = todo[word]; rest; rest &= rest - 1) {
+                const uint32_t slot = word * 64u + (uint32_t)__ffsll((unsigned long long)rest) - 1u;
+                const uint32_t t = (uint32_t)(batch + (uint64_t)slot * gridDim.x);
+                const FilterMap M = maps[tmap[slot]];
+                const int w = (int)M.width, h = (int)M.height;
+                const uint32_t per_row = (M.width + kTile - 1) / kTile, k = t - M.tfirst;
+                const int x0 = (int)((k % per_row) * kTile) - (int)kHalo, y0 = (int)((k / per_row) * kTile) - (int)kHalo;
+                const int x = x0 + (int)lane;
+                const bool col = x >= 0 && x < w;
+                // rows of this wave: wave, wave + 8, ...; which texels are filled and which empty
+#pragma unroll
+                for (uint32_t r = wave; r < kRegion; r += kTileWaves) {
+                    const int y = y0 + (int)r;
+                    const bool in = col && y >= 0 && y < h;
+                    const uint32_t m = in ? mark[M.first + (uint32_t)(x + y * w)] : 0u;
+                    const uint64_t f = __ballot(in && m <= base), e = __ballot(in && m > base);
+                    if (lane == 0) { fill0[r] = f; empty0[r] = e; }
+                }
+                __syncthreads();
+                // values of the filled texels next to an empty one; the others are never read
+#pragma unroll
+                for (uint32_t r = wave; r < kRegion; r += kTileWaves) {
+                    uint64_t e = empty0[r];
+                    if (r > 0) e |= empty0[r - 1];
+                    if (r < kRegion - 1) e |= empty0[r + 1];
+                    e |= (e << 1) | (e >> 1);
+                    float4 c = make_float4(0.f, 0.f, 0.f, kNever);
+                    if ((e & fill0[r]) >> lane & 1u) {
+                        c = img[M.first + (uint32_t)(x + (y0 + (int)r) * w)];
+                        c.w = 0.f;
+                    }
+                    val[r * kValPitch + lane] = c;
+                }
+                uint64_t filled = fill0[lane];
+                const uint64_t empty = empty0[lane];
+                __syncthreads();
+                const uint64_t strip = ((1ull << kStrip) - 1ull) << (wave * kStrip);
+                for (uint32_t s = 1; s <= nsteps; s++) {
+                    uint64_t f = row_above(filled) | filled | row_below(filled);
+                    f |= (f << 1) | (f >> 1);
+                    f &= empty & ~filled & (~0ull << s) & (~0ull >> s);
+                    if (lane < s || lane >= kRegion - s) f = 0;
+                    if (!__any(f != 0)) break;          // nothing more can be filled here (the same in every wave)
+                    filled |= f;
+                    uint32_t count = 0;
+                    uint64_t own = f & strip;
+                    for (uint64_t b = __ballot(own != 0); b; b = __ballot(own != 0)) {
+                        if (own) {
+                            const uint32_t c = (uint32_t)__ffsll((unsigned long long)own) - 1u;
+                            list[wave][count + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = (uint16_t)(lane * kRegion + c);
+                            own &= own - 1;
+                        }
+                        count += (uint32_t)__popcll((unsigned long long)b);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    for (uint32_t i = lane; i < count; i += 64) {
+                        const uint32_t at = list[wave][i];
+                        const int xc = (int)(at % kRegion), yc = (int)(at / kRegion), gx = x0 + xc, gy = y0 + yc;
+                        // neighbours clamped to the map (RRBuffer.cpp:930-941)
+                        const int xp = min(gx + 1, w - 1) - x0, xm = max(gx - 1, 0) - x0;
+                        const int yp = min(gy + 1, h - 1) - y0, ym = max(gy - 1, 0) - y0;
+                        const float sf = (float)s;
+                        auto old = [&](int i2, int j2) {
+                            const float4 v = val[j2 * (int)kValPitch + i2];
+                            const bool ok = v.w < sf;
+                            return make_float4(ok ? v.x : 0.f, ok ? v.y : 0.f, ok ? v.z : 0.f, ok ? 1.f : 0.f);
+                        };
+                        const float4 e = f4add(f4add(f4add(old(xp, yc), old(xm, yc)), old(xc, yp)), old(xc, ym));
+                        const float4 dg = f4add(f4add(f4add(old(xp, yp), old(xp, ym)), old(xm, yp)), old(xm, ym));
+                        const float4 d = f4add(f4mul(e, 1.6f), dg);
+                        const float4 nv = make_float4(d.x / d.w, d.y / d.w, d.z / d.w, sf);
+                        val[yc * (int)kValPitch + xc] = nv;
+                        if ((uint32_t)xc - kHalo < kTile && (uint32_t)yc - kHalo < kTile) {
+                            const uint32_t g = M.first + (uint32_t)(gx + gy * w);
+                            img[g] = make_float4(nv.x, nv.y, nv.z, 0.001f);
+                            mark[g] = base + s;
+                            last = base + s;
+                        }
+                    }
+                    __syncthreads();
+                }
+                if (wave == 0) {
+                    const uint64_t tile = ((1ull << kTile) - 1ull) << kHalo;
+                    const bool row = lane >= kHalo && lane < kHalo + kTile;
+                    const uint64_t hf = __ballot(row && (filled & tile)), he = __ballot(row && (empty & ~filled & tile));
+                    if (lane == 0) info[t] = (hf ? 1u : 0u) | (he ? 2u : 0u);
+                }
+                __syncthreads();
+            }
+        __syncthreads();
+    }
+    if (last) atomicMax(&block_last, last);
+    __syncthreads();
+    if (tid == 0 && block_last) atomicMax(last_step, block_last);
+}
+
+// after a fixed number of steps: did the last one still fill a texel?
+__global__ void k_grow_changed(const uint32_t* __restrict__ last_step, uint32_t n, uint32_t* __restrict__ changed)
+{
+    if (threadIdx.x == 0) changed[0] = *last_step == n ? 1u : 0u;
+}
+
+// lightmapGrow init (RRBuffer.cpp:889-893), for the wrapped form below
 __global__ __launch_bounds__(256) void k_grow_init(uint32_t total, const float4* __restrict__ img, float4* __restrict__ g)
 {
     const uint32_t t = blockIdx.x * 256 + threadIdx.x;
@@ -154,7 +337,8 @@ __global__ __launch_bounds__(256) void k_grow_init(uint32_t total, const float4*
     g[t] = c.w > 0 ? make_float4(c.x, c.y, c.z, 1.f) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// lightmapGrow by frontiers.  The reference's step (RRBuffer.cpp:897-947) changes exactly
+// lightmapGrow by frontiers, for wrapped maps (their neighbours are flat texel numbers, not a
+// neighbourhood that tiles).  The reference's step (RRBuffer.cpp:897-947) changes exactly
 // the empty texels that have a filled neighbour in the previous state, and those are the
 // still-empty texels that count a texel filled one step earlier among their neighbours.
 // So each step visits only its frontier: every frontier texel's value is computed from
@@ -467,6 +651,9 @@ __global__ __launch_bounds__(64) void k_seam_pass(const FilterMap* __restrict__ 
 
 static inline unsigned nblk(uint32_t n) { return (n + 255) / 256; }
 
+constexpr uint32_t kGrowBlocks = 512;                 // two workgroups of k_grow_tiles per CU
+constexpr uint32_t kGrowChunk = 2 * kTileSteps;       // steps between the host's looks
+
 __global__ void k_zero_u32(uint32_t* p, uint32_t n)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -496,12 +683,55 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
         k_smooth_finish<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, src);
     }
     // lightmapGrowForBilinearInterpolation
-    k_grow_bilinear<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, S.c, fp.wrap);
+    uint32_t steps = (uint32_t)(fp.spread_foreground > 0 ? fp.spread_foreground : 0);
+    k_grow_bilinear<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, S.c, steps && !fp.wrap ? S.mark : nullptr, fp.wrap);
     // lightmapGrow(spread)
     const float4* g = nullptr;
-    uint32_t steps = (uint32_t)(fp.spread_foreground > 0 ? fp.spread_foreground : 0);
     if (steps_used) *steps_used = 0;
-    if (steps) {
+    if (steps && !fp.wrap) {
+        // launches of 16 steps over the tiles, in place in S.c; S.changed[1] = the last step
+        // that filled a texel.  A launch whose last step filled nothing is the end: the
+        // reference stops at the first step that changes nothing (RRBuffer.cpp:948-949).
+        k_zero_u32<<<1, 256, 0, s>>>(S.changed, 20);
+        const unsigned grid = std::min(S.tiles, kGrowBlocks);
+        auto launch = [&](uint32_t b, uint32_t e) {
+            for (uint32_t q = b; q < e; q += kTileSteps)
+                k_grow_tiles<<<grid, kTileThreads, 0, s>>>(d_maps, nmaps, S.tiles, S.c, S.mark, S.front[0], q, std::min(kTileSteps, e - q), S.changed + 1);
+        };
+        if (fixed_steps >= 0) {
+            // graph-capturable form: a fixed number of steps, no host synchronisation
+            const uint32_t n = std::min<uint32_t>((uint32_t)fixed_steps, steps);
+            launch(0, n);
+            if (n && n < steps) k_grow_changed<<<1, 64, 0, s>>>(S.changed + 1, n, S.changed);
+            if (steps_used) *steps_used = n;
+        } else {
+            // chunks of launches, each followed by a copy of the last filling step; with pinned
+            // memory and events the host looks at chunk k while chunk k + 1 already runs
+            const uint32_t nchunks = steps / kGrowChunk + (steps % kGrowChunk ? 1u : 0u);
+            const bool ahead = S.host_log != nullptr;
+            uint32_t own[2];
+            uint32_t* log = ahead ? S.host_log : own;
+            auto chunk = [&](uint32_t k) -> hipError_t {
+                launch(k * kGrowChunk, std::min(steps, (k + 1) * kGrowChunk));
+                hipError_t r = hipMemcpyAsync(log + (k & 1u), S.changed + 1, 4, hipMemcpyDeviceToHost, s);
+                if (r == hipSuccess && ahead) r = hipEventRecord(S.ev[k & 1u], s);
+                return r;
+            };
+            auto wait = [&](uint32_t k) -> hipError_t { return ahead ? hipEventSynchronize(S.ev[k & 1u]) : hipStreamSynchronize(s); };
+            uint32_t k = 0, last = 0;
+            LSG_HIP(chunk(0));
+            for (;; k++) {
+                if (ahead && k + 1 < nchunks) LSG_HIP(chunk(k + 1));
+                LSG_HIP(wait(k));
+                last = log[k & 1u];
+                if (k + 1 >= nchunks || last < (k + 1) * kGrowChunk) break;
+                if (!ahead) LSG_HIP(chunk(k + 1));
+            }
+            // the chunk launched ahead must finish its copy before the buffers are reused
+            if (ahead && k + 1 < nchunks) LSG_HIP(wait(k + 1));
+            if (steps_used) *steps_used = std::min(steps, last + 1);
+        }
+    } else if (steps) {
         // frontier sizes rotate over S.changed[1..3] (step q reads [1 + q % 3]); step q reads
         // front[q & 1] and queues into the other list
         k_grow_init<<<nblk(total), 256, 0, s>>>(total, S.c, S.a);
@@ -579,9 +809,10 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
     return LSG_OK;
 }
 
-int scratch_alloc(FilterScratch& S, uint32_t total)
+int scratch_alloc(FilterScratch& S, uint32_t total, uint32_t tiles)
 {
     hipError_t e;
+    S.tiles = tiles;
     const size_t n = total ? total : 1;
     if ((e = hipMalloc(&S.a, 16 * n)) != hipSuccess) return hip_fail(e, "hipMalloc", __LINE__);
     if ((e = hipMalloc(&S.b, 16 * n)) != hipSuccess) return hip_fail(e, "hipMalloc", __LINE__);
@@ -652,14 +883,16 @@ int seams_set(SeamStore& S, uint32_t nmaps, const lsg_unwrap_seam* seams, const 
     return LSG_OK;
 }
 
-int maps_upload(const lsg_lightmap* maps, uint32_t nmaps, FilterMap** d_maps, uint32_t* total)
+int maps_upload(const lsg_lightmap* maps, uint32_t nmaps, FilterMap** d_maps, uint32_t* total, uint32_t* tiles)
 {
     std::vector<FilterMap> fm(nmaps);
-    uint32_t t = 0;
+    uint32_t t = 0, tl = 0;
     for (uint32_t m = 0; m < nmaps; m++) {
         if (!maps[m].width || !maps[m].height) return fail(LSG_ERR_INVALID, "lightmap %u has zero size", m);
         fm[m].first = t; fm[m].base = maps[m].rgba_base; fm[m].out_base = maps[m].rgbf_base;
         fm[m].width = maps[m].width; fm[m].height = maps[m].height;
+        fm[m].tfirst = tl;
+        tl += map_tiles(maps[m].width, maps[m].height);
         uint64_t nt = (uint64_t)t + (uint64_t)maps[m].width * maps[m].height;
         if (nt >= (1ull << 32)) return fail(LSG_ERR_LIMIT, "more than 2^32 texels");
         t = (uint32_t)nt;
@@ -667,7 +900,7 @@ int maps_upload(const lsg_lightmap* maps, uint32_t nmaps, FilterMap** d_maps, ui
     hipError_t e;
     if ((e = hipMalloc(d_maps, sizeof(FilterMap) * (nmaps ? nmaps : 1))) != hipSuccess) return hip_fail(e, "hipMalloc", __LINE__);
     if (nmaps && (e = hipMemcpy(*d_maps, fm.data(), sizeof(FilterMap) * nmaps, hipMemcpyHostToDevice)) != hipSuccess) return hip_fail(e, "h2d", __LINE__);
-    *total = t;
+    *total = t; *tiles = tl;
     return LSG_OK;
 }
 
@@ -675,7 +908,7 @@ int maps_upload(const lsg_lightmap* maps, uint32_t nmaps, FilterMap** d_maps, ui
 
 struct lsg_filter_plan {
     lsg::FilterMap* d_maps = nullptr;
-    uint32_t nmaps = 0, total = 0;
+    uint32_t nmaps = 0, total = 0, tiles = 0;
     lsg::FilterScratch S;
     lsg::SeamStore seams;
 };
@@ -689,8 +922,8 @@ extern "C" int lsg_filter_plan_create(const lsg_lightmap* maps, uint32_t nmaps, 
     if (!maps && nmaps) return fail(LSG_ERR_INVALID, "lsg_filter_plan_create: null maps");
     lsg_filter_plan* f = new (std::nothrow) lsg_filter_plan;
     if (!f) return fail(LSG_ERR_OOM, "lsg_filter_plan_create: host allocation");
-    int st = maps_upload(maps, nmaps, &f->d_maps, &f->total);
-    if (!st) st = scratch_alloc(f->S, f->total);
+    int st = maps_upload(maps, nmaps, &f->d_maps, &f->total, &f->tiles);
+    if (!st) st = scratch_alloc(f->S, f->total, f->tiles);
     if (st) { scratch_free(f->S); if (f->d_maps) (void)hipFree(f->d_maps); delete f; return st; }
     f->nmaps = nmaps;
     *out = f;
@@ -726,11 +959,11 @@ extern "C" int lsg_filter_lightmaps(const lsg_lightmap* maps, uint32_t nmaps, fl
 {
     if (!maps || !rgba || !params) return fail(LSG_ERR_INVALID, "lsg_filter_lightmaps: null argument");
     FilterMap* d_maps = nullptr;
-    uint32_t total = 0;
-    int st = maps_upload(maps, nmaps, &d_maps, &total);
+    uint32_t total = 0, tiles = 0;
+    int st = maps_upload(maps, nmaps, &d_maps, &total, &tiles);
     if (st) { if (d_maps) (void)hipFree(d_maps); return st; }
     FilterScratch S;
-    st = scratch_alloc(S, total);
+    st = scratch_alloc(S, total, tiles);
     if (!st) st = filter_run(d_maps, nmaps, total, (float4*)rgba, rgbf, *params, S, (hipStream_t)stream, true, -1, nullptr);
     if (!st) { hipError_t e = hipStreamSynchronize((hipStream_t)stream); if (e != hipSuccess) st = hip_fail(e, "sync", __LINE__); }
     scratch_free(S);
@@ -792,25 +1025,28 @@ static int noalloc_scratch(unsigned char** out)
 __global__ __launch_bounds__(256) void k_maps_from_lightmaps(const lsg_lightmap* __restrict__ lm, uint32_t nmaps,
                                                              FilterMap* __restrict__ fm)
 {
-    __shared__ uint32_t run[256];
+    __shared__ uint32_t run[256], trun[256];
     constexpr uint32_t kRun = (uint32_t)(kNoAllocMaps / 256);
     const uint32_t t = threadIdx.x, b = t * kRun, e = min(nmaps, b + kRun);
-    uint32_t s = 0;
-    for (uint32_t m = b; m < e; m++) s += lm[m].width * lm[m].height;
-    run[t] = s;
+    auto tiles = [](const lsg_lightmap& L) { return ((L.width + kTile - 1) / kTile) * ((L.height + kTile - 1) / kTile); };
+    uint32_t s = 0, ts = 0;
+    for (uint32_t m = b; m < e; m++) { s += lm[m].width * lm[m].height; ts += tiles(lm[m]); }
+    run[t] = s; trun[t] = ts;
     __syncthreads();
     for (uint32_t d = 1; d < 256; d *= 2) {
-        const uint32_t v = t >= d ? run[t - d] : 0u;
+        const uint32_t v = t >= d ? run[t - d] : 0u, tv = t >= d ? trun[t - d] : 0u;
         __syncthreads();
-        run[t] += v;
+        run[t] += v; trun[t] += tv;
         __syncthreads();
     }
-    uint32_t first = run[t] - s;
+    uint32_t first = run[t] - s, tfirst = trun[t] - ts;
     for (uint32_t m = b; m < e; m++) {
         const lsg_lightmap L = lm[m];
         fm[m].first = first; fm[m].base = L.rgba_base; fm[m].out_base = L.rgbf_base;
         fm[m].width = L.width; fm[m].height = L.height;
+        fm[m].tfirst = tfirst;
         first += L.width * L.height;
+        tfirst += tiles(L);
     }
 }
 static_assert(kNoAllocMaps % 256 == 0, "maps are summed in 256 runs");
@@ -822,9 +1058,11 @@ extern "C" int lsg_filter_lightmaps_noalloc(const lsg_lightmap* maps, uint32_t n
     if (!maps || !rgba || !params) return fail(LSG_ERR_INVALID, "lsg_filter_lightmaps_noalloc: null argument");
     if (nmaps > kNoAllocMaps) return fail(LSG_ERR_LIMIT, "lsg_filter_lightmaps_noalloc: %u lightmaps, at most %u", nmaps, (unsigned)kNoAllocMaps);
     uint64_t total = 0;
+    uint32_t tiles = 0;
     for (uint32_t m = 0; m < nmaps; m++) {
         if (!maps[m].width || !maps[m].height) return fail(LSG_ERR_INVALID, "lightmap %u has zero size", m);
         total += (uint64_t)maps[m].width * maps[m].height;
+        tiles += (total > kNoAllocTexels) ? 0u : map_tiles(maps[m].width, maps[m].height);
     }
     if (total > kNoAllocTexels)
         return fail(LSG_ERR_LIMIT, "lsg_filter_lightmaps_noalloc: %llu texels, at most %u", (unsigned long long)total, (unsigned)kNoAllocTexels);
@@ -842,6 +1080,7 @@ extern "C" int lsg_filter_lightmaps_noalloc(const lsg_lightmap* maps, uint32_t n
     S.front[0] = (uint32_t*)(base + kOffFront0); S.front[1] = (uint32_t*)(base + kOffFront1);
     S.mark = (uint32_t*)(base + kOffMark); S.flags = (uint8_t*)(base + kOffFlags);
     S.changed = (uint32_t*)(base + kOffChanged);
+    S.tiles = tiles;
     st = filter_run(d_maps, nmaps, (uint32_t)total, (float4*)rgba, rgbf, *params, S, s, true, -1, nullptr);
     if (!st) { hipError_t e = hipStreamSynchronize(s); if (e != hipSuccess) st = hip_fail(e, "sync", __LINE__); }
     return st;

@@ -118,6 +118,27 @@ def test_gpu_wrap_filters_vs_oracle(gpu, oracle, sigma, spread):
         plan.close()
 
 
+@pytest.mark.parametrize("spread", [1.0, 15.0, 16.0, 17.0, 32.0, 33.0, 1000.0])
+def test_gpu_grow_tiles_vs_oracle(gpu, oracle, spread):
+    """lightmapGrow at the edges of its 32-texel tiles and 16-step launches: few filled texels
+    (every tile reached from another one), full and empty maps, maps of one tile's size and
+    one texel more or less, maps one texel wide.  Same arithmetic in the same order, so the
+    bits are the oracle's."""
+    shapes = [(1, 1), (31, 32), (32, 33), (33, 31), (64, 65), (1, 200), (200, 1), (129, 97), (40, 40), (40, 40)]
+    rng = np.random.default_rng(int(spread))
+    imgs = [_random_map(rng, w, h, fill=0.002) for w, h in shapes[:-2]]
+    imgs.append(_random_map(rng, 40, 40, fill=2.0))
+    imgs.append(np.zeros((40, 40, 4), np.float32))
+    imgs[4][0, 0] = imgs[5][199, 0] = imgs[6][0, 0] = imgs[7][96, 128] = (0.5, 0.25, 1.0, 1.0)
+    plan = _FilterPlan(shapes)
+    try:
+        print(f"grow spread {spread}", flush=True)
+        _check(plan, imgs, oracle, 0.0, spread, False, tag="grow")
+        _check(plan, imgs, oracle, 1.0, spread, False, tag="blur, grow")
+    finally:
+        plan.close()
+
+
 @pytest.mark.parametrize("wrap", [False, True])
 def test_gpu_seams_vs_oracle(gpu, oracle, wrap):
     rng = np.random.default_rng(7 + wrap)
