@@ -2,19 +2,20 @@
 // matrix cores (v_mfma_f32_16x16x16_bf16: BF16 operands, FP32 accumulation).
 //
 // Network: 32 -> 64 -> 64 -> 64 -> 64 -> 4 (ReLU between layers), the last layer
-// padded to 16 outputs so every GEMM dimension is a multiple of 16.  Every product --
-// forward Z = A W, weight gradient dW = A^T dZ, input gradient dA = dZ W^T -- runs
-// through one hand-written MFMA GEMM whose operand addressing is given by strides,
-// so transposes cost nothing.  Elementwise work (bias, ReLU, BF16 rounding, loss,
-// Adam) is in small kernels.  Activations are stored in BF16 exactly where the
-// products consume them; the CPU oracle rounds at the same points.
+// padded to 16 outputs so every GEMM dimension is a multiple of 16.  Inference and the
+// training step are one kernel each, weights and activations in LDS; a training step adds a
+// second one that sums the workgroups' gradients and takes the Adam step.  Activations are
+// rounded to BF16 exactly where the products consume them; the CPU oracle rounds at the
+// same points.
 #include "lsgpu_internal.h"
+#include <algorithm>
 #include <vector>
 #include <cstring>
 #include <cmath>
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v4f4 __attribute__((ext_vector_type(4), aligned(4)));      // a caller's floats
 
 namespace lsg {
 
@@ -69,83 +70,6 @@ __global__ void k_to_bf16(const float* __restrict__ x, uint16_t* __restrict__ y,
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) y[i] = f2bf(x[i]);
-}
-
-// Z += bias (per column), A = bf16(relu(Z)) (or bf16(Z) for the last layer)
-__global__ void k_bias_act(float* __restrict__ Z, const float* __restrict__ bias, uint16_t* __restrict__ A, uint32_t rows,
-                           uint32_t cols, int relu)
-{
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * cols) return;
-    const float z = Z[i] + bias[i % cols];
-    Z[i] = z;
-    if (A) A[i] = f2bf(relu ? (z > 0.f ? z : 0.f) : z);
-}
-
-// loss and output gradient.  y[n x 16] (first 4 used), t[n x 3] targets.
-// L = mean_i [ sum_c (y_ic - t_ic)^2 + lambda (y_i3 - e_i)^2 ],  e_i = sqrt(mean_c (y_ic - t_ic)^2) (no gradient)
-__global__ void k_loss_grad(const float* __restrict__ y, const float* __restrict__ t, uint32_t n, uint32_t nvalid, float lambda,
-                            float* __restrict__ dy, uint16_t* __restrict__ dyb, float* __restrict__ loss_acc)
-{
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    float l = 0.f;
-    float g[16];
-    for (int c = 0; c < 16; c++) g[c] = 0.f;
-    if (i < nvalid && i < n) {
-        const float* yi = y + 16 * (size_t)i;
-        const float* ti = t + 3 * (size_t)i;
-        float se = 0.f;
-        for (int c = 0; c < 3; c++) { const float d = yi[c] - ti[c]; se += d * d; g[c] = 2.f * d / (float)nvalid; }
-        const float e = sqrtf(se / 3.f);
-        const float de = yi[3] - e;
-        g[3] = 2.f * lambda * de / (float)nvalid;
-        l = se + lambda * de * de;
-    }
-    if (i < n)
-        for (int c = 0; c < 16; c++) { dy[16 * (size_t)i + c] = g[c]; dyb[16 * (size_t)i + c] = f2bf(g[c]); }
-    // block reduction of the loss (every thread of the block takes part)
-    __shared__ float s[256];
-    s[threadIdx.x] = l;
-    __syncthreads();
-    for (int w = 128; w; w >>= 1) { if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w]; __syncthreads(); }
-    if (threadIdx.x == 0) atomicAdd(loss_acc, s[0]);
-}
-
-// dZ = dA * relu'(Z) rounded to bf16
-__global__ void k_relu_back(const float* __restrict__ dA, const float* __restrict__ Z, uint16_t* __restrict__ dZb,
-                            float* __restrict__ dZ, uint32_t n)
-{
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float g = Z[i] > 0.f ? dA[i] : 0.f;
-    dZ[i] = g;
-    dZb[i] = f2bf(g);
-}
-
-// db[c] = sum over rows of dZ[r][c]
-__global__ void k_colsum(const float* __restrict__ dZ, uint32_t rows, uint32_t cols, float* __restrict__ db)
-{
-    const uint32_t c = blockIdx.x;
-    float s = 0.f;
-    for (uint32_t r = threadIdx.x; r < rows; r += 256) s += dZ[(size_t)r * cols + c];
-    __shared__ float sh[256];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w; w >>= 1) { if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w]; __syncthreads(); }
-    if (threadIdx.x == 0) db[c] = sh[0];
-}
-
-// Adam (Kingma & Ba 2015) on the fp32 master parameters; mask zeroes padded outputs
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v,
-                       const uint8_t* __restrict__ mask, uint32_t n, float lr, float b1, float b2, float eps, float c1, float c2)
-{
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n || !mask[i]) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi; v[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
 // Inference in one launch: the whole network per 16-row tile, one tile per wave at a
@@ -230,6 +154,257 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float* __restrict__ x, 
     }
 }
 
+// One training step's gradients: forward, loss and backward of 64 rows at a time per
+// workgroup (16 per wave), everything in LDS, the weight gradients of all its rows in MFMA
+// accumulators (15 tiles per wave), then one partial sum per workgroup in memory.
+//   forward   Z^T = W^T A^T: a lane gets four consecutive outputs of one row, so activations
+//             are written as 8-byte pieces of rows, which the next product's operand reads
+//   backward  dA^T = W dZ^T in the same form, masked by the layer's activations
+//   dW        = A^T dZ over the workgroup's 64 rows: both operands are read along the rows
+//             of transposed copies (feature-major) written beside the row-major ones
+// Biases' gradients sum the unrounded dZ.  Loss of row i: sum_c (y_ic - t_ic)^2 + lambda (y_i3 -
+// e_i)^2, e_i = sqrt(mean_c (y_ic - t_ic)^2) held constant, averaged over the n rows.
+//
+// Bound by the chain of ten small products and their barriers, 30 us a workgroup; the products
+// are 0.9 GFLOP a step of 8192 rows, 1 us of the matrix cores.  Before, a launch per product and
+// elementwise pass (26 a step), with dW by 16 to 64 waves that each walked all rows: 0.98 ms a
+// step of 8192 rows -> 37 us (30 us + 5 us of k_mlp_update).
+constexpr int kRows = 64, kPitch = kRows + kPad;         // rows per workgroup pass; LDS pitch of 64-wide rows
+constexpr uint32_t kTrainBlocks = 256;                   // workgroups of a step, at most (one per CU)
+constexpr int kWtElems = 64 * (kFeat + kPad) + 3 * 64 * (64 + kPad) + 16 * (64 + kPad);
+constexpr int kWrElems = 3 * 64 * (64 + kPad) + 64 * (16 + kPad);
+
+__device__ inline void put4(uint16_t* p, v4f v)
+{
+    v4s b;
+    for (int i = 0; i < 4; i++) b[i] = (short)f2bf(v[i]);
+    *(v4s*)p = b;
+}
+
+__global__ __launch_bounds__(256) void k_mlp_train(const float* __restrict__ x, const float* __restrict__ t, uint32_t n, float lambda,
+                                                   const uint16_t* __restrict__ wb, const float* __restrict__ p, MlpOffsets off,
+                                                   uint32_t nparams, float* __restrict__ partial, float* __restrict__ loss_part)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t wt[kWtElems];           // W_l transposed, [out][in]
+    __shared__ __attribute__((aligned(16))) uint16_t wr[kWrElems];           // W_l of layers 1..4, [in][out]
+    __shared__ __attribute__((aligned(16))) uint16_t actT[(kFeat + 4 * 64) * kPitch];   // inputs of layer l, [feature][row]
+    __shared__ __attribute__((aligned(16))) uint16_t dzT[2][64 * kPitch];    // dZ of a layer, [output][row]
+    __shared__ __attribute__((aligned(16))) uint16_t rowbuf[4][2][16 * (64 + kPad)];    // a wave's rows, [row][feature]
+    __shared__ float bias[kBElems], dbsum[4][kBElems], lsum[4];
+    constexpr int kInL[kLayers] = {kFeat, 64, 64, 64, 64}, kOutL[kLayers] = {64, 64, 64, 64, 16};
+    constexpr int kTofs[kLayers] = {0, 64 * (kFeat + kPad), 64 * (kFeat + kPad) + 64 * (64 + kPad), 64 * (kFeat + kPad) + 2 * 64 * (64 + kPad),
+                                    64 * (kFeat + kPad) + 3 * 64 * (64 + kPad)};
+    constexpr int kRofs[kLayers] = {0, 0, 64 * (64 + kPad), 2 * 64 * (64 + kPad), 3 * 64 * (64 + kPad)};
+    constexpr int kAofs[kLayers] = {0, kFeat * kPitch, (kFeat + 64) * kPitch, (kFeat + 128) * kPitch, (kFeat + 192) * kPitch};
+    constexpr int kBofs[kLayers] = {0, 64, 128, 192, 256};
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, kq = (lane >> 4) * 4;
+#pragma unroll
+    for (int l = 0; l < kLayers; l++) {
+        const int in = kInL[l], out = kOutL[l];
+        for (int e = tid * 4; e < in * out; e += 1024) {
+            const int k = e / out, c = e % out;
+            const v4s w = *(const v4s*)(wb + off.w[l] + e);
+            for (int i = 0; i < 4; i++) wt[kTofs[l] + (c + i) * (in + kPad) + k] = (uint16_t)w[i];
+            if (l) *(v4s*)(wr + kRofs[l] + k * (out + kPad) + c) = w;
+        }
+        for (int c = tid; c < out; c += 256) bias[kBofs[l] + c] = p[off.b[l] + c];
+    }
+    auto wave_sync = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    v4f dw0[2], dw1[4], dw2[4], dw3[4], dw4 = zero, db[4][4], db4 = zero;
+#pragma unroll
+    for (int i = 0; i < 4; i++) { dw1[i] = zero; dw2[i] = zero; dw3[i] = zero; for (int l = 0; l < 4; l++) db[l][i] = zero; }
+    dw0[0] = zero; dw0[1] = zero;
+    float loss = 0.f;
+    const int myrow = wave * 16 + r;                     // the lane's row (column of the transposed products) in the pass
+    const uint64_t passes = ((uint64_t)n + kRows - 1) / kRows;
+    for (uint64_t ps = blockIdx.x; ps < passes; ps += gridDim.x) {
+        __syncthreads();                                 // weights in place; the previous pass is read
+        uint16_t* cur = rowbuf[wave][0];
+        uint16_t* nxt = rowbuf[wave][1];
+        {
+            // rows of x, four lanes each; rows past the batch are zero
+            const int rr = lane >> 2, k0 = (lane & 3) * 8;
+            const uint64_t row = ps * kRows + (uint64_t)(wave * 16 + rr);
+            v4f a = zero, b = zero;
+            if (row < n) { a = *(const v4f4*)(x + row * kFeat + k0); b = *(const v4f4*)(x + row * kFeat + k0 + 4); }
+            put4(cur + rr * (kFeat + kPad) + k0, a);
+            put4(cur + rr * (kFeat + kPad) + k0 + 4, b);
+            for (int i = 0; i < 4; i++) {
+                actT[(k0 + i) * kPitch + wave * 16 + rr] = f2bf(a[i]);
+                actT[(k0 + 4 + i) * kPitch + wave * 16 + rr] = f2bf(b[i]);
+            }
+        }
+        wave_sync();
+        const uint64_t row = ps * kRows + (uint64_t)myrow;
+        v4f y = zero;
+        uint32_t on[kLayers - 1] = {};                   // outputs past the ReLU, 16 bits a layer
+#pragma unroll
+        for (int l = 0; l < kLayers; l++) {
+            const int in = kInL[l], out = kOutL[l];
+#pragma unroll
+            for (int mt = 0; mt < out / 16; mt++) {
+                v4f acc = zero;
+#pragma unroll
+                for (int k0 = 0; k0 < in; k0 += 16)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const v4s*)(wt + kTofs[l] + (mt * 16 + r) * (in + kPad) + k0 + kq),
+                                                                    *(const v4s*)(cur + r * (in + kPad) + k0 + kq), acc, 0, 0, 0);
+                const int o = mt * 16 + kq;
+                for (int i = 0; i < 4; i++) acc[i] += bias[kBofs[l] + o + i];
+                if (l < kLayers - 1) {
+                    for (int i = 0; i < 4; i++) {
+                        if (acc[i] > 0.f) on[l] |= 1u << (mt * 4 + i);
+                        else acc[i] = 0.f;
+                    }
+                    put4(nxt + r * (64 + kPad) + o, acc);
+                    for (int i = 0; i < 4; i++) actT[kAofs[l < kLayers - 1 ? l + 1 : 0] + (o + i) * kPitch + myrow] = f2bf(acc[i]);
+                } else y = acc;
+            }
+            wave_sync();
+            uint16_t* s = cur; cur = nxt; nxt = s;
+        }
+        // loss and dY: the lanes with kq = 0 hold a row's four outputs
+        v4f g = zero;
+        if (kq == 0 && row < n) {
+            const float* ti = t + row * 3;
+            float se = 0.f;
+            for (int c = 0; c < 3; c++) { const float d = y[c] - ti[c]; se += d * d; g[c] = 2.f * d / (float)n; }
+            const float e = sqrtf(se / 3.f), de = y[3] - e;
+            g[3] = 2.f * lambda * de / (float)n;
+            loss += se + lambda * de * de;
+        }
+        put4(nxt + r * (16 + kPad) + kq, g);
+        for (int i = 0; i < 4; i++) { dzT[0][(kq + i) * kPitch + myrow] = f2bf(g[i]); db4[i] += g[i]; }
+        __syncthreads();
+        // dW of a layer: this wave's tiles, over the pass's 64 rows
+        auto grad = [&](const uint16_t* A, const uint16_t* D, int mi, int ni, v4f acc) {
+#pragma unroll
+            for (int k0 = 0; k0 < kRows; k0 += 16)
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const v4s*)(A + (mi * 16 + r) * kPitch + k0 + kq),
+                                                                *(const v4s*)(D + (ni * 16 + r) * kPitch + k0 + kq), acc, 0, 0, 0);
+            return acc;
+        };
+#pragma unroll
+        for (int l = kLayers - 1; l >= 0; l--) {
+            const uint16_t* A = actT + kAofs[l];
+            const uint16_t* D = dzT[(kLayers - 1 - l) & 1];
+            if (l == 4) dw4 = grad(A, D, wave, 0, dw4);
+            else if (l == 0) { for (int i = 0; i < 2; i++) dw0[i] = grad(A, D, i, wave, dw0[i]); }
+            else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (l == 3) dw3[i] = grad(A, D, i, wave, dw3[i]);
+                    else if (l == 2) dw2[i] = grad(A, D, i, wave, dw2[i]);
+                    else dw1[i] = grad(A, D, i, wave, dw1[i]);
+                }
+            }
+            if (l == 0) break;
+            // dA through the layer, masked by where its input passed the ReLU: the layer below's dZ
+            uint16_t* s = cur; cur = nxt; nxt = s;       // cur = this layer's dZ rows
+            wave_sync();
+            const int out = kOutL[l];
+            uint16_t* E = dzT[(kLayers - l) & 1];
+#pragma unroll
+            for (int mt = 0; mt < 4; mt++) {
+                v4f acc = zero;
+#pragma unroll
+                for (int k0 = 0; k0 < out; k0 += 16)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const v4s*)(wr + kRofs[l] + (mt * 16 + r) * (out + kPad) + k0 + kq),
+                                                                    *(const v4s*)(cur + r * (out + kPad) + k0 + kq), acc, 0, 0, 0);
+                const int o = mt * 16 + kq;
+                for (int i = 0; i < 4; i++) acc[i] = on[l - 1] >> (mt * 4 + i) & 1u ? acc[i] : 0.f;
+                db[l - 1][mt] += acc;
+                put4(nxt + r * (64 + kPad) + o, acc);
+                for (int i = 0; i < 4; i++) E[(o + i) * kPitch + myrow] = f2bf(acc[i]);
+            }
+            __syncthreads();
+        }
+    }
+    // this workgroup's partial sums
+    float* P = partial + (size_t)blockIdx.x * nparams;
+    auto store = [&](int l, int mi, int ni, v4f a) {
+        for (int i = 0; i < 4; i++) P[off.w[l] + (mi * 16 + kq + i) * kOutL[l] + ni * 16 + r] = a[i];
+    };
+    store(4, wave, 0, dw4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (i < 2) store(0, i, wave, dw0[i]);
+        store(1, i, wave, dw1[i]); store(2, i, wave, dw2[i]); store(3, i, wave, dw3[i]);
+    }
+    // biases: over the lanes of one output, then over the waves
+    auto over_rows = [&](float v) { for (int o = 8; o; o >>= 1) v += __shfl_xor(v, o); return v; };
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+#pragma unroll
+        for (int l = 0; l < 4; l++)
+#pragma unroll
+            for (int mt = 0; mt < 4; mt++) {
+                const float v = over_rows(db[l][mt][i]);
+                if (r == 0) dbsum[wave][kBofs[l] + mt * 16 + kq + i] = v;
+            }
+        const float v = over_rows(db4[i]);
+        if (r == 0) dbsum[wave][kBofs[4] + kq + i] = v;
+    }
+    loss = over_rows(loss);
+    if (lane == 0) lsum[wave] = loss;
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < kLayers; l++)
+        for (int c = tid; c < kOutL[l]; c += 256) {
+            const int b = kBofs[l] + c;
+            P[off.b[l] + c] = (dbsum[0][b] + dbsum[1][b]) + (dbsum[2][b] + dbsum[3][b]);
+        }
+    if (tid == 0) loss_part[blockIdx.x] = (lsum[0] + lsum[1]) + (lsum[2] + lsum[3]);
+}
+
+// the workgroups' partial gradients added (64 parameters per workgroup, four lanes' shares of
+// the parts each, in a fixed order) and, with lr > 0, the Adam step (Kingma & Ba 2015) on
+// the fp32 master parameters and their BF16 copies; mask keeps the padded outputs.  The first
+// workgroup also adds the loss.
+struct AdamArgs { float* p; float* m; float* v; uint16_t* wb; const uint8_t* mask; float lr, b1, b2, eps, c1, c2; };
+
+__global__ __launch_bounds__(256) void k_mlp_update(const float* __restrict__ partial, uint32_t parts, uint32_t nparams, float* __restrict__ g,
+                                                    AdamArgs A, const float* __restrict__ loss_part, float* __restrict__ loss)
+{
+    __shared__ float s[4][64];
+    const uint32_t c = threadIdx.x & 63u, q = threadIdx.x >> 6, i = blockIdx.x * 64 + c;
+    float sum = 0.f;
+    if (i < nparams) {
+#pragma unroll 8
+        for (uint32_t w = q; w < parts; w += 4) sum += partial[(size_t)w * nparams + i];
+    }
+    s[q][c] = sum;
+    __syncthreads();
+    if (q == 0 && i < nparams) {
+        const float gi = (s[0][c] + s[1][c]) + (s[2][c] + s[3][c]);
+        g[i] = gi;
+        if (A.lr > 0 && A.mask[i]) {
+            const float mi = A.b1 * A.m[i] + (1.f - A.b1) * gi;
+            const float vi = A.b2 * A.v[i] + (1.f - A.b2) * gi * gi;
+            A.m[i] = mi; A.v[i] = vi;
+            const float pi = A.p[i] - A.lr * (mi / A.c1) / (sqrtf(vi / A.c2) + A.eps);
+            A.p[i] = pi;
+            A.wb[i] = f2bf(pi);
+        }
+    }
+    if (blockIdx.x == 0) {
+        __syncthreads();
+        s[q][c] = threadIdx.x < parts ? loss_part[threadIdx.x] : 0.f;
+        __syncthreads();
+        float* f = &s[0][0];
+        for (uint32_t w = 128; w; w >>= 1) {
+            if (threadIdx.x < w) f[threadIdx.x] += f[threadIdx.x + w];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *loss = f[0];
+    }
+}
+static_assert(kTrainBlocks <= 256, "k_mlp_update adds at most 256 losses");
+
 static inline unsigned nb(uint64_t n) { return (unsigned)((n + 255) / 256); }
 
 struct MlpImpl {
@@ -237,17 +412,13 @@ struct MlpImpl {
     size_t wofs[kLayers], bofs[kLayers], nparams = 0;
     float* d_p = nullptr; float* d_g = nullptr; float* d_m = nullptr; float* d_v = nullptr; uint8_t* d_mask = nullptr;
     uint16_t* d_wb = nullptr;                    // bf16 weights (same offsets as d_p; biases unused)
-    uint16_t* d_a[kLayers + 1] = {};             // bf16 activations: a[0] = input, a[l+1] = relu(z[l])
-    float* d_z[kLayers] = {};                    // fp32 pre-activations
-    float* d_dz = nullptr; uint16_t* d_dzb = nullptr; float* d_da = nullptr;
+    float* d_part = nullptr;                     // partial gradients of a step's workgroups, then their losses
     float* d_loss = nullptr;
     uint64_t step = 0;
     ~MlpImpl()
     {
         auto f = [](void* p) { if (p) (void)hipFree(p); };
-        f(d_p); f(d_g); f(d_m); f(d_v); f(d_mask); f(d_wb); f(d_dz); f(d_dzb); f(d_da); f(d_loss);
-        for (int l = 0; l <= kLayers; l++) f(d_a[l]);
-        for (int l = 0; l < kLayers; l++) f(d_z[l]);
+        f(d_p); f(d_g); f(d_m); f(d_v); f(d_mask); f(d_wb); f(d_part); f(d_loss);
     }
 };
 
@@ -257,17 +428,6 @@ static int gemm(const uint16_t* A, int sAm, int sAk, const uint16_t* B, int sBk,
     const int tiles = (M / 16) * (N / 16);
     k_gemm_bf16<<<(tiles + 3) / 4, 256, 0, s>>>(A, sAm, sAk, B, sBk, sBn, C, ldc, M, N, K, acc);
     return LSG_OK;
-}
-
-// forward over rows [0, n) of the input already in d_a[0] (n multiple of 16)
-static void forward(MlpImpl& M, uint32_t n, hipStream_t s)
-{
-    for (int l = 0; l < kLayers; l++) {
-        const int in = kIn[l], out = kOut[l];
-        // Z[n x out] = A[n x in] * W[in x out]  (W row-major in x out)
-        gemm(M.d_a[l], in, 1, M.d_wb + M.wofs[l], out, 1, M.d_z[l], out, (int)n, out, in, 0, s);
-        k_bias_act<<<nb((uint64_t)n * out), 256, 0, s>>>(M.d_z[l], M.d_p + M.bofs[l], M.d_a[l + 1], n, out, l < kLayers - 1);
-    }
 }
 
 } // namespace lsg
@@ -294,9 +454,7 @@ int lsg_mlp_create(uint32_t max_batch, lsg_mlp** out)
     hipError_t e;
 #define AL(p, bytes) do { if ((e = hipMalloc(&(p), (bytes))) != hipSuccess) { delete m; return hip_fail(e, "hipMalloc", __LINE__); } } while (0)
     AL(M.d_p, 4 * o); AL(M.d_g, 4 * o); AL(M.d_m, 4 * o); AL(M.d_v, 4 * o); AL(M.d_mask, o); AL(M.d_wb, 2 * o);
-    for (int l = 0; l <= kLayers; l++) AL(M.d_a[l], 2 * (size_t)max_batch * (l == 0 ? kIn[0] : kOut[l - 1]));
-    for (int l = 0; l < kLayers; l++) AL(M.d_z[l], 4 * (size_t)max_batch * kOut[l]);
-    AL(M.d_dz, 4 * (size_t)max_batch * 64); AL(M.d_dzb, 2 * (size_t)max_batch * 64); AL(M.d_da, 4 * (size_t)max_batch * 64);
+    AL(M.d_part, 4 * ((size_t)kTrainBlocks * o + kTrainBlocks));
     AL(M.d_loss, 16);
 #undef AL
     std::vector<uint8_t> mask(o, 1);
@@ -367,31 +525,17 @@ int lsg_mlp_train_step(lsg_mlp* m, const float* x, const float* t, uint32_t n, f
     MlpImpl& M = m->impl;
     if (n > M.max_batch) return fail(LSG_ERR_LIMIT, "lsg_mlp_train_step: n %u > max_batch %u", n, M.max_batch);
     hipStream_t s = (hipStream_t)stream;
-    const uint32_t pad = (n + 15) / 16 * 16;
-    if (pad != n) LSG_HIP(hipMemsetAsync(M.d_a[0], 0, 2 * (size_t)pad * kFeat, s));
-    k_to_bf16<<<nb((uint64_t)n * kFeat), 256, 0, s>>>(x, M.d_a[0], n * kFeat);
-    forward(M, pad, s);
-    LSG_HIP(hipMemsetAsync(M.d_loss, 0, 4, s));
-    LSG_HIP(hipMemsetAsync(M.d_g, 0, 4 * M.nparams, s));
-    // output gradient dY (layer 4: 16 columns)
-    k_loss_grad<<<nb(pad), 256, 0, s>>>(M.d_z[kLayers - 1], t, pad, n, lambda, M.d_dz, M.d_dzb, M.d_loss);
-    for (int l = kLayers - 1; l >= 0; l--) {
-        const int in = kIn[l], out = kOut[l];
-        // dW[in x out] = A^T[in x n] dZ[n x out]:  A(m=i,k=r) = a[r*in + i], B(k=r,n=c) = dzb[r*out + c]
-        gemm(M.d_a[l], 1, in, M.d_dzb, out, 1, M.d_g + M.wofs[l], out, in, out, (int)pad, 0, s);
-        k_colsum<<<out, 256, 0, s>>>(M.d_dz, pad, out, M.d_g + M.bofs[l]);
-        if (l == 0) break;
-        // dA[n x in] = dZ[n x out] W^T[out x in]:  A(m=r,k=c) = dzb[r*out + c], B(k=c,n=i) = W[i*out + c]
-        gemm(M.d_dzb, out, 1, M.d_wb + M.wofs[l], 1, out, M.d_da, in, (int)pad, in, out, 0, s);
-        k_relu_back<<<nb((uint64_t)pad * in), 256, 0, s>>>(M.d_da, M.d_z[l - 1], M.d_dzb, M.d_dz, pad * in);
-    }
+    MlpOffsets off;
+    for (int l = 0; l < kLayers; l++) { off.w[l] = (uint32_t)M.wofs[l]; off.b[l] = (uint32_t)M.bofs[l]; }
+    const uint32_t parts = (uint32_t)std::min<uint64_t>(((uint64_t)n + kRows - 1) / kRows, kTrainBlocks);
+    float* loss_part = M.d_part + (size_t)kTrainBlocks * M.nparams;
+    k_mlp_train<<<parts, 256, 0, s>>>(x, t, n, lambda, M.d_wb, M.d_p, off, (uint32_t)M.nparams, M.d_part, loss_part);
+    AdamArgs A{M.d_p, M.d_m, M.d_v, M.d_wb, M.d_mask, lr, 0.9f, 0.999f, 1e-8f, 1.f, 1.f};
     if (lr > 0) {
         M.step++;
-        const float b1 = 0.9f, b2 = 0.999f;
-        const float c1 = 1.f - powf(b1, (float)M.step), c2 = 1.f - powf(b2, (float)M.step);
-        k_adam<<<nb(M.nparams), 256, 0, s>>>(M.d_p, M.d_g, M.d_m, M.d_v, M.d_mask, (uint32_t)M.nparams, lr, b1, b2, 1e-8f, c1, c2);
-        k_to_bf16<<<nb(M.nparams), 256, 0, s>>>(M.d_p, M.d_wb, (uint32_t)M.nparams);
+        A.c1 = 1.f - powf(A.b1, (float)M.step); A.c2 = 1.f - powf(A.b2, (float)M.step);
     }
+    k_mlp_update<<<(unsigned)((M.nparams + 63) / 64), 256, 0, s>>>(M.d_part, parts, (uint32_t)M.nparams, M.d_g, A, loss_part, M.d_loss);
     LSG_HIP(hipGetLastError());
     if (loss) {
         float l = 0;

@@ -66,6 +66,40 @@ def test_mlp_gradients_match_oracle(gpu, oracle):
             o += blk
 
 
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 130, 16385])
+def test_training_step_vs_oracle(gpu, oracle, n):
+    """One training step at the edges of its 64-row passes, and with more passes than
+    workgroups (16385): loss and gradients against the oracle, which rounds to BF16 at the same
+    points (a different order of the FP32 sums can flip a rounding, at most 2^-8 of a value in
+    each of five layers); the same bits when repeated; and the parameters after an Adam
+    step, p - lr g / (|g| + eps) on the first, to the rounding of a handful of FP32 operations."""
+    from lightsprintsdk_amd.learned import Surrogate
+    from lightsprintsdk_amd.collider import DeviceBuffer
+    rng = np.random.default_rng(n)
+    net = Surrogate(max_batch=(n + 15) // 16 * 16, seed=3)
+    p = net.init_params(3)
+    p[-16 * 65:] += (rng.normal(size=16 * 65) * 0.05).astype(np.float32)   # make the last layer non-trivial
+    net.set_params(p)
+    p = net.get_params()
+    x = rng.uniform(-1, 1, size=(n, 32)).astype(np.float32)
+    t = rng.normal(size=(n, 3)).astype(np.float32)
+    dx, dt = DeviceBuffer.from_array(x), DeviceBuffer.from_array(t)
+    print(f"train {n} rows", flush=True)
+    loss = net.step(dx, dt, n, lr=0.0, want_loss=True)
+    g = net.get_grads()
+    lo, _, go = oracle.mlp_loss_grad(p, x, t, lam=0.5, bf16=True)
+    assert abs(loss - lo) <= 5 * 2.0 ** -8 * abs(lo)
+    assert np.linalg.norm(g - go) <= 5 * 2.0 ** -8 * np.linalg.norm(go)
+    assert net.step(dx, dt, n, lr=0.0, want_loss=True) == loss
+    np.testing.assert_array_equal(net.get_grads().view(np.uint32), g.view(np.uint32))
+    np.testing.assert_array_equal(net.get_params(), p)
+    lr = 1e-2
+    net.step(dx, dt, n, lr=lr, want_loss=False)
+    g64 = g.astype(np.float64)
+    # 1 - b2 = 1e-3 in FP32 is off by 6e-5 of itself, in v and in its correction
+    np.testing.assert_allclose(net.get_params(), p - lr * g64 / (np.abs(g64) + 1e-8), rtol=0, atol=2e-4 * lr + 2.0 ** -23)
+
+
 def test_mlp_training_converges(gpu):
     from lightsprintsdk_amd.learned import Surrogate
     rng = np.random.default_rng(9)
