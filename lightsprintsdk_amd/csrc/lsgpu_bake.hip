@@ -1,8 +1,8 @@
 // lsgpu_bake.hip -- whole-scene lightmap bake plan: RRSolver::updateLightmaps
 // (RRSolver/lightmap.cpp:943-1163) for many objects in one go on gfx950.
 //
-// A plan owns, in HBM, every object's texels and SubTexels (rasterised once on the
-// host), one RGBA temp texel array for all lightmaps, the RGBF output, the filter
+// A plan owns, in HBM, every object's texels and SubTexels (rasterised once,
+// all objects together), one RGBA temp texel array for all lightmaps, the RGBF output, the filter
 // scratch and the per-triangle first-gather work.  One run is
 //   first gather per triangle (gatherPerTrianglePhysical, gather.cpp:843-952)
 //   -> exitance = irradiance * albedo + emittance          (k_exitance)
@@ -39,6 +39,15 @@ __global__ __launch_bounds__(256) void k_exitance(uint32_t nt, const float4* __r
                                       e.y * albedo[3 * (size_t)t + 1] + emit[3 * (size_t)t + 1],
                                       e.z * albedo[3 * (size_t)t + 2] + emit[3 * (size_t)t + 2], 0.f);
     ex[2 * (size_t)t + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// the first gather's work: one texel per triangle, covering the whole triangle
+__global__ __launch_bounds__(256) void k_triangle_texels(uint32_t nt, lsg_texel* __restrict__ tex, lsg_subtexel* __restrict__ sub)
+{
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= nt) return;
+    tex[t] = lsg_texel{t, t, 1u | (255u << 16), 0x80000000u | t};
+    sub[t] = lsg_subtexel{t, {0.f, 0.f, 1.f, 0.f, 0.f, 1.f}, 1.f};
 }
 
 // exitance = emittance only, the light the first gather's hemisphere rays may see: the
@@ -226,54 +235,51 @@ int lsg_bake_create(lsg_scene* scene, const lsg_bake_object* objects, uint32_t n
     B.ntri = scene->impl.col->impl.ntri;
     auto bail = [&](int st) { delete b; return st; };
     // 1. rasterise every object (lightmap.cpp:83-335) into one texel/SubTexel list
-    std::vector<lsg_texel> tex;
-    std::vector<lsg_subtexel> sub;
+    std::vector<RasterObject> ro(nobjects);
+    std::vector<const float*> uv(nobjects);
+    std::vector<const uint32_t*> ids(nobjects);
     uint32_t slot = 0;
+    uint64_t tris = 0;
     for (uint32_t o = 0; o < nobjects; o++) {
         const lsg_bake_object& ob = objects[o];
-        uint32_t nt = 0, ns = 0;
-        int st = lsg_rasterize_texels(ob.tri_uv, ob.tri_ids, ob.ntri, ob.width, ob.height, o, nullptr, &nt, nullptr, &ns, slot);
-        if (st) return bail(st);
-        size_t t0 = tex.size(), s0 = sub.size();
-        tex.resize(t0 + nt); sub.resize(s0 + ns);
-        st = lsg_rasterize_texels(ob.tri_uv, ob.tri_ids, ob.ntri, ob.width, ob.height, o, tex.data() + t0, &nt, sub.data() + s0, &ns, slot);
-        if (st) return bail(st);
-        for (size_t k = t0; k < tex.size(); k++) tex[k].sub_begin += (uint32_t)s0;
-        lsg_lightmap m{slot, ob.width, ob.height, slot};
-        B.maps.push_back(m);
-        uint64_t ns64 = (uint64_t)slot + (uint64_t)ob.width * ob.height;
+        if (ob.ntri && (!ob.tri_uv || !ob.tri_ids)) return bail(fail(LSG_ERR_INVALID, "lsg_bake_create: object %u has null arrays", o));
+        if (!ob.width || !ob.height || (uint64_t)ob.width * ob.height > (1ull << 28))
+            return bail(fail(LSG_ERR_INVALID, "lsg_bake_create: bad map size %ux%u", ob.width, ob.height));
+        ro[o] = RasterObject{(uint32_t)tris, ob.ntri, ob.width, ob.height, slot, o};
+        uv[o] = ob.tri_uv; ids[o] = ob.tri_ids;
+        B.maps.push_back(lsg_lightmap{slot, ob.width, ob.height, slot});
+        const uint64_t ns64 = (uint64_t)slot + (uint64_t)ob.width * ob.height;
         if (ns64 >= (1ull << 31)) return bail(fail(LSG_ERR_LIMIT, "lsg_bake_create: more than 2^31 lightmap texels"));
+        tris += ob.ntri;
+        if (tris >= (1ull << 32)) return bail(fail(LSG_ERR_LIMIT, "lsg_bake_create: more than 2^32 triangles"));
         slot = (uint32_t)ns64;
     }
-    B.ntex = (uint32_t)tex.size(); B.nsub = (uint32_t)sub.size(); B.nmaps = nobjects; B.nslots = slot;
+    RasterOut list;
+    int st = raster_objects(ro.data(), nobjects, uv.data(), ids.data(), false, list, nullptr);
+    if (st) return bail(st);
+    B.ntex = list.ntex; B.nsub = list.nsub; B.nmaps = nobjects; B.nslots = slot;
+    B.d_tex = list.tex; B.d_sub = list.sub;
+    list.tex = nullptr; list.sub = nullptr;
     hipError_t e;
 #define AL(p, n) do { if ((e = hipMalloc(&(p), (n) ? (n) : 16)) != hipSuccess) return bail(hip_fail(e, "hipMalloc", __LINE__)); } while (0)
 #define UP(d, h, n) do { if ((n) && (e = hipMemcpy((d), (h), (n), hipMemcpyHostToDevice)) != hipSuccess) return bail(hip_fail(e, "h2d", __LINE__)); } while (0)
-    AL(B.d_tex, sizeof(lsg_texel) * tex.size()); UP(B.d_tex, tex.data(), sizeof(lsg_texel) * tex.size());
-    AL(B.d_sub, sizeof(lsg_subtexel) * sub.size()); UP(B.d_sub, sub.data(), sizeof(lsg_subtexel) * sub.size());
+    if (!B.d_tex) AL(B.d_tex, 0);
+    if (!B.d_sub) AL(B.d_sub, 0);
     AL(B.d_rgba, 16 * (size_t)slot);
     AL(B.d_rgbf, 12 * (size_t)slot);
     AL(B.d_queue, 64);
-    AL(B.d_walk, 32 * tex.size());
+    AL(B.d_walk, 32 * (size_t)B.ntex);
     // 2. first-gather work: one texel per triangle covering the whole triangle
-    std::vector<lsg_texel> ttex(B.ntri);
-    std::vector<lsg_subtexel> tsub(B.ntri);
-    for (uint32_t t = 0; t < B.ntri; t++) {
-        ttex[t] = lsg_texel{t, t, 1u | (255u << 16), 0x80000000u | t};
-        tsub[t].triangle = t;
-        const float uv[6] = {0, 0, 1, 0, 0, 1};
-        memcpy(tsub[t].uv, uv, sizeof uv);
-        tsub[t].area = 1.f;
-    }
-    AL(B.d_ttex, sizeof(lsg_texel) * B.ntri); UP(B.d_ttex, ttex.data(), sizeof(lsg_texel) * B.ntri);
-    AL(B.d_tsub, sizeof(lsg_subtexel) * B.ntri); UP(B.d_tsub, tsub.data(), sizeof(lsg_subtexel) * B.ntri);
+    AL(B.d_ttex, sizeof(lsg_texel) * B.ntri);
+    AL(B.d_tsub, sizeof(lsg_subtexel) * B.ntri);
+    if (B.ntri) k_triangle_texels<<<nblk(B.ntri), 256>>>(B.ntri, B.d_ttex, B.d_tsub);
     AL(B.d_irr, 16 * (size_t)B.ntri);
     AL(B.d_albedo, 12 * (size_t)B.ntri); UP(B.d_albedo, albedo, 12 * (size_t)B.ntri);
     AL(B.d_emit, 12 * (size_t)B.ntri); UP(B.d_emit, emittance, 12 * (size_t)B.ntri);
 #undef AL
 #undef UP
     uint32_t tiles = 0;
-    int st = maps_upload(B.maps.data(), B.nmaps, &B.d_maps, &B.ftotal, &tiles);
+    st = maps_upload(B.maps.data(), B.nmaps, &B.d_maps, &B.ftotal, &tiles);
     if (st) return bail(st);
     if ((st = scratch_alloc(B.S, B.ftotal, tiles))) return bail(st);
     int dev = 0;
@@ -281,6 +287,7 @@ int lsg_bake_create(lsg_scene* scene, const lsg_bake_object* objects, uint32_t n
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) B.cus = prop.multiProcessorCount;
     default_tuning(B.tuning);
+    if ((e = hipStreamSynchronize(nullptr)) != hipSuccess) return bail(hip_fail(e, "sync", __LINE__));
     *out = b;
     return LSG_OK;
 }

@@ -209,6 +209,24 @@ int pack4_device(ColliderImpl& C, const Node4* nodes4);
 int sah_rebuild(const float* nodes, uint32_t nnodes, int32_t root, float* out, uint32_t* out_nodes, int32_t* out_root,
                 uint32_t* out_depth);
 
+// ---- texel rasterisation (lsgpu_raster.hip) ---------------------------------------------
+struct RasterObject {
+    uint32_t tri_begin, ntri;      // its triangles among all objects' (in object order)
+    uint32_t width, height;
+    uint32_t slot;                 // out_index of its texel (0, 0); objects' texels follow one another
+    uint32_t id;
+};
+struct RasterOut {                 // device lists, texels of object after object
+    lsg_texel* tex = nullptr;
+    lsg_subtexel* sub = nullptr;
+    uint32_t ntex = 0, nsub = 0;
+    uint32_t cap_t = 0xffffffffu, cap_s = 0xffffffffu;     // with more than this, only the counts
+    ~RasterOut() { if (tex) (void)hipFree(tex); if (sub) (void)hipFree(sub); }
+};
+// uv[o], ids[o]: host arrays of object o (6 floats and an index per triangle).  Synchronous on st.
+int raster_objects(const RasterObject* objs, uint32_t nobj, const float* const* uv, const uint32_t* const* ids, bool counts_only,
+                   RasterOut& out, hipStream_t st);
+
 } // namespace lsg
 
 struct lsg_collider { lsg::ColliderImpl impl; };

@@ -1,7 +1,7 @@
-// lsgpu_raster.hip -- texel rasterisation of one lightmap on the GPU (gfx950).
+// lsgpu_raster.hip -- texel rasterisation of lightmaps on the GPU (gfx950).
 //
 // Produces what enumerateTexelsPartial (RRSolver/lightmap.cpp:83-404, steps 1-2) gives the
-// final gather for one object: every texel the object's unwrap covers, the pieces
+// final gather for an object: every texel the object's unwrap covers, the pieces
 // (SubTexels, gather.h:60-65) of each triangle inside it, and the texel's coverage flags
 // (gather.h:68-80) -- by a design of this library:
 //   1. each triangle's candidate texels are the cells of its bounding box in texel units;
@@ -12,12 +12,20 @@
 //      by texel index, so a texel's pieces come in triangle order and texels row-major;
 //   4. runs of one texel become texel records; every pair writes its pieces (corner
 //      coordinates in triangle space, area) at its scanned offset.
+// All objects of a bake go through these steps together: their texels' numbers do not overlap
+// and grow with the object, so one sort gives every object's list in turn.  The steps are
+// short (2 to 30 us a kernel for 20 maps of 256^2) and what an object costs is launches, waits and
+// allocations; one object at a time, counted first and then rasterised again, a bake of 20
+// objects with 50,000 triangles took 64 ms to set up, together 3.0.
 // Kept from the reference because they are its interface: the flag bits, the 0.03-texel
 // edge tolerance of the edge flags (lightmap.cpp:292), the quadrant rule for an edge that
 // crosses both texel axes (lightmap.cpp:302-311), and areaInMapSpace = half the piece's
 // area in uv units (the reference's triangle-space area times the triangle's map area).
 #include "lsgpu_internal.h"
+#include <algorithm>
 #include <cmath>
+#include <cstring>
+#include <utility>
 #include <vector>
 
 namespace lsg {
@@ -27,13 +35,17 @@ namespace {
 enum : uint32_t { QX0Y0 = 1, QX1Y0 = 2, QX0Y1 = 4, QX1Y1 = 8, EX0 = 16, EX1 = 32, EY0 = 64, EY1 = 128 };
 
 // a triangle's uv corners, its candidate box of texels and its index in the mesh
-struct TriBox { float2 u0, u1, u2; uint32_t x0, y0, w, id; };
+struct TriBox { float2 u0, u1, u2; uint32_t x0, y0, w, id, obj; };
 
 __global__ __launch_bounds__(256) void k_raster_boxes(const float* __restrict__ uv, const uint32_t* __restrict__ ids, uint32_t ntri,
-                                                      uint32_t W, uint32_t H, TriBox* __restrict__ tb, uint32_t* __restrict__ cnt)
+                                                      const RasterObject* __restrict__ objs, uint32_t nobj,
+                                                      TriBox* __restrict__ tb, uint32_t* __restrict__ cnt)
 {
     const uint32_t t = blockIdx.x * 256 + threadIdx.x;
     if (t >= ntri) return;
+    uint32_t lo = 0, hi = nobj;
+    while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (objs[mid].tri_begin <= t) lo = mid; else hi = mid; }
+    const uint32_t W = objs[lo].width, H = objs[lo].height;
     const float* u = uv + 6 * (size_t)t;
     const float fw = (float)W, fh = (float)H;
     const float2 p0 = make_float2(u[0] * fw, u[1] * fh), p1 = make_float2(u[2] * fw, u[3] * fh), p2 = make_float2(u[4] * fw, u[5] * fh);
@@ -42,6 +54,7 @@ __global__ __launch_bounds__(256) void k_raster_boxes(const float* __restrict__ 
     TriBox b;
     b.u0 = make_float2(u[0], u[1]); b.u1 = make_float2(u[2], u[3]); b.u2 = make_float2(u[4], u[5]);
     b.id = ids[t];
+    b.obj = lo;
     b.x0 = b.y0 = b.w = 0;
     uint32_t n = 0;
     const float lx = fminf(p0.x, fminf(p1.x, p2.x)), hx = fmaxf(p0.x, fmaxf(p1.x, p2.x));
@@ -149,29 +162,32 @@ __device__ inline int clip_candidate(const TriBox& b, uint32_t x, uint32_t y, fl
 
 // per candidate: (pieces << 8 | flags), and 1 where the pair is not empty
 __global__ __launch_bounds__(256) void k_raster_count(const uint32_t* __restrict__ off, uint32_t ntri, const TriBox* __restrict__ tb,
-                                                      uint32_t C, float fw, float fh, uint16_t* __restrict__ info,
+                                                      uint32_t C, const RasterObject* __restrict__ objs, uint16_t* __restrict__ info,
                                                       uint32_t* __restrict__ nz)
 {
     const uint32_t c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
     uint32_t x, y;
     const uint32_t t = candidate(off, ntri, tb, c, x, y);
+    const RasterObject& o = objs[tb[t].obj];
     float2 poly[8], q0;
-    const int n = clip_candidate(tb[t], x, y, fw, fh, poly, q0);
+    const int n = clip_candidate(tb[t], x, y, (float)o.width, (float)o.height, poly, q0);
     info[c] = n ? (uint16_t)(((uint32_t)(n - 2) << 8) | coverage_flags(poly, n)) : (uint16_t)0;
     nz[c] = n ? 1u : 0u;
 }
 
+// keys: the texel's number from slot0 on
 __global__ __launch_bounds__(256) void k_raster_compact(const uint32_t* __restrict__ off, uint32_t ntri, const TriBox* __restrict__ tb,
-                                                        uint32_t C, uint32_t W, const uint32_t* __restrict__ nz,
-                                                        const uint32_t* __restrict__ pos, uint32_t* __restrict__ keys,
-                                                        uint32_t* __restrict__ vals)
+                                                        uint32_t C, const RasterObject* __restrict__ objs, uint32_t slot0,
+                                                        const uint32_t* __restrict__ nz, const uint32_t* __restrict__ pos,
+                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ vals)
 {
     const uint32_t c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C || !nz[c]) return;
     uint32_t x, y;
-    candidate(off, ntri, tb, c, x, y);
-    keys[pos[c]] = x + y * W;
+    const uint32_t t = candidate(off, ntri, tb, c, x, y);
+    const RasterObject& o = objs[tb[t].obj];
+    keys[pos[c]] = o.slot - slot0 + x + y * o.width;
     vals[pos[c]] = c;
 }
 
@@ -189,8 +205,8 @@ __global__ __launch_bounds__(256) void k_raster_runs(const uint32_t* __restrict_
 __global__ __launch_bounds__(256) void k_raster_texels(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals, uint32_t np,
                                                        const uint16_t* __restrict__ info, const uint32_t* __restrict__ head,
                                                        const uint32_t* __restrict__ ord, const uint32_t* __restrict__ soff,
-                                                       uint32_t object_id, uint32_t out_base, lsg_texel* __restrict__ texels,
-                                                       uint32_t* __restrict__ too_many)
+                                                       const RasterObject* __restrict__ objs, uint32_t nobj, uint32_t slot0,
+                                                       uint32_t sub_base, lsg_texel* __restrict__ texels, uint32_t* __restrict__ too_many)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= np || !head[i]) return;
@@ -203,22 +219,27 @@ __global__ __launch_bounds__(256) void k_raster_texels(const uint32_t* __restric
     }
     if (count > 0xffffu) { atomicMax(too_many, count); count = 0xffffu; }
     lsg_texel T;
-    T.out_index = out_base + key;
-    T.sub_begin = soff[i];
+    T.out_index = slot0 + key;
+    T.sub_begin = sub_base + soff[i];
     T.sub_count_flags = count | (flags << 16);
-    T.key = object_id * 0x9E3779B1u + key;      // stable per-texel seed id
+    uint32_t lo = 0, hi = nobj;
+    while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (objs[mid].slot - slot0 <= key) lo = mid; else hi = mid; }
+    T.key = objs[lo].id * 0x9E3779B1u + (key - (objs[lo].slot - slot0));      // stable per-texel seed id
     texels[ord[i]] = T;
 }
 
 __global__ __launch_bounds__(256) void k_raster_emit(const uint32_t* __restrict__ off, uint32_t ntri, const TriBox* __restrict__ tb,
                                                      const uint32_t* __restrict__ vals, uint32_t np, const uint32_t* __restrict__ soff,
-                                                     float fw, float fh, float area_scale, lsg_subtexel* __restrict__ subs)
+                                                     const RasterObject* __restrict__ objs, lsg_subtexel* __restrict__ subs)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= np) return;
     uint32_t x, y;
     const uint32_t t = candidate(off, ntri, tb, vals[i], x, y);
     const TriBox b = tb[t];
+    const RasterObject& ob = objs[b.obj];
+    const float fw = (float)ob.width, fh = (float)ob.height;
+    const float area_scale = (float)(0.25 / ((double)ob.width * (double)ob.height));
     float2 poly[8], q0;
     const int n = clip_candidate(b, x, y, fw, fh, poly, q0);
     // triangle-space coordinates: p - corner 0 = a e1 + b e2, with the edges from the
@@ -246,64 +267,58 @@ __global__ __launch_bounds__(256) void k_raster_emit(const uint32_t* __restrict_
 
 inline unsigned blocks(uint64_t n) { return (unsigned)((n + 255) / 256); }
 
-struct DevArena {
-    std::vector<void*> ptrs;
-    ~DevArena() { for (void* p : ptrs) (void)hipFree(p); }
-    template <class T> int get(T** p, size_t n)
+// one allocation for a step's arrays: parts are added, then placed
+struct Scratch {
+    std::vector<std::pair<void**, size_t>> parts;
+    void* base = nullptr;
+    ~Scratch() { if (base) (void)hipFree(base); }
+    template <class T> void add(T** p, size_t n) { parts.push_back({(void**)p, sizeof(T) * n}); }
+    int place()
     {
-        void* q = nullptr;
-        hipError_t e = hipMalloc(&q, sizeof(T) * (n ? n : 1));
-        if (e != hipSuccess) return hip_fail(e, "hipMalloc", __LINE__);
-        ptrs.push_back(q);
-        *p = (T*)q;
+        size_t n = 0;
+        for (auto& q : parts) n += (q.second + 255) / 256 * 256;
+        hipError_t e = hipMalloc(&base, n ? n : 256);
+        if (e != hipSuccess) { base = nullptr; return hip_fail(e, "hipMalloc", __LINE__); }
+        char* c = (char*)base;
+        for (auto& q : parts) { *q.first = c; c += (q.second + 255) / 256 * 256; }
         return LSG_OK;
     }
 };
 
-} // namespace
+constexpr uint64_t kGroupCandidates = 1ull << 26;        // candidates rasterised together, unless one object has more
 
-// One object's texels and pieces on the device.  counts_only: stop once the counts are
-// known (texels/subs untouched).  Otherwise texels/subs are device arrays of at least the
-// counts a counting call returned.  Synchronous on st.
-int raster_object(const float* d_uv, const uint32_t* d_ids, uint32_t ntri, uint32_t W, uint32_t H, uint32_t object_id,
-                  uint32_t out_base, bool counts_only, lsg_texel* texels, uint32_t cap_t, lsg_subtexel* subs, uint32_t cap_s,
-                  uint32_t* ntex, uint32_t* nsub, hipStream_t st)
+// The texels and pieces of objects [o0, o1), whose triangles are [t0, t1) and have C
+// candidates.  The counts are added to out; then, unless counts_only or out's caps are too
+// small, the lists are appended to what out holds.
+int raster_group(const RasterObject* objs, const RasterObject* d_objs, uint32_t o0, uint32_t o1, uint32_t t0, uint32_t t1, const TriBox* tb,
+                 const uint32_t* cnt, uint32_t C, bool counts_only, RasterOut& out, hipStream_t st)
 {
-    *ntex = 0; *nsub = 0;
-    if (!ntri) return LSG_OK;
-    DevArena A;
-    int e;
-    TriBox* tb; uint32_t *cnt, *off, *stmp, *tot;
-    if ((e = A.get(&tb, ntri)) || (e = A.get(&cnt, ntri)) || (e = A.get(&off, (size_t)ntri + 1)) || (e = A.get(&tot, 4)))
-        return e;
-    if ((e = A.get(&stmp, scan_tmp_words(ntri)))) return e;
-    k_raster_boxes<<<blocks(ntri), 256, 0, st>>>(d_uv, d_ids, ntri, W, H, tb, cnt);
-    if ((e = scan_exclusive_u32(cnt, off, ntri, tot, stmp, st))) return e;
-    // candidates: 64-bit sum check on the host (each box is at most W*H <= 2^28 cells)
-    std::vector<uint32_t> hc(ntri);
-    LSG_HIP(hipMemcpyAsync(hc.data(), cnt, 4 * (size_t)ntri, hipMemcpyDeviceToHost, st));
-    LSG_HIP(hipStreamSynchronize(st));
-    uint64_t C64 = 0;
-    for (uint32_t t = 0; t < ntri; t++) C64 += hc[t];
-    if (C64 >= (1ull << 31)) return fail(LSG_ERR_LIMIT, "lsg_rasterize_texels: %llu candidate texels", (unsigned long long)C64);
-    const uint32_t C = (uint32_t)C64;
     if (!C) return LSG_OK;
-    uint16_t* info; uint32_t *nz, *pos, *ctmp;
-    if ((e = A.get(&info, C)) || (e = A.get(&nz, C)) || (e = A.get(&pos, C)) || (e = A.get(&ctmp, scan_tmp_words(C)))) return e;
-    k_raster_count<<<blocks(C), 256, 0, st>>>(off, ntri, tb, C, (float)W, (float)H, info, nz);
-    if ((e = scan_exclusive_u32(nz, pos, C, tot, ctmp, st))) return e;
+    const uint32_t ntri = t1 - t0, slot0 = objs[o0].slot;
+    int e;
+    tb += t0;
+    Scratch A;
+    uint32_t *off, *tot, *nz, *pos, *tmp;
+    uint16_t* info;
+    A.add(&off, (size_t)ntri + 1); A.add(&tot, 4); A.add(&info, C); A.add(&nz, C); A.add(&pos, C);
+    A.add(&tmp, std::max(scan_tmp_words(ntri), scan_tmp_words(C)));
+    if ((e = A.place())) return e;
+    if ((e = scan_exclusive_u32(cnt + t0, off, ntri, tot, tmp, st))) return e;
+    k_raster_count<<<blocks(C), 256, 0, st>>>(off, ntri, tb, C, d_objs, info, nz);
+    if ((e = scan_exclusive_u32(nz, pos, C, tot, tmp, st))) return e;
     uint32_t np = 0;
     LSG_HIP(hipMemcpyAsync(&np, tot, 4, hipMemcpyDeviceToHost, st));
     LSG_HIP(hipStreamSynchronize(st));
     if (!np) return LSG_OK;
+    Scratch P;
     uint32_t *keys, *vals, *k2, *v2, *sorttmp, *pieces, *head, *soff, *ord, *ptmp;
-    if ((e = A.get(&keys, np)) || (e = A.get(&vals, np)) || (e = A.get(&k2, np)) || (e = A.get(&v2, np)) ||
-        (e = A.get(&sorttmp, sort_tmp_words(np))) || (e = A.get(&pieces, np)) || (e = A.get(&head, np)) ||
-        (e = A.get(&soff, np)) || (e = A.get(&ord, np)) || (e = A.get(&ptmp, scan_tmp_words(np))))
-        return e;
-    k_raster_compact<<<blocks(C), 256, 0, st>>>(off, ntri, tb, C, W, nz, pos, keys, vals);
+    P.add(&keys, np); P.add(&vals, np); P.add(&k2, np); P.add(&v2, np); P.add(&sorttmp, sort_tmp_words(np)); P.add(&pieces, np);
+    P.add(&head, np); P.add(&soff, np); P.add(&ord, np); P.add(&ptmp, scan_tmp_words(np));
+    if ((e = P.place())) return e;
+    k_raster_compact<<<blocks(C), 256, 0, st>>>(off, ntri, tb, C, d_objs, slot0, nz, pos, keys, vals);
+    const uint64_t span = (uint64_t)objs[o1 - 1].slot - slot0 + (uint64_t)objs[o1 - 1].width * objs[o1 - 1].height;
     int bits = 1;
-    while (bits < 32 && ((uint64_t)1 << bits) < (uint64_t)W * H) bits++;
+    while (bits < 32 && ((uint64_t)1 << bits) < span) bits++;
     if ((e = sort_pairs_u32(keys, vals, k2, v2, np, bits, sorttmp, st))) return e;
     k_raster_runs<<<blocks(np), 256, 0, st>>>(keys, vals, np, info, pieces, head);
     if ((e = scan_exclusive_u32(pieces, soff, np, tot, ptmp, st))) return e;
@@ -311,18 +326,76 @@ int raster_object(const float* d_uv, const uint32_t* d_ids, uint32_t ntri, uint3
     uint32_t h[2] = {0, 0};
     LSG_HIP(hipMemcpyAsync(h, tot, 8, hipMemcpyDeviceToHost, st));
     LSG_HIP(hipStreamSynchronize(st));
-    *nsub = h[0]; *ntex = h[1];
-    if (counts_only) return LSG_OK;
-    if (!texels || !subs || cap_t < h[1] || cap_s < h[0])
-        return fail(LSG_ERR_LIMIT, "lsg_rasterize_texels: need %u texels / %u subtexels", h[1], h[0]);
+    const uint32_t nt0 = out.ntex, ns0 = out.nsub;
+    out.ntex += h[1]; out.nsub += h[0];
+    if (counts_only || out.ntex > out.cap_t || out.nsub > out.cap_s) return LSG_OK;
+    // room for the lists (grown by a copy when an earlier group has some)
+    lsg_texel* T = nullptr;
+    lsg_subtexel* S = nullptr;
+    LSG_HIP(hipMalloc(&T, sizeof(lsg_texel) * (size_t)out.ntex));
+    hipError_t he = hipMalloc(&S, sizeof(lsg_subtexel) * (size_t)out.nsub);
+    if (he != hipSuccess) { (void)hipFree(T); return hip_fail(he, "hipMalloc", __LINE__); }
+    std::swap(T, out.tex); std::swap(S, out.sub);
+    if (nt0) he = hipMemcpyAsync(out.tex, T, sizeof(lsg_texel) * (size_t)nt0, hipMemcpyDeviceToDevice, st);
+    if (he == hipSuccess && ns0) he = hipMemcpyAsync(out.sub, S, sizeof(lsg_subtexel) * (size_t)ns0, hipMemcpyDeviceToDevice, st);
+    if (he == hipSuccess && (T || S)) he = hipStreamSynchronize(st);
+    if (T) (void)hipFree(T);
+    if (S) (void)hipFree(S);
+    LSG_HIP(he);
     LSG_HIP(hipMemsetAsync(tot + 2, 0, 4, st));
-    k_raster_texels<<<blocks(np), 256, 0, st>>>(keys, vals, np, info, head, ord, soff, object_id, out_base, texels, tot + 2);
-    const float area_scale = (float)(0.25 / ((double)W * (double)H));
-    k_raster_emit<<<blocks(np), 256, 0, st>>>(off, ntri, tb, vals, np, soff, (float)W, (float)H, area_scale, subs);
+    k_raster_texels<<<blocks(np), 256, 0, st>>>(keys, vals, np, info, head, ord, soff, d_objs + o0, o1 - o0, slot0, ns0, out.tex + nt0, tot + 2);
+    k_raster_emit<<<blocks(np), 256, 0, st>>>(off, ntri, tb, vals, np, soff, d_objs, out.sub + ns0);
+    LSG_HIP(hipGetLastError());
     uint32_t worst = 0;
     LSG_HIP(hipMemcpyAsync(&worst, tot + 2, 4, hipMemcpyDeviceToHost, st));
     LSG_HIP(hipStreamSynchronize(st));
     if (worst) return fail(LSG_ERR_LIMIT, "lsg_rasterize_texels: a texel has %u subtexels (at most 65535)", worst);
+    return LSG_OK;
+}
+
+} // namespace
+
+int raster_objects(const RasterObject* objs, uint32_t nobj, const float* const* uv, const uint32_t* const* ids, bool counts_only,
+                   RasterOut& out, hipStream_t st)
+{
+    const uint64_t ntri64 = nobj ? (uint64_t)objs[nobj - 1].tri_begin + objs[nobj - 1].ntri : 0;
+    if (!ntri64) return LSG_OK;
+    const uint32_t ntri = (uint32_t)ntri64;
+    int e;
+    Scratch A;
+    float* d_uv;
+    uint32_t *d_ids, *cnt;
+    TriBox* tb;
+    RasterObject* d_objs;
+    A.add(&d_uv, 6 * (size_t)ntri); A.add(&d_ids, ntri); A.add(&tb, ntri); A.add(&cnt, ntri); A.add(&d_objs, nobj);
+    if ((e = A.place())) return e;
+    std::vector<uint32_t> hc(7 * (size_t)ntri);          // uv and ids of all objects, later the candidate counts
+    for (uint32_t o = 0; o < nobj; o++)
+        if (objs[o].ntri) {
+            memcpy(hc.data() + 6 * (size_t)objs[o].tri_begin, uv[o], 24 * (size_t)objs[o].ntri);
+            memcpy(hc.data() + 6 * (size_t)ntri + objs[o].tri_begin, ids[o], 4 * (size_t)objs[o].ntri);
+        }
+    LSG_HIP(hipMemcpyAsync(d_uv, hc.data(), 24 * (size_t)ntri, hipMemcpyHostToDevice, st));
+    LSG_HIP(hipMemcpyAsync(d_ids, hc.data() + 6 * (size_t)ntri, 4 * (size_t)ntri, hipMemcpyHostToDevice, st));
+    LSG_HIP(hipMemcpyAsync(d_objs, objs, sizeof(RasterObject) * nobj, hipMemcpyHostToDevice, st));
+    k_raster_boxes<<<blocks(ntri), 256, 0, st>>>(d_uv, d_ids, ntri, d_objs, nobj, tb, cnt);
+    LSG_HIP(hipStreamSynchronize(st));                   // hc is read
+    LSG_HIP(hipMemcpyAsync(hc.data(), cnt, 4 * (size_t)ntri, hipMemcpyDeviceToHost, st));
+    LSG_HIP(hipStreamSynchronize(st));
+    // 64-bit candidate sums (each box is at most W*H <= 2^28 cells), objects taken together up
+    // to kGroupCandidates
+    uint64_t sum = 0;
+    for (uint32_t o = 0, o0 = 0; o < nobj; o++) {
+        uint64_t c = 0;
+        for (uint32_t t = objs[o].tri_begin; t < objs[o].tri_begin + objs[o].ntri; t++) c += hc[t];
+        if (c >= (1ull << 31)) return fail(LSG_ERR_LIMIT, "lsg_rasterize_texels: %llu candidate texels", (unsigned long long)c);
+        if (sum && sum + c > kGroupCandidates) {
+            if ((e = raster_group(objs, d_objs, o0, o, objs[o0].tri_begin, objs[o].tri_begin, tb, cnt, (uint32_t)sum, counts_only, out, st))) return e;
+            o0 = o; sum = 0;
+        }
+        sum += c;
+        if (o + 1 == nobj) return raster_group(objs, d_objs, o0, nobj, objs[o0].tri_begin, ntri, tb, cnt, (uint32_t)sum, counts_only, out, st);
+    }
     return LSG_OK;
 }
 
@@ -338,37 +411,18 @@ extern "C" int lsg_rasterize_texels(const float* tri_uv, const uint32_t* tri_ids
     if (!width || !height || (uint64_t)width * height > (1ull << 28))
         return fail(LSG_ERR_INVALID, "lsg_rasterize_texels: bad map size %ux%u", width, height);
     if (!device_ready()) return fail(LSG_ERR_NO_DEVICE, "lsg_rasterize_texels: no gfx950 device");
-    const uint32_t cap_t = *ntexels, cap_s = *nsubs;
     const bool counts_only = !texels && !subs;
     if (!counts_only && (!texels || !subs)) return fail(LSG_ERR_INVALID, "lsg_rasterize_texels: give both output arrays");
-    hipStream_t st = nullptr;
-    float* d_uv = nullptr;
-    uint32_t* d_ids = nullptr;
-    lsg_texel* d_t = nullptr;
-    lsg_subtexel* d_s = nullptr;
-    auto done = [&](int r) {
-        if (d_uv) (void)hipFree(d_uv);
-        if (d_ids) (void)hipFree(d_ids);
-        if (d_t) (void)hipFree(d_t);
-        if (d_s) (void)hipFree(d_s);
-        return r;
-    };
-    hipError_t e;
-    if ((e = hipMalloc(&d_uv, 24 * (size_t)(ntri ? ntri : 1))) != hipSuccess) return done(hip_fail(e, "hipMalloc", __LINE__));
-    if ((e = hipMalloc(&d_ids, 4 * (size_t)(ntri ? ntri : 1))) != hipSuccess) return done(hip_fail(e, "hipMalloc", __LINE__));
-    if (ntri && (e = hipMemcpy(d_uv, tri_uv, 24 * (size_t)ntri, hipMemcpyHostToDevice)) != hipSuccess) return done(hip_fail(e, "h2d", __LINE__));
-    if (ntri && (e = hipMemcpy(d_ids, tri_ids, 4 * (size_t)ntri, hipMemcpyHostToDevice)) != hipSuccess) return done(hip_fail(e, "h2d", __LINE__));
-    uint32_t nt = 0, ns = 0;
-    int r = raster_object(d_uv, d_ids, ntri, width, height, object_id, out_base, true, nullptr, 0, nullptr, 0, &nt, &ns, st);
-    if (r) return done(r);
-    *ntexels = nt; *nsubs = ns;
-    if (counts_only) return done(LSG_OK);
-    if (cap_t < nt || cap_s < ns) return done(fail(LSG_ERR_LIMIT, "lsg_rasterize_texels: need %u texels / %u subtexels", nt, ns));
-    if ((e = hipMalloc(&d_t, sizeof(lsg_texel) * (size_t)(nt ? nt : 1))) != hipSuccess) return done(hip_fail(e, "hipMalloc", __LINE__));
-    if ((e = hipMalloc(&d_s, sizeof(lsg_subtexel) * (size_t)(ns ? ns : 1))) != hipSuccess) return done(hip_fail(e, "hipMalloc", __LINE__));
-    r = raster_object(d_uv, d_ids, ntri, width, height, object_id, out_base, false, d_t, nt, d_s, ns, &nt, &ns, st);
-    if (r) return done(r);
-    if (nt && (e = hipMemcpy(texels, d_t, sizeof(lsg_texel) * (size_t)nt, hipMemcpyDeviceToHost)) != hipSuccess) return done(hip_fail(e, "d2h", __LINE__));
-    if (ns && (e = hipMemcpy(subs, d_s, sizeof(lsg_subtexel) * (size_t)ns, hipMemcpyDeviceToHost)) != hipSuccess) return done(hip_fail(e, "d2h", __LINE__));
-    return done(LSG_OK);
+    RasterOut out;
+    out.cap_t = *ntexels; out.cap_s = *nsubs;
+    const RasterObject ob{0, ntri, width, height, out_base, object_id};
+    int r = raster_objects(&ob, 1, &tri_uv, &tri_ids, counts_only, out, nullptr);
+    if (r) return r;
+    *ntexels = out.ntex; *nsubs = out.nsub;
+    if (counts_only) return LSG_OK;
+    if (out.ntex > out.cap_t || out.nsub > out.cap_s)
+        return fail(LSG_ERR_LIMIT, "lsg_rasterize_texels: need %u texels / %u subtexels", out.ntex, out.nsub);
+    if (out.ntex) LSG_HIP(hipMemcpy(texels, out.tex, sizeof(lsg_texel) * (size_t)out.ntex, hipMemcpyDeviceToHost));
+    if (out.nsub) LSG_HIP(hipMemcpy(subs, out.sub, sizeof(lsg_subtexel) * (size_t)out.nsub, hipMemcpyDeviceToHost));
+    return LSG_OK;
 }

@@ -6,6 +6,8 @@ triangulate from different first vertices, so they are compared on what the gath
 filters read: the set of covered texels, each texel's flags, and for every (texel, triangle)
 the covered area and the polygon's corners; plus the orders (texels row-major, pieces in
 triangle order) and the closed forms the oracle is pinned by."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -198,3 +200,48 @@ def test_gpu_raster_deterministic_and_ids(gpu):
     assert np.all(a[0]["out_index"] >= 1000)
     assert np.all((a[0]["key"] - np.uint32(3 * 0x9E3779B1 & 0xFFFFFFFF)) == a[0]["out_index"] - 1000)
     assert set(np.unique(a[1]["triangle"])) <= set(ids)
+
+
+def test_gpu_plan_rasterises_objects_together(gpu):
+    """A bake plan's texel and piece lists (all objects rasterised together) are the lists of
+    its objects rasterised one at a time, one after another: odd map sizes, an object without
+    triangles, one whose triangles cover nothing, one with a single texel."""
+    from lightsprintsdk_amd import bake as B
+    from lightsprintsdk_amd import native as N
+    rng = np.random.default_rng(4)
+    sizes = [(33, 17), (8, 8), (1, 1), (64, 65), (5, 3)]
+    counts = [40, 0, 3, 120, 6]
+    nt = sum(counts)
+    verts = rng.uniform(-1, 1, (3 * nt, 3)).astype(np.float32)
+    idx = np.arange(3 * nt, dtype=np.uint32).reshape(-1, 3)
+    uv = rng.uniform(0, 1, (nt, 6)).astype(np.float32)
+    uv[nt - 6:] = 2.0                                     # the last object's cover nothing
+    ids = rng.permutation(nt).astype(np.uint32)
+    gs = B.GatherScene(verts, idx, np.zeros_like(verts), np.full(nt, 3, np.uint8), np.zeros((nt, 8), np.float32), [])
+    objs = (N.BakeObject * len(sizes))()
+    ref_t, ref_s, keep, t, slot = [], [], [], 0, 0
+    for k, ((w, h), c) in enumerate(zip(sizes, counts)):
+        u, i = np.ascontiguousarray(uv[t:t + c]), np.ascontiguousarray(ids[t:t + c])
+        keep += [u, i]
+        objs[k] = N.BakeObject(u.ctypes.data, i.ctypes.data, c, w, h)
+        tex, sub = B.rasterize(u, i, w, h, k, slot)
+        tex = tex.copy()
+        tex["sub_begin"] += sum(len(q) for q in ref_s)
+        ref_t.append(tex)
+        ref_s.append(sub)
+        t += c
+        slot += w * h
+    zero = np.zeros((nt, 3), np.float32)
+    h = ctypes.c_void_p()
+    N.check(N.lib().lsg_bake_create(gs._h, objs, len(sizes), zero.ctypes.data, zero.ctypes.data, ctypes.byref(h)), "lsg_bake_create")
+    try:
+        inf = N.BakeInfo()
+        N.check(N.lib().lsg_bake_info_get(h, ctypes.byref(inf)), "info")
+        rt, rs = np.concatenate(ref_t), np.concatenate(ref_s)
+        assert (inf.num_texels, inf.num_subtexels) == (len(rt), len(rs)) and len(rt)
+        gt, gs_ = np.empty_like(rt), np.empty_like(rs)
+        N.check(N.lib().lsg_memcpy_d2h(gt.ctypes.data, inf.texels, gt.nbytes), "d2h")
+        N.check(N.lib().lsg_memcpy_d2h(gs_.ctypes.data, inf.subtexels, gs_.nbytes), "d2h")
+        assert gt.tobytes() == rt.tobytes() and gs_.tobytes() == rs.tobytes()
+    finally:
+        N.lib().lsg_bake_destroy(h)
