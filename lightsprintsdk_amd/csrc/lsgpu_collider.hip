@@ -489,25 +489,21 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
     if (aborting && *aborting) return fail(LSG_ERR_ABORTED, "collider build aborted");
 
     // per-triangle precompute + keys
-    uint32_t *d_keys = nullptr, *d_vals = nullptr, *d_k2 = nullptr, *d_v2 = nullptr, *d_bytes = nullptr, *d_nvalid = nullptr;
-    float4 *d_plane_u = nullptr, *d_sv_u = nullptr, *d_ev_u = nullptr, *d_blo_u = nullptr, *d_bhi_u = nullptr;
-    uint32_t *d_hist = nullptr, *d_offs = nullptr, *d_stmp = nullptr;
-    int *d_first = nullptr, *d_last = nullptr, *d_split = nullptr, *d_pn = nullptr, *d_pl = nullptr;
-    float4 *d_plo = nullptr, *d_phi = nullptr, *d_nlo = nullptr, *d_nhi = nullptr;
-    uint32_t *d_arrive = nullptr, *d_depth = nullptr;
-    auto cleanup = [&]() {
-        dfree(d_keys); dfree(d_vals); dfree(d_k2); dfree(d_v2); dfree(d_bytes); dfree(d_nvalid);
-        dfree(d_plane_u); dfree(d_sv_u); dfree(d_ev_u); dfree(d_blo_u); dfree(d_bhi_u); dfree(d_hist); dfree(d_offs); dfree(d_stmp);
-        dfree(d_first); dfree(d_last); dfree(d_split); dfree(d_pn); dfree(d_pl);
-        dfree(d_plo); dfree(d_phi); dfree(d_nlo); dfree(d_nhi); dfree(d_arrive); dfree(d_depth);
-    };
-#define CK(x) do { if ((st = (x))) { cleanup(); return st; } } while (0)
-#define CKH(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { cleanup(); return hip_fail(e_, #x, __LINE__); } } while (0)
+    uint32_t *d_keys, *d_vals, *d_k2, *d_v2, *d_bytes, *d_nvalid, *d_hist, *d_offs, *d_stmp, *d_arrive, *d_depth;
+    float4 *d_plane_u, *d_sv_u, *d_ev_u, *d_blo_u, *d_bhi_u, *d_plo, *d_phi, *d_nlo, *d_nhi;
+    int *d_first, *d_last, *d_split, *d_pn, *d_pl;
+#define CK(x) do { if ((st = (x))) return st; } while (0)
+#define CKH(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) return hip_fail(e_, #x, __LINE__); } while (0)
     const size_t N = nt ? nt : 1;
-    CK(dalloc(&d_keys, N)); CK(dalloc(&d_vals, N)); CK(dalloc(&d_k2, N)); CK(dalloc(&d_v2, N));
-    CK(dalloc(&d_bytes, N)); CK(dalloc(&d_nvalid, 1));
-    CK(dalloc(&d_plane_u, N)); CK(dalloc(&d_sv_u, N)); CK(dalloc(&d_ev_u, N)); CK(dalloc(&d_blo_u, N)); CK(dalloc(&d_bhi_u, N));
-    CKH(hipMemset(d_nvalid, 0, 4));
+    const unsigned sort_blocks = blocks((uint32_t)N, RS_TILE);
+    Scratch A;                                       // everything the build needs, sized for nt valid triangles
+    A.add(&d_keys, N); A.add(&d_vals, N); A.add(&d_k2, N); A.add(&d_v2, N); A.add(&d_bytes, N); A.add(&d_nvalid, 1);
+    A.add(&d_plane_u, N); A.add(&d_sv_u, N); A.add(&d_ev_u, N); A.add(&d_blo_u, N); A.add(&d_bhi_u, N);
+    A.add(&d_hist, 256 * (size_t)sort_blocks); A.add(&d_offs, 256 * (size_t)sort_blocks); A.add(&d_stmp, scan_tmp_words(256 * sort_blocks));
+    A.add(&d_plo, N); A.add(&d_phi, N); A.add(&d_nlo, N); A.add(&d_nhi, N);
+    A.add(&d_first, N); A.add(&d_last, N); A.add(&d_split, N); A.add(&d_pn, N); A.add(&d_pl, N); A.add(&d_arrive, N); A.add(&d_depth, 1);
+    CK(A.place());
+    CKH(hipMemsetAsync(d_nvalid, 0, 4, nullptr));
     if (nt)
         k_tri_setup<<<blocks(nt), 256>>>(C.d_verts, C.d_idx, nt, make_float3(mn[0], mn[1], mn[2]),
                                          make_float3(scale[0], scale[1], scale[2]), d_keys, d_vals, d_plane_u, d_sv_u, d_ev_u,
@@ -516,14 +512,11 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
     uint32_t nvalid = 0;
     CKH(hipMemcpy(&nvalid, d_nvalid, 4, hipMemcpyDeviceToHost));
     C.nvalid = nvalid;
-    if (aborting && *aborting) { cleanup(); return fail(LSG_ERR_ABORTED, "collider build aborted"); }
+    if (aborting && *aborting) return fail(LSG_ERR_ABORTED, "collider build aborted");
 
     // sort (key, triangle) pairs: 4 passes of 8 bits
     if (nt > 1) {
         unsigned nb = blocks(nt, RS_TILE);
-        CK(dalloc(&d_hist, 256 * (size_t)nb));
-        CK(dalloc(&d_offs, 256 * (size_t)nb));
-        CK(dalloc(&d_stmp, scan_tmp_words(256 * nb)));
         uint32_t *ki = d_keys, *vi = d_vals, *ko = d_k2, *vo = d_v2;
         for (int shift = 0; shift < 32; shift += 8) {
             k_rs_hist<<<nb, 256>>>(ki, nt, shift, d_hist);
@@ -541,7 +534,6 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
     CK(dalloc(&C.d_slot, nt, &C.bytes));
     CKH(hipMemset(C.d_slot, 0, sizeof(uint32_t) * (size_t)(nt ? nt : 1)));   // degenerate triangles: never hit
     CK(dalloc(&C.d_queue, kRayQueues, &C.bytes));
-    CK(dalloc(&d_plo, n)); CK(dalloc(&d_phi, n));
     if (n) k_write_tris<<<blocks(n), 256>>>(n, d_vals, d_plane_u, d_sv_u, d_ev_u, d_bytes, d_blo_u, d_bhi_u,
                                             C.d_plane, C.d_rest, d_plo, d_phi, C.d_slot);
     CKH(hipGetLastError());
@@ -552,8 +544,6 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
     else if (n <= leafmax) C.root = make_leaf(0, n);
     else {
         const int ni = (int)n - 1;
-        CK(dalloc(&d_first, ni)); CK(dalloc(&d_last, ni)); CK(dalloc(&d_split, ni)); CK(dalloc(&d_pn, ni)); CK(dalloc(&d_pl, n));
-        CK(dalloc(&d_nlo, ni)); CK(dalloc(&d_nhi, ni)); CK(dalloc(&d_arrive, ni)); CK(dalloc(&d_depth, 1));
         CKH(hipMemset(d_arrive, 0, 4 * (size_t)ni));
         CKH(hipMemset(d_depth, 0, 4));
         k_karras<<<blocks(ni), 256>>>(d_keys, (int)n, d_first, d_last, d_split, d_pn, d_pl);
@@ -565,7 +555,7 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
                 uint32_t root_done = 0;
                 CKH(hipMemcpy(&root_done, d_arrive, 4, hipMemcpyDeviceToHost));
                 if (root_done) break;
-                if (k > 4096) { cleanup(); return fail(LSG_ERR_INVALID, "refit: no progress"); }
+                if (k > 4096) return fail(LSG_ERR_INVALID, "refit: no progress");
             }
         }
         k_write_nodes<<<blocks(ni), 256>>>((int)n, leafmax, C.margin, d_first, d_last, d_split, d_pn, d_plo, d_phi, d_nlo, d_nhi,
@@ -580,7 +570,7 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
             Node* s2 = nullptr;
             uint32_t nn = 0, d = 0;
             st = sah_rebuild_device(d_first, d_last, d_split, (int)n, leafmax, C.d_nodes, &s2, &nn, &d);
-            if (st > 1) { cleanup(); return st; }
+            if (st > 1) return st;
             if (st == 0) {
                 const int have = stack_size_for_depth(C.depth), want = stack_size_for_depth(d);
                 if (want && (!have || want <= have)) {
@@ -595,7 +585,6 @@ static int build(ColliderImpl& C, const float* verts, uint32_t nv, const uint32_
         }
     }
     CKH(hipDeviceSynchronize());
-    cleanup();
 #undef CK
 #undef CKH
     if (!stack_size_for_depth(C.depth))

@@ -9,6 +9,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <utility>
+#include <vector>
 #include "lsgpu.h"
 
 namespace lsg {
@@ -208,6 +210,27 @@ int pack4_device(ColliderImpl& C, const Node4* nodes4);
 // 1 = fewer than two leaves, 2 = malformed tree
 int sah_rebuild(const float* nodes, uint32_t nnodes, int32_t root, float* out, uint32_t* out_nodes, int32_t* out_root,
                 uint32_t* out_depth);
+
+// ---- scratch of the build steps ----------------------------------------------------------
+// one allocation for a step's arrays: parts are added, then placed
+struct Scratch {
+    std::vector<std::pair<void**, size_t>> parts;
+    void* base = nullptr;
+    Scratch() = default;
+    Scratch(const Scratch&) = delete;
+    ~Scratch() { if (base) (void)hipFree(base); }
+    template <class T> void add(T** p, size_t n) { parts.push_back({(void**)p, sizeof(T) * n}); }
+    int place()
+    {
+        size_t n = 0;
+        for (auto& q : parts) n += (q.second + 255) / 256 * 256;
+        hipError_t e = hipMalloc(&base, n ? n : 256);
+        if (e != hipSuccess) { base = nullptr; return hip_fail(e, "hipMalloc", __LINE__); }
+        char* c = (char*)base;
+        for (auto& q : parts) { *q.first = c; c += (q.second + 255) / 256 * 256; }
+        return LSG_OK;
+    }
+};
 
 // ---- texel rasterisation (lsgpu_raster.hip) ---------------------------------------------
 struct RasterObject {

@@ -267,24 +267,6 @@ __global__ __launch_bounds__(256) void k_raster_emit(const uint32_t* __restrict_
 
 inline unsigned blocks(uint64_t n) { return (unsigned)((n + 255) / 256); }
 
-// one allocation for a step's arrays: parts are added, then placed
-struct Scratch {
-    std::vector<std::pair<void**, size_t>> parts;
-    void* base = nullptr;
-    ~Scratch() { if (base) (void)hipFree(base); }
-    template <class T> void add(T** p, size_t n) { parts.push_back({(void**)p, sizeof(T) * n}); }
-    int place()
-    {
-        size_t n = 0;
-        for (auto& q : parts) n += (q.second + 255) / 256 * 256;
-        hipError_t e = hipMalloc(&base, n ? n : 256);
-        if (e != hipSuccess) { base = nullptr; return hip_fail(e, "hipMalloc", __LINE__); }
-        char* c = (char*)base;
-        for (auto& q : parts) { *q.first = c; c += (q.second + 255) / 256 * 256; }
-        return LSG_OK;
-    }
-};
-
 constexpr uint64_t kGroupCandidates = 1ull << 26;        // candidates rasterised together, unless one object has more
 
 // The texels and pieces of objects [o0, o1), whose triangles are [t0, t1) and have C

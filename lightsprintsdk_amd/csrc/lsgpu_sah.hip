@@ -2,16 +2,21 @@
 //
 // The same tree as the host rebuild (lsgpu_sah.cpp, lsg_bvh_rebuild_sah), built breadth
 // first: the leaves of the LBVH (triangle ranges of at most leaf_size, in the order of their
-// triangles) are rebuilt top-down, one wave per node of a level.  A wave bins its leaves'
-// centroids (32 bins per axis, as many as leaves below 32) into LDS, one lane picks the
-// cheapest split as the host does (area(left)·n(left) + area(right)·n(right) over the three
-// axes; equal centroids split the range in half), and the wave partitions its leaves stably
-// into the other buffer, collecting the children's boxes and centroid bounds.  Box and bound
+// triangles) are rebuilt top-down, one wave per node of a level (16 waves from kMidTask leaves
+// on).  It bins its leaves' centroids (32 bins per axis, as many as leaves below 32) into LDS, a
+// wave picks the cheapest split as the host does (area(left)·n(left) + area(right)·n(right) over
+// the three axes; equal centroids split the range in half), and the leaves are partitioned
+// stably into the other buffer, collecting the children's boxes and centroid bounds.  Box and bound
 // reductions are exact (min/max over floats as order-preserving integers), the split
 // arithmetic is the host's, and nodes are numbered in preorder (left child = node + 1, right
 // child = node + leaves on the left), so the result equals the host's node for node.
 // Tasks of 2^15 leaves or more (the top levels) take the same steps across the chip:
-// many workgroups bin, one lane splits, a scan of left/right flags partitions.
+// many workgroups bin, one wave splits, a scan of left/right flags partitions.
+//
+// The levels are short and depend on one another, so what a level costs is its slowest node and
+// the host's look at the next level's size.  50,000 triangles: 18 levels of 150 us (one lane
+// walking 3 x 32 bins twice, one wave over the root's 25,000 leaves) -> 94 us for the seven with
+// large nodes and 32 us below them, the collider's build 4.5 ms -> 3.1 ms.
 #include "lsgpu_internal.h"
 #include <algorithm>
 #include <cmath>
@@ -24,6 +29,7 @@ constexpr int kSahBins = 32;
 
 struct SahLeaf { int32_t ref; float b[6]; float c[3]; };
 struct SahTask { uint32_t begin, end, id, depth; float clo[3], chi[3]; };
+struct SahLevel { uint32_t ntask, maxm; };         // a level's tasks and the most leaves of one
 
 // floats as integers of the same order (-0 as +0), for atomic min/max
 __device__ inline int f2o(float x)
@@ -89,9 +95,10 @@ __global__ __launch_bounds__(256) void k_sah_root(const SahLeaf* __restrict__ L,
     else if (threadIdx.x < 6) atomicMax(&cb[threadIdx.x], s[threadIdx.x]);
 }
 
-__global__ void k_sah_root_task(const int* __restrict__ cb, uint32_t n, SahTask* __restrict__ t)
+__global__ void k_sah_root_task(const int* __restrict__ cb, uint32_t n, SahTask* __restrict__ t, SahLevel* __restrict__ lev)
 {
     if (threadIdx.x) return;
+    lev->ntask = 1; lev->maxm = n;
     SahTask r;
     r.begin = 0; r.end = n; r.id = 0; r.depth = 1;
     for (int a = 0; a < 3; a++) { r.clo[a] = o2f(cb[a]); r.chi[a] = o2f(cb[3 + a]); }
@@ -115,61 +122,91 @@ __device__ inline int bin_of(const SahLeaf& f, const SahTask& T, int a, float sc
     return min((int)((f.c[a] - T.clo[a]) * sc), nb - 1);
 }
 
-// the host's split search (lsgpu_sah.cpp) on a task's bins: dec = (axis or -1 for halves,
-// last bin on the left, leaves on the left)
+struct SahSweep { uint32_t c; float b[6]; };
+
+__device__ inline void sweep_add(SahSweep& a, bool on, int lane_delta)
+{
+    // the bins of another lane of this half wave added to this lane's, in range
+    SahSweep o;
+    o.c = lane_delta < 0 ? (uint32_t)__shfl_up((int)a.c, -lane_delta, 32) : (uint32_t)__shfl_down((int)a.c, lane_delta, 32);
+    for (int e = 0; e < 6; e++) {
+        o.b[e] = lane_delta < 0 ? __shfl_up(a.b[e], -lane_delta, 32) : __shfl_down(a.b[e], lane_delta, 32);
+        if (on) a.b[e] = (e & 1) ? fmaxf(a.b[e], o.b[e]) : fminf(a.b[e], o.b[e]);
+    }
+    if (on) a.c += o.c;
+}
+
+__device__ inline float sweep_area(const SahSweep& s)
+{
+    const float dx = s.b[1] - s.b[0], dy = s.b[3] - s.b[2], dz = s.b[5] - s.b[4];
+    return dx * dy + dy * dz + dz * dx;
+}
+
+// The host's split search (lsgpu_sah.cpp) on a task's bins: dec = (axis or -1 for halves, last
+// bin on the left, leaves on the left).  One wave: a lane per (axis, bin), axes 0 and 1 in the
+// half waves, then axis 2.  Boxes and counts of the bins up to a lane's and after it come from
+// scans (minima and maxima are exact in any order), every split's cost is the host's
+// expression, and of equal costs the first in the host's order is taken.  A NaN cost is never
+// below another, so it is taken only where the host meets it first.
 __device__ inline void sah_choose(const int (*cnt)[kSahBins], const int (*box)[kSahBins][6], int nb, const bool* ok, uint32_t m,
                                   int* dec)
 {
-    float best = 0.f;
+    const uint32_t lane = threadIdx.x & 63u;
+    const int k = (int)(lane & 31u);
+    uint64_t best = ~0ull;                       // (ordered cost, axis, bin)
+    uint32_t first = ~0u;                        // (axis, bin, NaN) of the first split
+    uint32_t left[2];
+    for (int pass = 0; pass < 2; pass++) {
+        const int a = pass ? 2 : (int)(lane >> 5);
+        const bool have = (pass == 0 || lane < 32) && k < nb;
+        SahSweep s{0u, {3.0e38f, -3.0e38f, 3.0e38f, -3.0e38f, 3.0e38f, -3.0e38f}};
+        if (have) {
+            s.c = (uint32_t)cnt[a][k];
+            for (int e = 0; e < 6; e++) s.b[e] = o2f(box[a][k][e]);
+        }
+        SahSweep r = s;
+        for (int d = 1; d < 32; d <<= 1) {
+            sweep_add(s, k >= d, -d);
+            sweep_add(r, k + d < 32, d);
+        }
+        left[pass] = s.c;
+        const float ra = __shfl_down(r.c ? sweep_area(r) : 0.f, 1, 32);
+        const uint32_t rc = (uint32_t)__shfl_down((int)r.c, 1, 32);
+        const bool okay = a == 0 ? ok[0] : (a == 1 ? ok[1] : ok[2]);
+        if (have && okay && k < nb - 1 && s.c && rc) {
+            const float cost = sweep_area(s) * (float)s.c + ra * (float)rc;
+            const uint32_t at = (uint32_t)(a * 32 + k);
+            const bool nan = cost != cost;
+            first = min(first, at * 2u + (nan ? 1u : 0u));
+            if (!nan) best = min(best, (uint64_t)((uint32_t)f2o(cost) ^ 0x80000000u) << 32 | at);
+        }
+    }
+    for (int o = 32; o; o >>= 1) {
+        first = min(first, (uint32_t)__shfl_xor((int)first, o));
+        const uint64_t b = (uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)best, o) | (uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)(best >> 32), o) << 32;
+        best = min(best, b);
+    }
     int bax = -1, bk = -1;
-    for (int a = 0; a < 3; a++) {
-        if (!ok[a]) continue;
-        float ra[kSahBins];
-        uint32_t rc[kSahBins];
-        float acc[6] = {3.0e38f, -3.0e38f, 3.0e38f, -3.0e38f, 3.0e38f, -3.0e38f};
-        uint32_t c = 0;
-        for (int k = nb - 1; k >= 0; k--) {
-            for (int e = 0; e < 6; e++) {
-                const float v = o2f(box[a][k][e]);
-                acc[e] = (e & 1) ? fmaxf(acc[e], v) : fminf(acc[e], v);
-            }
-            c += (uint32_t)cnt[a][k];
-            const float dx = acc[1] - acc[0], dy = acc[3] - acc[2], dz = acc[5] - acc[4];
-            ra[k] = c ? dx * dy + dy * dz + dz * dx : 0.f;
-            rc[k] = c;
-        }
-        for (int e = 0; e < 6; e++) acc[e] = (e & 1) ? -3.0e38f : 3.0e38f;
-        c = 0;
-        for (int k = 0; k < nb - 1; k++) {
-            for (int e = 0; e < 6; e++) {
-                const float v = o2f(box[a][k][e]);
-                acc[e] = (e & 1) ? fmaxf(acc[e], v) : fminf(acc[e], v);
-            }
-            c += (uint32_t)cnt[a][k];
-            if (!c || !rc[k + 1]) continue;
-            const float dx = acc[1] - acc[0], dy = acc[3] - acc[2], dz = acc[5] - acc[4];
-            const float cost = (dx * dy + dy * dz + dz * dx) * (float)c + ra[k + 1] * (float)rc[k + 1];
-            if (bax < 0 || cost < best) { best = cost; bax = a; bk = k; }
-        }
-    }
     uint32_t nl = m / 2;
-    if (bax >= 0) {
-        nl = 0;
-        for (int k = 0; k <= bk; k++) nl += (uint32_t)cnt[bax][k];
+    if (first != ~0u) {
+        const uint32_t at = (first & 1u) ? first >> 1 : (uint32_t)best;
+        bax = (int)(at >> 5); bk = (int)(at & 31u);
+        nl = (uint32_t)__shfl((int)(bax == 2 ? left[1] : left[0]), bax == 1 ? 32 + bk : bk);
     }
-    dec[0] = bax; dec[1] = bk; dec[2] = (int)nl;
+    if (lane == 0) { dec[0] = bax; dec[1] = bk; dec[2] = (int)nl; }
 }
 
 // a split task's node (children's boxes, a leaf child's ref from dst) and its children of
 // two or more leaves as the next level's tasks
 __device__ inline void sah_emit(const SahTask& T, uint32_t nl, const int (*child)[12], const SahLeaf* dst, Node* out, SahTask* next,
-                                uint32_t* nnext, uint32_t* depth)
+                                SahLevel* nlev, uint32_t* depth)
 {
     atomicMax(depth, T.depth);
     float nodef[16];
     // the children of two or more leaves become tasks, appended with one atomic
     const uint32_t nkids = (nl >= 2 ? 1u : 0u) + (T.end - T.begin - nl >= 2 ? 1u : 0u);
-    uint32_t slot = nkids ? atomicAdd(nnext, nkids) : 0u;
+    uint32_t slot = nkids ? atomicAdd(&nlev->ntask, nkids) : 0u;
+    if (nkids) atomicMax(&nlev->maxm, max(nl, T.end - T.begin - nl));
     for (int s = 0; s < 2; s++) {
         const uint32_t b = s == 0 ? T.begin : T.begin + nl, e = s == 0 ? T.begin + nl : T.end;
         const uint32_t ms = e - b;
@@ -202,10 +239,12 @@ __device__ inline void bins_init(int* cnt, int* box, uint32_t tid, uint32_t nthr
     }
 }
 
+// per child: box lo/hi x y z (6), centroid lo x y z, hi x y z (6)
+__device__ constexpr bool child_high(int e) { return e < 6 ? (e & 1) != 0 : e >= 9; }
+
 __device__ inline void child_init(int* child, uint32_t tid)
 {
-    // per child: box lo/hi x y z (6), centroid lo x y z, hi x y z (6)
-    if (tid < 24) child[tid] = ((tid % 12) < 6 ? ((tid & 1) ? f2o(-3.0e38f) : f2o(3.0e38f)) : ((tid % 12) < 9 ? f2o(3.0e38f) : f2o(-3.0e38f)));
+    if (tid < 24) child[tid] = child_high((int)(tid % 12)) ? f2o(-3.0e38f) : f2o(3.0e38f);
 }
 
 __device__ inline void bin_leaf(const SahLeaf& f, const SahTask& T, const bool* ok, const float* sc, int nb, int (*cnt)[kSahBins],
@@ -234,61 +273,107 @@ __device__ inline void child_add(int* cbx, const SahLeaf& f)
     }
 }
 
-// one node of a level per wave: bins, split, stable partition src -> dst, children
-__global__ __launch_bounds__(64) void k_sah_level(const SahTask* __restrict__ tasks, const SahLeaf* __restrict__ src,
-                                                  SahLeaf* __restrict__ dst, Node* __restrict__ out, SahTask* __restrict__ next,
-                                                  uint32_t* __restrict__ nnext, uint32_t* __restrict__ depth)
+// the smaller (larger) of v over the 16 lanes of a row, in every lane of it
+template <bool MAX> __device__ inline int row_extreme(int v)
+{
+    auto pick = [](int a, int b) { return MAX ? max(a, b) : min(a, b); };
+    v = pick(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true));      // lane ^ 1
+    v = pick(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true));      // lane ^ 2
+    v = pick(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true));     // mirrored in 8
+    v = pick(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true));     // mirrored in 16
+    return v;
+}
+
+// the nodes of a level of lo to hi - 1 leaves, one per workgroup of TH lanes: bins, split, stable
+// partition src -> dst, children.  The children's boxes and centroid bounds are kept per lane and
+// reduced once (all lanes of a wave adding to one LDS word would serialise).
+template <int TH>
+__global__ __launch_bounds__(TH) void k_sah_level(const SahTask* __restrict__ tasks, const SahLevel* __restrict__ lev, uint32_t lo, uint32_t hi,
+                                                  const SahLeaf* __restrict__ src, SahLeaf* __restrict__ dst, Node* __restrict__ out,
+                                                  SahTask* __restrict__ next, SahLevel* __restrict__ nlev, uint32_t* __restrict__ depth)
 {
     __shared__ int s_cnt[3][kSahBins];
     __shared__ int s_box[3][kSahBins][6];
     __shared__ int s_child[2][12];
     __shared__ int s_dec[3];                // axis (-1: halves), bin, leaves on the left
-    const uint32_t lane = threadIdx.x;
-    const SahTask T = tasks[blockIdx.x];
-    const uint32_t m = T.end - T.begin;
-    bool ok[3];
-    float sc[3];
-    const int nb = task_bins(T, ok, sc);
-    bins_init(&s_cnt[0][0], &s_box[0][0][0], lane, 64);
-    child_init(&s_child[0][0], lane);
-    __syncthreads();
-    for (uint32_t k = T.begin + lane; k < T.end; k += 64) bin_leaf(src[k], T, ok, sc, nb, s_cnt, s_box);
-    __syncthreads();
-    if (lane == 0) sah_choose(s_cnt, s_box, nb, ok, m, s_dec);
-    __syncthreads();
-    const int bax = s_dec[0], bk = s_dec[1];
-    const uint32_t nl = (uint32_t)s_dec[2];
-    uint32_t ldone = 0, rdone = 0;
-    for (uint32_t base = T.begin; base < T.end; base += 64) {
-        const uint32_t k = base + lane;
-        const bool valid = k < T.end;
-        SahLeaf f;
-        bool left = false;
-        if (valid) {
-            f = src[k];
-            left = bax < 0 ? (k - T.begin < m / 2) : (bin_of(f, T, bax, sc[bax], nb) <= bk);
+    __shared__ uint32_t s_left[TH / 64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t ntask = lev->ntask;
+    for (uint32_t q = blockIdx.x; q < ntask; q += gridDim.x) {
+        const SahTask T = tasks[q];
+        const uint32_t m = T.end - T.begin;
+        if (m < lo || m >= hi) continue;
+        bool ok[3];
+        float sc[3];
+        const int nb = task_bins(T, ok, sc);
+        bins_init(&s_cnt[0][0], &s_box[0][0][0], tid, TH);
+        child_init(&s_child[0][0], tid);
+        __syncthreads();
+        for (uint32_t k = T.begin + tid; k < T.end; k += TH) bin_leaf(src[k], T, ok, sc, nb, s_cnt, s_box);
+        __syncthreads();
+        if (wave == 0) sah_choose(s_cnt, s_box, nb, ok, m, s_dec);
+        __syncthreads();
+        const int bax = s_dec[0], bk = s_dec[1];
+        const uint32_t nl = (uint32_t)s_dec[2];
+        const float clo = bax == 0 ? T.clo[0] : (bax == 1 ? T.clo[1] : T.clo[2]), scb = bax == 0 ? sc[0] : (bax == 1 ? sc[1] : sc[2]);
+        uint32_t ldone = 0;
+        int ext[2][12];
+        for (int c = 0; c < 2; c++)
+            for (int e = 0; e < 12; e++) ext[c][e] = child_high(e) ? f2o(-3.0e38f) : f2o(3.0e38f);
+        for (uint32_t base = T.begin; base < T.end; base += TH) {
+            const uint32_t k = base + tid;
+            const bool valid = k < T.end;
+            SahLeaf f;
+            bool left = false;
+            if (valid) {
+                f = src[k];
+                const float c = bax == 0 ? f.c[0] : (bax == 1 ? f.c[1] : f.c[2]);
+                left = bax < 0 ? (k - T.begin < m / 2) : (min((int)((c - clo) * scb), nb - 1) <= bk);      // bin_of on that axis
+            }
+            const uint64_t lm = __ballot(valid && left);
+            uint32_t before = ldone, all = (uint32_t)__popcll(lm);
+            if (TH > 64) {
+                if (lane == 0) s_left[wave] = all;
+                __syncthreads();
+                all = 0;
+                for (uint32_t w = 0; w < TH / 64; w++) {
+                    if (w < wave) before += s_left[w];
+                    all += s_left[w];
+                }
+                __syncthreads();
+            }
+            before += (uint32_t)__popcll(lm & ((1ull << lane) - 1ull));     // leaves on the left before this one
+            if (valid) {
+                dst[left ? T.begin + before : T.begin + nl + (k - T.begin - before)] = f;
+                int v[12];
+                for (int e = 0; e < 6; e++) v[e] = f2o(f.b[e]);
+                for (int a = 0; a < 3; a++) v[6 + a] = v[9 + a] = f2o(f.c[a]);
+                for (int c = 0; c < 2; c++)
+                    if (left == (c == 0))
+                        for (int e = 0; e < 12; e++) ext[c][e] = child_high(e) ? max(ext[c][e], v[e]) : min(ext[c][e], v[e]);
+            }
+            ldone += all;
         }
-        const uint64_t lm = __ballot(valid && left), rm = __ballot(valid && !left);
-        const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
-        if (valid) {
-            const uint32_t at = left ? T.begin + ldone + (uint32_t)__popcll(lm & below)
-                                     : T.begin + nl + rdone + (uint32_t)__popcll(rm & below);
-            dst[at] = f;
-            child_add(s_child[left ? 0 : 1], f);
-        }
-        ldone += (uint32_t)__popcll(lm);
-        rdone += (uint32_t)__popcll(rm);
+        for (int c = 0; c < 2; c++)
+            for (int e = 0; e < 12; e++) {
+                const int v = child_high(e) ? row_extreme<true>(ext[c][e]) : row_extreme<false>(ext[c][e]);
+                if ((lane & 15u) == 0) { if (child_high(e)) atomicMax(&s_child[c][e], v); else atomicMin(&s_child[c][e], v); }
+            }
+        __syncthreads();
+        if (tid == 0) sah_emit(T, nl, s_child, dst, out, next, nlev, depth);
+        __syncthreads();
     }
-    __syncthreads();
-    if (lane == 0) sah_emit(T, nl, s_child, dst, out, next, nnext, depth);
 }
 
 // ---- one big task across the chip ------------------------------------------------------
 // The top levels have a handful of tasks over millions of leaves: each is binned by many
 // workgroups (LDS bins merged into global ones with the same exact integer min/max and
-// counts), split by one lane with the same search, partitioned stably by a scan of its
+// counts), split by one wave with the same search, partitioned stably by a scan of its
 // left/right flags, and emitted as k_sah_level emits.
 constexpr uint32_t kBigTask = 1u << 15;
+// from here on a task has 16 waves (the build of 50,000 triangles takes 3.03 to 3.16 ms with the
+// line anywhere from 2^7 to 2^11; one wave for all: 4.5 ms)
+constexpr uint32_t kMidTask = 1u << 9;
 
 struct SahBig {
     int cnt[3][kSahBins];
@@ -327,9 +412,8 @@ __global__ __launch_bounds__(256) void k_big_bin(const SahTask* __restrict__ tas
     }
 }
 
-__global__ void k_big_split(const SahTask* __restrict__ task, SahBig* __restrict__ B)
+__global__ __launch_bounds__(64) void k_big_split(const SahTask* __restrict__ task, SahBig* __restrict__ B)
 {
-    if (threadIdx.x) return;
     const SahTask T = *task;
     bool ok[3];
     float sc[3];
@@ -370,16 +454,15 @@ __global__ __launch_bounds__(256) void k_big_scatter(const SahTask* __restrict__
         const uint32_t k = threadIdx.x, e = k % 12;
         int* g = &B->child[0][0] + k;
         const int v = (&s_child[0][0])[k];
-        const bool hi = e < 6 ? (e & 1) != 0 : e >= 9;
-        if (hi) atomicMax(g, v); else atomicMin(g, v);
+        if (child_high((int)e)) atomicMax(g, v); else atomicMin(g, v);
     }
 }
 
 __global__ void k_big_emit(const SahTask* __restrict__ task, const SahLeaf* __restrict__ dst, const SahBig* __restrict__ B,
-                           Node* __restrict__ out, SahTask* __restrict__ next, uint32_t* __restrict__ nnext, uint32_t* __restrict__ depth)
+                           Node* __restrict__ out, SahTask* __restrict__ next, SahLevel* __restrict__ nlev, uint32_t* __restrict__ depth)
 {
     if (threadIdx.x) return;
-    sah_emit(*task, (uint32_t)B->dec[2], B->child, dst, out, next, nnext, depth);
+    sah_emit(*task, (uint32_t)B->dec[2], B->child, dst, out, next, nlev, depth);
 }
 
 // ---- BVH2 -> BVH4 collapse ------------------------------------------------------------
@@ -536,80 +619,75 @@ int sah_rebuild_device(const int* d_first, const int* d_last, const int* d_split
     *out_nodes = nullptr; *out_count = 0; *out_depth = 0;
     const int ni = nprim - 1;
     if (ni < 1) return 1;
-    uint32_t *flag = nullptr, *pos = nullptr, *tmp = nullptr, *total = nullptr, *cnt = nullptr, *dep = nullptr;
-    int* cb = nullptr;
-    SahLeaf *L0 = nullptr, *L1 = nullptr;
-    SahTask *T0 = nullptr, *T1 = nullptr, *tsmall = nullptr;
-    SahBig* big = nullptr;
+    constexpr uint32_t kMaxLevels = 4096, kAhead = 4;    // levels launched between the host's looks
+    uint32_t *flag, *pos, *tmp, *total, *dep;
+    int* cb;
+    SahLeaf *L0, *L1;
+    SahTask *T0, *T1;
+    SahBig* big;
+    SahLevel* lev;
     Node* out = nullptr;
-    auto cleanup = [&]() {
-        sfree(flag); sfree(pos); sfree(tmp); sfree(total); sfree(cnt); sfree(dep); sfree(cb);
-        sfree(L0); sfree(L1); sfree(T0); sfree(T1); sfree(tsmall); sfree(big);
-    };
-#define SK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { cleanup(); sfree(out); return hip_fail(e_, #x, __LINE__); } } while (0)
+#define SK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { sfree(out); return hip_fail(e_, #x, __LINE__); } } while (0)
     const unsigned gb = (unsigned)((ni + 255) / 256);
-    SK(hipMalloc(&flag, 4 * (size_t)nprim));
-    SK(hipMalloc(&pos, 4 * (size_t)nprim));
-    SK(hipMalloc(&tmp, 4 * scan_tmp_words((uint32_t)nprim)));
-    SK(hipMalloc(&total, 4));
-    SK(hipMemset(flag, 0, 4 * (size_t)nprim));
+    Scratch A, B;
+    A.add(&flag, nprim); A.add(&pos, nprim); A.add(&tmp, scan_tmp_words((uint32_t)nprim)); A.add(&total, 1); A.add(&dep, 1); A.add(&cb, 6);
+    A.add(&big, 1); A.add(&lev, kMaxLevels + kAhead + 2);
+    if (int st = A.place()) return st;
+    SK(hipMemsetAsync(flag, 0, 4 * (size_t)nprim, nullptr));
+    SK(hipMemsetAsync(dep, 0, 4, nullptr));
+    SK(hipMemsetAsync(lev, 0, sizeof(SahLevel) * (kMaxLevels + kAhead + 2), nullptr));
     k_sah_mark<<<gb, 256>>>(ni, d_first, d_last, d_split, leafmax, flag);
     SK(hipGetLastError());
-    if (int st = scan_exclusive_u32(flag, pos, (uint32_t)nprim, total, tmp, nullptr)) { cleanup(); return st; }
+    if (int st = scan_exclusive_u32(flag, pos, (uint32_t)nprim, total, tmp, nullptr)) return st;
     uint32_t n = 0;
     SK(hipMemcpy(&n, total, 4, hipMemcpyDeviceToHost));
-    if (n < 2) { cleanup(); return 1; }
-    SK(hipMalloc(&L0, sizeof(SahLeaf) * (size_t)n));
-    SK(hipMalloc(&L1, sizeof(SahLeaf) * (size_t)n));
+    if (n < 2) return 1;
+    const uint32_t cap = n / 2 + 1;
+    B.add(&L0, n); B.add(&L1, n); B.add(&T0, cap); B.add(&T1, cap);
+    if (int st = B.place()) return st;
+    SK(hipMalloc(&out, sizeof(Node) * (size_t)(n - 1)));
     k_sah_gather<<<gb, 256>>>(ni, d_first, d_last, d_split, leafmax, d_nodes, pos, L0);
-    SK(hipGetLastError());
     // the root task: every leaf, its centroid bounds
-    SK(hipMalloc(&cb, 24));
     {
         const int init[6] = {0x7f7fffff, 0x7f7fffff, 0x7f7fffff, (int)0x80800000, (int)0x80800000, (int)0x80800000};
         SK(hipMemcpy(cb, init, 24, hipMemcpyHostToDevice));   // lo = max float, hi = ordered -max float
     }
     k_sah_root<<<std::min(1024u, (n + 255) / 256), 256>>>(L0, n, cb);
-    const uint32_t cap = n / 2 + 1;
-    SK(hipMalloc(&T0, sizeof(SahTask) * (size_t)cap));
-    SK(hipMalloc(&T1, sizeof(SahTask) * (size_t)cap));
-    k_sah_root_task<<<1, 64>>>(cb, n, T0);
-    SK(hipMalloc(&out, sizeof(Node) * (size_t)(n - 1)));
-    SK(hipMalloc(&cnt, 4));
-    SK(hipMalloc(&dep, 4));
-    SK(hipMemset(dep, 0, 4));
+    k_sah_root_task<<<1, 64>>>(cb, n, T0, lev);
     SK(hipGetLastError());
-    // tasks of at least kBigTask leaves go across the chip (the top levels); the host reads
-    // the task list while it is short to find them.  flag, pos and tmp are free by now and
-    // hold the big tasks' flags, their prefix and the scan's scratch.
-    constexpr uint32_t kHostTasks = 1024;
-    SK(hipMalloc(&big, sizeof(SahBig)));
-    SK(hipMalloc(&tsmall, sizeof(SahTask) * kHostTasks));
-    std::vector<SahTask> ht, small;
+    // While a level has tasks of kMidTask leaves or more, the host looks at every level: tasks of
+    // at least kBigTask leaves go across the chip, and the host reads the task list while it
+    // is short to find them.  Below that, kAhead levels are launched at a time, each taking its
+    // number of tasks from the level before.  flag, pos and tmp are free by now and hold the
+    // big tasks' flags, their prefix and the scan's scratch.
+    constexpr uint32_t kHostTasks = 1024, kGrid = 16384, kNoLimit = 0xffffffffu;
+    std::vector<SahTask> ht;
     std::vector<uint32_t> bigs;
-    uint32_t ntask = 1;
+    SahLevel now{1, n};
     SahLeaf *src = L0, *dst = L1;
     SahTask *tin = T0, *tout = T1;
-    for (uint32_t level = 0; ntask; level++) {
-        if (level > 4096) { cleanup(); sfree(out); return fail(LSG_ERR_INVALID, "sah_rebuild_device: no progress"); }
-        SK(hipMemset(cnt, 0, 4));
-        bigs.clear();
-        small.clear();
-        if (ntask <= kHostTasks) {
-            ht.resize(ntask);
-            SK(hipMemcpy(ht.data(), tin, sizeof(SahTask) * ntask, hipMemcpyDeviceToHost));
-            for (uint32_t i = 0; i < ntask; i++) {
-                if (ht[i].end - ht[i].begin >= kBigTask) bigs.push_back(i);
-                else small.push_back(ht[i]);
+    for (uint32_t level = 0; now.ntask;) {
+        if (level > kMaxLevels) { sfree(out); return fail(LSG_ERR_INVALID, "sah_rebuild_device: no progress"); }
+        if (now.maxm < kMidTask) {
+            uint64_t bound = now.ntask;
+            for (uint32_t j = 0; j < kAhead; j++, bound *= 2) {
+                k_sah_level<64><<<(unsigned)std::min<uint64_t>(std::min<uint64_t>(bound, cap), kGrid), 64>>>(tin, lev + level, 0, kNoLimit, src, dst, out,
+                                                                                                    tout, lev + level + 1, dep);
+                level++;
+                std::swap(src, dst);
+                std::swap(tin, tout);
             }
-        }
-        if (bigs.empty()) {
-            k_sah_level<<<ntask, 64>>>(tin, src, dst, out, tout, cnt, dep);
         } else {
-            if (!small.empty()) {
-                SK(hipMemcpy(tsmall, small.data(), sizeof(SahTask) * small.size(), hipMemcpyHostToDevice));
-                k_sah_level<<<(unsigned)small.size(), 64>>>(tsmall, src, dst, out, tout, cnt, dep);
+            bigs.clear();
+            if (now.maxm >= kBigTask && now.ntask <= kHostTasks) {
+                ht.resize(now.ntask);
+                SK(hipMemcpy(ht.data(), tin, sizeof(SahTask) * now.ntask, hipMemcpyDeviceToHost));
+                for (uint32_t i = 0; i < now.ntask; i++) if (ht[i].end - ht[i].begin >= kBigTask) bigs.push_back(i);
             }
+            const unsigned grid = std::min(now.ntask, kGrid);
+            k_sah_level<64><<<grid, 64>>>(tin, lev + level, 0, kMidTask, src, dst, out, tout, lev + level + 1, dep);
+            k_sah_level<1024><<<std::min(grid, 1024u), 1024>>>(tin, lev + level, kMidTask, bigs.empty() ? kNoLimit : kBigTask, src, dst, out, tout,
+                                                               lev + level + 1, dep);
             for (uint32_t i : bigs) {
                 const SahTask* t = tin + i;
                 const uint32_t m = ht[i].end - ht[i].begin;
@@ -618,20 +696,20 @@ int sah_rebuild_device(const int* d_first, const int* d_last, const int* d_split
                 k_big_bin<<<g, 256>>>(t, src, big);
                 k_big_split<<<1, 64>>>(t, big);
                 k_big_flag<<<g, 256>>>(t, src, big, flag);
-                if (int st = scan_exclusive_u32(flag, pos, m, nullptr, tmp, nullptr)) { cleanup(); sfree(out); return st; }
+                if (int st = scan_exclusive_u32(flag, pos, m, nullptr, tmp, nullptr)) { sfree(out); return st; }
                 k_big_scatter<<<g, 256>>>(t, src, dst, flag, pos, big);
-                k_big_emit<<<1, 64>>>(t, dst, big, out, tout, cnt, dep);
+                k_big_emit<<<1, 64>>>(t, dst, big, out, tout, lev + level + 1, dep);
             }
+            level++;
+            std::swap(src, dst);
+            std::swap(tin, tout);
         }
         SK(hipGetLastError());
-        SK(hipMemcpy(&ntask, cnt, 4, hipMemcpyDeviceToHost));
-        if (ntask > cap) { cleanup(); sfree(out); return fail(LSG_ERR_INVALID, "sah_rebuild_device: %u tasks over %u", ntask, cap); }
-        std::swap(src, dst);
-        std::swap(tin, tout);
+        SK(hipMemcpy(&now, lev + level, sizeof now, hipMemcpyDeviceToHost));
+        if (now.ntask > cap) { sfree(out); return fail(LSG_ERR_INVALID, "sah_rebuild_device: %u tasks over %u", now.ntask, cap); }
     }
     uint32_t d = 0;
     SK(hipMemcpy(&d, dep, 4, hipMemcpyDeviceToHost));
-    cleanup();
 #undef SK
     *out_nodes = out; *out_count = n - 1; *out_depth = d;
     return 0;
@@ -645,38 +723,28 @@ int collapse4_device(ColliderImpl& C, uint32_t budget, Node4** nodes4)
 {
     *nodes4 = nullptr;
     const uint32_t nn = C.nnodes;
-    uint32_t *H = nullptr, *cnt = nullptr, *prefix = nullptr, *pnext = nullptr, *tmp = nullptr, *total = nullptr,
-             *need = nullptr;
-    C4Work *w0 = nullptr, *w1 = nullptr;
+    uint32_t *H, *cnt, *prefix, *pnext, *tmp, *total, *need;
+    C4Work *w0, *w1;
     Node4* out = nullptr;
-    auto cleanup = [&]() {
-        sfree(H); sfree(cnt); sfree(prefix); sfree(pnext); sfree(tmp); sfree(total); sfree(need);
-        sfree(w0); sfree(w1);
-    };
-#define SK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { cleanup(); sfree(out); return hip_fail(e_, #x, __LINE__); } } while (0)
+#define SK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { sfree(out); return hip_fail(e_, #x, __LINE__); } } while (0)
     const unsigned gb = (nn + 255) / 256;
-    SK(hipMalloc(&H, 4 * (size_t)nn));
-    SK(hipMemset(H, 0, 4 * (size_t)nn));
+    Scratch A;
+    A.add(&H, nn); A.add(&w0, nn); A.add(&w1, nn); A.add(&cnt, nn); A.add(&prefix, nn); A.add(&pnext, nn); A.add(&tmp, scan_tmp_words(nn));
+    A.add(&total, 1); A.add(&need, 1);
+    if (int st = A.place()) return st;
+    SK(hipMemsetAsync(H, 0, 4 * (size_t)nn, nullptr));
     uint32_t hroot = 0;
     for (uint32_t k = 1;; k++) {
         k_c4_height<<<gb, 256>>>(nn, C.d_nodes, H, k);
         if (k % 8 == 0) {
             SK(hipMemcpy(&hroot, H + C.root, 4, hipMemcpyDeviceToHost));
             if (hroot) break;
-            if (k > 4096) { cleanup(); return fail(LSG_ERR_INVALID, "collapse4: no progress"); }
+            if (k > 4096) return fail(LSG_ERR_INVALID, "collapse4: no progress");
         }
     }
     SK(hipGetLastError());
-    if (hroot > budget) { cleanup(); return fail(LSG_ERR_LIMIT, "collapse4: tree height %u over stack budget %u", hroot, budget); }
+    if (hroot > budget) return fail(LSG_ERR_LIMIT, "collapse4: tree height %u over stack budget %u", hroot, budget);
     SK(hipMalloc(&out, sizeof(Node4) * (size_t)nn));
-    SK(hipMalloc(&w0, sizeof(C4Work) * (size_t)nn));
-    SK(hipMalloc(&w1, sizeof(C4Work) * (size_t)nn));
-    SK(hipMalloc(&cnt, 4 * (size_t)nn));
-    SK(hipMalloc(&prefix, 4 * (size_t)nn));
-    SK(hipMalloc(&pnext, 4 * (size_t)nn));
-    SK(hipMalloc(&tmp, 4 * scan_tmp_words(nn)));
-    SK(hipMalloc(&total, 4));
-    SK(hipMalloc(&need, 4));
     SK(hipMemset(need, 0, 4));
     {
         const C4Work r{C.root, 0u, 0u};
@@ -684,10 +752,10 @@ int collapse4_device(ColliderImpl& C, uint32_t budget, Node4** nodes4)
     }
     uint32_t nw = 1, n4 = 1;
     while (nw) {
-        if (n4 > nn) { cleanup(); sfree(out); return fail(LSG_ERR_INVALID, "collapse4: more BVH4 nodes than BVH2 nodes"); }
+        if (n4 > nn) { sfree(out); return fail(LSG_ERR_INVALID, "collapse4: more BVH4 nodes than BVH2 nodes"); }
         const unsigned g = (nw + 255) / 256;
         k_c4_open<<<g, 256>>>(w0, nw, C.d_nodes, H, budget, out, cnt, pnext, need);
-        if (int st = scan_exclusive_u32(cnt, prefix, nw, total, tmp, nullptr)) { cleanup(); sfree(out); return st; }
+        if (int st = scan_exclusive_u32(cnt, prefix, nw, total, tmp, nullptr)) { sfree(out); return st; }
         k_c4_link<<<g, 256>>>(w0, nw, prefix, pnext, n4, out, w1);
         SK(hipGetLastError());
         uint32_t t = 0;
@@ -698,7 +766,6 @@ int collapse4_device(ColliderImpl& C, uint32_t budget, Node4** nodes4)
     }
     uint32_t sn = 0;
     SK(hipMemcpy(&sn, need, 4, hipMemcpyDeviceToHost));
-    cleanup();
 #undef SK
     *nodes4 = out;
     C.nnodes4 = n4; C.root4 = 0; C.stack_need = sn;

@@ -54,6 +54,35 @@ def test_gpu_tree_equals_oracle_tree(gpu, oracle, freq, leaf):
     np.testing.assert_array_equal(t_sah["nodes"].view(np.uint32), want["nodes"].view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [2, 3, 5, 31, 33, 63, 64, 65, 130, 511, 512, 513, 1025, 3000])
+@pytest.mark.parametrize("kind", ["soup", "flat", "stacked"])
+def test_gpu_sah_tree_at_task_sizes(gpu, n, kind):
+    """The GPU SAH rebuild equals the host's node for node where a node's leaves fill a wave, or
+    pass from one wave to sixteen, with an axis whose centroids coincide (flat) and with many
+    equal centroids (stacked: split in halves)."""
+    from lightsprintsdk_amd.collider import rebuild_sah
+    rng = np.random.default_rng(n)
+    c = rng.uniform(-1, 1, (n, 1, 3))
+    if kind == "flat":
+        c[..., 1] = 0.25
+    if kind == "stacked":
+        c = c[rng.integers(0, max(1, n // 40), n)]
+    e = rng.uniform(-0.05, 0.05, (n, 3, 3))
+    if kind == "flat":
+        e[..., 1] = 0
+    if kind == "stacked":
+        e[:] = e[:1]
+    V = np.ascontiguousarray((c + e).reshape(-1, 3), np.float32)
+    I = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    lb = _col(V, I, 1, lbvh_only=True).download_tree()
+    want = rebuild_sah(lb)
+    got = _col(V, I, 1).download_tree()
+    assert got["root"] == want["root"]
+    if want["depth"] <= lb["depth"]:
+        assert got["depth"] == want["depth"]
+        np.testing.assert_array_equal(got["nodes"].view(np.uint32), want["nodes"].view(np.uint32))
+
+
 def test_gpu_vs_oracle_small(gpu, oracle):
     V, I = scenes.icosphere(10, seed=12)
     R = scenes.random_rays(V, 20000, seed=13)
