@@ -118,6 +118,33 @@ def test_gpu_wrap_filters_vs_oracle(gpu, oracle, sigma, spread):
         plan.close()
 
 
+@pytest.mark.parametrize("wrap", [False, True])
+@pytest.mark.parametrize("sigma", [0.0, 0.5, 1.16, 1.2, 2.5])
+def test_gpu_blur_tiles_vs_oracle(gpu, oracle, sigma, wrap):
+    """Blur passes in tiles, at the tiles' edges and where the halo is wider than the map: no
+    pass, one, the most a launch takes, one more, several launches; and an infinite texel, which
+    a neighbour outside the blur flags still reaches times a weight of 0.  The same terms in
+    the same order as the oracle's."""
+    shapes = [(1, 1), (2, 3), (4, 40), (31, 32), (32, 33), (33, 31), (64, 65), (1, 70), (70, 1), (100, 41)]
+    rng = np.random.default_rng(int(sigma * 100) + wrap)
+    imgs = [_random_map(rng, w, h, fill=0.8) for w, h in shapes]
+    for m in imgs:
+        m[..., 3] = np.where(m[..., 3] > 0, np.float32(1), 0)      # all edges and quadrants
+    imgs[6][0, 5, 0] = np.inf
+    imgs[6][40, 63, 1] = np.inf
+    plan = _FilterPlan(shapes)
+    try:
+        print(f"blur sigma {sigma} wrap {wrap}", flush=True)
+        got = plan.run(imgs, sigma, 3.0, wrap)
+        for k, m in enumerate(imgs):
+            with np.errstate(invalid="ignore"):
+                rgba, rgbf = oracle.filter_lightmap_ex(m, sigma=sigma, spread=3.0, wrap=wrap)
+            np.testing.assert_array_equal(got[k][0], rgba, err_msg=f"map {k} rgba")
+            np.testing.assert_array_equal(got[k][1], rgbf, err_msg=f"map {k} rgbf")
+    finally:
+        plan.close()
+
+
 @pytest.mark.parametrize("spread", [1.0, 15.0, 16.0, 17.0, 32.0, 33.0, 1000.0])
 def test_gpu_grow_tiles_vs_oracle(gpu, oracle, spread):
     """lightmapGrow at the edges of its 32-texel tiles and 16-step launches: few filled texels
