@@ -315,9 +315,9 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur_tiles(const FilterMap* __
 //
 // One launch does what 16 launches over a frontier list did (each a few hundred to a few
 // thousand texels: 8 to 16 us of launch and latency).  5 maps of 1013 x 731, 96 steps: 1.54 ms +
-// 0.26 ms to seed the list -> 0.55 ms (8 launches of 68 us; reading the marks with their
+// 0.26 ms to seed the list -> 0.52 ms (8 launches of 65 us; reading the marks with their
 // halos alone takes 12 us); a light-layer call of 9 maps of 97^2, five chains: 5.6 -> 2.9 ms.  256
-// threads a tile: 0.72 ms, 1024: 0.58 ms (two workgroups per CU either way, by LDS).
+// threads a tile: 0.70 ms, 1024: 0.69 ms (two workgroups per CU either way, by LDS).
 constexpr uint32_t kHalo = 16, kRegion = 64, kTileSteps = 16, kTileThreads = 512, kTileWaves = kTileThreads / 64;
 constexpr uint32_t kStrip = kRegion / kTileWaves;       // columns of a wave
 constexpr uint32_t kValPitch = kRegion + 1;             // odd: a column's texels lie in different banks
@@ -442,16 +442,21 @@ __global__ __launch_bounds__(kTileThreads) void k_grow_tiles(const FilterMap* __
                         const float4 e = f4add(f4add(f4add(old(xp, yc), old(xm, yc)), old(xc, yp)), old(xc, ym));
                         const float4 dg = f4add(f4add(f4add(old(xp, yp), old(xp, ym)), old(xm, yp)), old(xm, ym));
                         const float4 d = f4add(f4mul(e, 1.6f), dg);
-                        const float4 nv = make_float4(d.x / d.w, d.y / d.w, d.z / d.w, sf);
-                        val[yc * (int)kValPitch + xc] = nv;
-                        if ((uint32_t)xc - kHalo < kTile && (uint32_t)yc - kHalo < kTile) {
-                            const uint32_t g = M.first + (uint32_t)(gx + gy * w);
-                            img[g] = make_float4(nv.x, nv.y, nv.z, 0.001f);
-                            mark[g] = base + s;
-                            last = base + s;
-                        }
+                        val[yc * (int)kValPitch + xc] = make_float4(d.x / d.w, d.y / d.w, d.z / d.w, sf);
                     }
                     __syncthreads();
+                }
+                // the tile's new texels (not written in the steps, whose barriers would wait for
+                // the stores)
+                for (uint32_t i = tid; i < kTile * kTile; i += kTileThreads) {
+                    const uint32_t xc = kHalo + i % kTile, yc = kHalo + i / kTile;
+                    const float4 v = val[yc * kValPitch + xc];
+                    if (v.w > 0.f && v.w < kNever) {
+                        const uint32_t g = M.first + (uint32_t)((x0 + (int)xc) + (y0 + (int)yc) * w);
+                        img[g] = make_float4(v.x, v.y, v.z, 0.001f);
+                        mark[g] = base + (uint32_t)v.w;
+                        last = max(last, base + (uint32_t)v.w);
+                    }
                 }
                 if (wave == 0) {
                     const uint64_t tile = ((1ull << kTile) - 1ull) << kHalo;
