@@ -58,3 +58,32 @@ def test_gpu_encode_bake(gpu):
         np.testing.assert_array_equal(got, model(rgba, bg, 0, 1, 0))
         assert got.max() > 0
     plan.close()
+
+
+@pytest.mark.parametrize("fmt", [0, 2])
+def test_gpu_encode_bytes_at_their_borders(gpu, fmt):
+    """sRGB bytes where the binary32 power alone cannot tell the byte: every value whose
+    power is within a few units in the last place of k / 256, values a little further, and
+    0, 1, negatives, huge values, infinities and NaN; against the closed form in binary64."""
+    k = np.arange(1, 257) / 256.0
+    mid = (k ** (1.0 / np.float64(np.float32(0.45)))).astype(np.float32)
+    vals = [mid]
+    for _ in range(4):
+        vals.append(np.nextafter(vals[-1], np.float32(9)))
+    lo = mid
+    for _ in range(4):
+        lo = np.nextafter(lo, np.float32(-1))
+        vals.append(lo)
+    for r in (2.0 ** -10, 2.0 ** -9, 2.0 ** -8):
+        vals += [mid * np.float32(1 + r / 4), mid * np.float32(1 - r / 4), mid * np.float32(1 + r), mid * np.float32(1 - r)]
+    rng = np.random.default_rng(6)
+    vals.append(np.float32(10) ** rng.uniform(-9, 1, 20000).astype(np.float32))
+    vals.append(np.float32([0, -0.0, 1, -1, -1e-3, 1e-45, 1e-38, 1e9, 3e38, -3e38, np.inf, -np.inf, np.nan]))
+    x = np.concatenate(vals).astype(np.float32)
+    x = x[:len(x) // 3 * 3].reshape(-1, 3)
+    rgba = np.ones((len(x), 4), np.float32)
+    rgba[:, :3] = x
+    bg = np.zeros(4, np.float32)
+    with np.errstate(all="ignore"):
+        want = model(rgba, bg, fmt, 1, 0)
+    np.testing.assert_array_equal(_encode(rgba, fmt, 1, 0, bg), want)
