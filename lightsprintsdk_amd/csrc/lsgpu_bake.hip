@@ -267,7 +267,7 @@ int lsg_bake_create(lsg_scene* scene, const lsg_bake_object* objects, uint32_t n
     if (!B.d_sub) AL(B.d_sub, 0);
     AL(B.d_rgba, 16 * (size_t)slot);
     AL(B.d_rgbf, 12 * (size_t)slot);
-    AL(B.d_queue, 64);
+    AL(B.d_queue, 4 * kQueueWords);
     AL(B.d_walk, 32 * (size_t)B.ntex);
     // 2. first-gather work: one texel per triangle covering the whole triangle
     AL(B.d_ttex, sizeof(lsg_texel) * B.ntri);

@@ -1503,7 +1503,7 @@ __global__ __launch_bounds__(256) void k_gather_grouped_layers(GatherArgs A)
 
 __global__ void k_queue_reset(uint32_t* counters, uint32_t n)
 {
-    if (threadIdx.x < n) counters[threadIdx.x] = 0;
+    if (threadIdx.x < n) counters[threadIdx.x * kQueueStride] = 0;
 }
 
 // Capped at 128 VGPRs it runs 4 waves per SIMD, measured faster than 3 with more
@@ -1518,25 +1518,37 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     __shared__ uint32_t pscr[WAVES * kPermScr];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t home = Q.nqueues > 1 ? blockIdx.x % Q.nqueues : 0;
-    for (uint32_t qi = 0; qi < Q.nqueues; qi++) {
-        const uint32_t q = (home + qi) % Q.nqueues;
-        const uint32_t t0 = (uint32_t)((uint64_t)Q.ntiles * q / Q.nqueues);
-        const uint32_t t1 = (uint32_t)((uint64_t)Q.ntiles * (q + 1) / Q.nqueues);
-        for (;;) {
-            uint32_t k = 0;
-            if (lane == 0) k = atomicAdd(&Q.counters[q], 1u);
-            k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);   // lane 0's tile, scalar
-            const uint32_t tile = t0 + k;
-            if (tile >= t1) break;           // this queue is exhausted for every lane of the wave
-            const uint32_t a = tile * Q.tile, b = min(A.ntex, a + Q.tile);
-            for (uint32_t ti = a; ti < b; ti++)
-                if constexpr (REFILL) gather_texel_refill<STACK, FEAT>(A, ti, lane, stk + tid, lq + tid, lqj + tid, 64 * WAVES,
-                                                                     subc + (tid >> 6) * kFrame * kSubCache,
-                                                                     pscr + (tid >> 6) * kPermScr);
-                else gather_texel<STACK, false, 64, false, FEAT>(A, ti, lane, stk + tid, lq + tid, lqj + tid, 64 * WAVES,
-                                                                subc + (tid >> 6) * kFrame * kSubCache,
-                                                                pscr + (tid >> 6) * kPermScr);
+    const uint32_t shift = Q.nqueues > 1 ? 3u : 0u;      // 8 queues or 1
+    auto first_tile = [&](uint32_t i) { return (uint32_t)((uint64_t)Q.ntiles * i >> shift); };
+    uint32_t q = home;
+    for (;;) {
+        const uint32_t t0 = first_tile(q), t1 = first_tile(q + 1);
+        uint32_t k = 0;
+        if (lane == 0) k = atomicAdd(&Q.counters[q * kQueueStride], 1u);
+        k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);   // lane 0's tile, scalar
+        const uint32_t tile = t0 + k;
+        if (tile >= t1) {
+            // this queue is exhausted: on to the next one that had tiles left when looked at (a
+            // lane per queue, from the home queue on); counters only grow, so this ends
+            const uint32_t ql = (home + lane) % Q.nqueues;
+            bool open = false;
+            if (lane < Q.nqueues) {
+                const uint32_t taken = __hip_atomic_load(&Q.counters[ql * kQueueStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                open = taken < first_tile(ql + 1) - first_tile(ql);
+            }
+            const uint64_t left = __ballot(open);
+            if (!left) break;
+            q = (home + (uint32_t)__ffsll((unsigned long long)left) - 1u) % Q.nqueues;
+            continue;
         }
+        const uint32_t a = tile * Q.tile, b = min(A.ntex, a + Q.tile);
+        for (uint32_t ti = a; ti < b; ti++)
+            if constexpr (REFILL) gather_texel_refill<STACK, FEAT>(A, ti, lane, stk + tid, lq + tid, lqj + tid, 64 * WAVES,
+                                                                 subc + (tid >> 6) * kFrame * kSubCache,
+                                                                 pscr + (tid >> 6) * kPermScr);
+            else gather_texel<STACK, false, 64, false, FEAT>(A, ti, lane, stk + tid, lq + tid, lqj + tid, 64 * WAVES,
+                                                            subc + (tid >> 6) * kFrame * kSubCache,
+                                                            pscr + (tid >> 6) * kPermScr);
     }
 }
 
@@ -1625,8 +1637,8 @@ int gather_args(lsg_scene* s, const lsg_texel* texels, uint32_t ntexels, const l
     A.pq = nullptr;
     {
         SceneImpl& SP = s->impl;
-        if (!SP.d_pq) LSG_HIP(hipMalloc(&SP.d_pq, sizeof(uint32_t) * 8 * kQueueSlots));
-        A.pq = SP.d_pq + 8 * (__atomic_fetch_add(&SP.pq_next, 1u, __ATOMIC_RELAXED) % kQueueSlots);
+        if (!SP.d_pq) LSG_HIP(hipMalloc(&SP.d_pq, sizeof(uint32_t) * kQueueWords * kQueueSlots));
+        A.pq = SP.d_pq + kQueueWords * (__atomic_fetch_add(&SP.pq_next, 1u, __ATOMIC_RELAXED) % kQueueSlots);
     }
     return LSG_OK;
 }
