@@ -488,7 +488,7 @@ typedef struct lsg_bake_object {
 
 /* launch shape of the persistent gather; 0 = default (picked by lsg_bake_autotune) */
 typedef struct lsg_bake_tuning {
-    uint32_t tile;             /* texels per work-queue fetch (default 2) */
+    uint32_t tile;             /* texels per work-queue fetch (default 1 up to 131072 texels, else 2) */
     uint32_t waves_per_block;  /* 2, 4 or 8 (default 4) */
     uint32_t blocks_per_cu;    /* persistent workgroups per compute unit (default 4) */
     uint32_t xcd_queues;       /* 8 = one work queue per XCD, 1 = one global queue (default 8) */

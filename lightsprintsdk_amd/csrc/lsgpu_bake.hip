@@ -128,9 +128,14 @@ struct BakeImpl {
     }
 };
 
-static void default_tuning(lsg_bake_tuning& t)
+// Tiles of two texels halve the additions to the queues' counters, tiles of one end a launch more
+// evenly: with 4096 waves at work, 21,890 texels of 256 rays take 1.010 ms against 1.068, 92,744
+// texels 2.83 against 2.85, and 735,719 texels of 64 rays 8.20 against 8.00 ms.
+constexpr uint32_t kSingleTiles = 1u << 17;
+
+static void default_tuning(lsg_bake_tuning& t, uint32_t ntex)
 {
-    if (!t.tile) t.tile = 2;
+    if (!t.tile) t.tile = ntex <= kSingleTiles ? 1 : 2;
     if (!t.waves_per_block) t.waves_per_block = 4;
     if (!t.blocks_per_cu) t.blocks_per_cu = 4;
     if (!t.xcd_queues) t.xcd_queues = 8;
@@ -145,7 +150,7 @@ static int run_gather_final(BakeImpl& B, const lsg_gather_params* p, const lsg_t
     if (e) return e;
     A.walk_buf = B.d_walk; A.walk_cap = B.ntex;   // the plan's own records: nothing allocated under capture
     lsg_bake_tuning t = B.tuning;
-    default_tuning(t);
+    default_tuning(t, B.ntex);
     WorkQueue Q;
     Q.counters = B.d_queue; Q.nqueues = t.xcd_queues > 1 ? 8 : 1; Q.tile = t.tile;
     Q.ntiles = (ntex + t.tile - 1) / t.tile;
@@ -286,7 +291,7 @@ int lsg_bake_create(lsg_scene* scene, const lsg_bake_object* objects, uint32_t n
     (void)hipGetDevice(&dev);
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) B.cus = prop.multiProcessorCount;
-    default_tuning(B.tuning);
+    default_tuning(B.tuning, B.ntex);
     if ((e = hipStreamSynchronize(nullptr)) != hipSuccess) return bail(hip_fail(e, "sync", __LINE__));
     *out = b;
     return LSG_OK;
@@ -313,7 +318,7 @@ int lsg_bake_set_tuning(lsg_bake* b, const lsg_bake_tuning* t)
         return fail(LSG_ERR_INVALID, "waves_per_block must be 2, 4 or 8");
     if (t->tile > 1024 || t->blocks_per_cu > 64 || t->lane_refill > 2) return fail(LSG_ERR_INVALID, "tuning out of range");
     b->impl.tuning = *t;
-    default_tuning(b->impl.tuning);
+    default_tuning(b->impl.tuning, b->impl.ntex);
     b->impl.graph_key.clear();   // invalidate a captured graph
     return LSG_OK;
 }
