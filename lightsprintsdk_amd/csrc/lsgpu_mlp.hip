@@ -76,9 +76,8 @@ __global__ void k_to_bf16(const float* __restrict__ x, uint16_t* __restrict__ y,
 // time, four waves per workgroup, workgroups striding over 64-row groups (the weights are
 // loaded into LDS once per workgroup).  The weights (transposed, BF16) and biases sit in LDS; each
 // wave's activations ping-pong between two LDS tiles.  The products are the same MFMA
-// calls in the same order as k_gemm_bf16's (same lane layout, same K steps), and bias,
-// ReLU and BF16 rounding are k_bias_act's, so the output equals the layered forward
-// pass bit for bit.
+// calls in the same order as k_gemm_bf16's (same lane layout, same K steps); bias, ReLU and
+// BF16 rounding come at the points the training step has them.
 // LDS rows are padded by 4 elements (8 bytes): 16 lanes reading 16 rows at one column
 // then hit 16 different bank pairs instead of one bank (row pitches of 64/128 bytes)
 constexpr int kPad = 4;

@@ -72,6 +72,32 @@ def test_plan_tunings_and_graph_replays_identical(gpu):
     assert not np.array_equal(moved, base)
 
 
+@pytest.mark.parametrize("size", [1, 2, 24])
+@pytest.mark.parametrize("scene,quality", [("room", 65), ("room", 200), ("field", 65), ("field", 200)])
+def test_plan_handouts_and_queues(gpu, scene, quality, size):
+    """Closed scenes (a wave waits for all of a handout) and open ones (it does not), with fewer
+    tiles than queues and than waves: refilled lanes sum the same rays in another order (at most
+    quality + light rays roundings of 2^-24 each), and every launch shape gives the same bits."""
+    from lightsprintsdk_amd import bake as B
+    sc = (S.box_room(seed=6, n_boxes=3, target_tris=600, lightmap_size=24) if scene == "room"
+          else S.object_field(seed=6, n_objects=3, target_tris=600, lightmap_range=(24, 24), area=10.0))
+    for ob in sc.objects:
+        ob.width = ob.height = size
+    plan = B.BakePlan(sc, B.GatherParams(quality=quality, ray_length_min=S.minimal_safe_distance(sc.verts), seed=5))
+
+    def run(**t):
+        plan.set_tuning(**t)
+        plan.run(first=True, graph=False, filtering=False)
+        return plan.rgba().copy()
+    base = run()
+    for t in (dict(xcd_queues=1), dict(tile=3, waves_per_block=2), dict(tile=1, waves_per_block=8, blocks_per_cu=1)):
+        np.testing.assert_array_equal(run(**t).view(np.uint32), base.view(np.uint32), err_msg=str(t))
+    plain = run(lane_refill=1)
+    np.testing.assert_array_equal(base[:, 3].view(np.uint32), plain[:, 3].view(np.uint32))
+    np.testing.assert_allclose(base[:, :3], plain[:, :3], rtol=2 * quality * 2.0 ** -24, atol=1e-7)
+    plan.close()
+
+
 def test_autotune_picks_a_candidate(gpu, tmp_path):
     from lightsprintsdk_amd import bake as B
     sc = _scene()
