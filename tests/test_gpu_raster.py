@@ -202,20 +202,28 @@ def test_gpu_raster_deterministic_and_ids(gpu):
     assert set(np.unique(a[1]["triangle"])) <= set(ids)
 
 
-def test_gpu_plan_rasterises_objects_together(gpu):
+@pytest.mark.parametrize("groups", [1, 2])
+def test_gpu_plan_rasterises_objects_together(gpu, groups):
     """A bake plan's texel and piece lists (all objects rasterised together) are the lists of
     its objects rasterised one at a time, one after another: odd map sizes, an object without
-    triangles, one whose triangles cover nothing, one with a single texel."""
+    triangles, one whose triangles cover nothing, one with a single texel.  With two maps of
+    6000^2 crossed by a sliver (36M candidates each, few texels) the objects do not fit one
+    group of 2^26 candidates."""
     from lightsprintsdk_amd import bake as B
     from lightsprintsdk_amd import native as N
     rng = np.random.default_rng(4)
     sizes = [(33, 17), (8, 8), (1, 1), (64, 65), (5, 3)]
     counts = [40, 0, 3, 120, 6]
+    if groups == 2:
+        sizes, counts = [(6000, 6000), (9, 7), (8, 8), (6000, 6000), (5, 3)], [1, 20, 0, 1, 6]
     nt = sum(counts)
     verts = rng.uniform(-1, 1, (3 * nt, 3)).astype(np.float32)
     idx = np.arange(3 * nt, dtype=np.uint32).reshape(-1, 3)
     uv = rng.uniform(0, 1, (nt, 6)).astype(np.float32)
     uv[nt - 6:] = 2.0                                     # the last object's cover nothing
+    if groups == 2:
+        uv[0] = (0, 0, 1, 1, 1, 0.9998)
+        uv[21] = (0, 1, 1, 0, 0.9997, 0)
     ids = rng.permutation(nt).astype(np.uint32)
     gs = B.GatherScene(verts, idx, np.zeros_like(verts), np.full(nt, 3, np.uint8), np.zeros((nt, 8), np.float32), [])
     objs = (N.BakeObject * len(sizes))()
