@@ -206,14 +206,16 @@ __device__ inline bool trace_begin(TraceState& S, const ColliderView& c, const f
 }
 
 // One triangle against the ray: slot p with plane pl and record (sv, ev, mt) (all zero where
-// the caller has not read it: LATE reads it here, once the plane test passes).
+// the caller has not read it: LATE reads it here, once the plane test passes).  True when it
+// is an accepted hit that ends the search (the ray's state alone does not tell: S.ref is kDone
+// on every ray's last leaf too, and S.best starts as the clipped range).
 template <bool WIDE, bool LATE, class Filter>
-__device__ inline void test_triangle(TraceState& S, const Filter& flt, const ColliderView& c, uint32_t p, const float4 pl, float4 sv,
+__device__ inline bool test_triangle(TraceState& S, const Filter& flt, const ColliderView& c, uint32_t p, const float4 pl, float4 sv,
                                      float4 ev, uint4 mt)
 {
     float ndd;
     const float t = plane_distance(pl, S.o, S.d, ndd);
-    if (!(t >= S.lo && t <= S.bound)) return;
+    if (!(t >= S.lo && t <= S.bound)) return false;
     if constexpr (LATE) {
         // the whole record in one round trip
         sv = load_at<WIDE, float4>(c.rest, p, 48u, 0u); ev = load_at<WIDE, float4>(c.rest, p, 48u, 16u);
@@ -221,13 +223,15 @@ __device__ inline void test_triangle(TraceState& S, const Filter& flt, const Col
         __builtin_amdgcn_sched_barrier(0);
     }
     float u, v;
-    if (!srlnp_hit(sv, ev, mt.z, S.o, S.d, t, u, v)) return;
+    if (!srlnp_hit(sv, ev, mt.z, S.o, S.d, t, u, v)) return false;
     // a tie goes to the lower triangle index
-    if (t == S.best && S.slot != kNoSlot && mt.x >= load_at<WIDE, uint32_t>(c.rest, S.slot, 48u, 32u)) return;
-    if (!flt.accept(mt.x, ndd < 0, t, u, v)) return;
+    if (t == S.best && S.slot != kNoSlot && mt.x >= load_at<WIDE, uint32_t>(c.rest, S.slot, 48u, 32u)) return false;
+    if (!flt.accept(mt.x, ndd < 0, t, u, v)) return false;
     S.best = t; S.slot = p;
     S.bound = flt.clamp(t);
-    if (flt.done(t)) S.ref = kDone;
+    if (!flt.done(t)) return false;
+    S.ref = kDone;
+    return true;
 }
 
 // Loop shape: "while-while" with speculative traversal (Aila & Laine, HPG 2009).
@@ -273,14 +277,13 @@ __device__ inline bool trace_run(TraceState& S, const Filter& flt, const Collide
                     const uint4 mt0 = load_at<WIDE, uint4>(c.rest, p, 48u, 32u), mt1 = load_at<WIDE, uint4>(c.rest, q, 48u, 32u);
                     __builtin_amdgcn_sched_barrier(0);
                     if (STATS) ntest += q - p + 1;
-                    test_triangle<WIDE, false>(S, flt, c, p, pl0, sv0, ev0, mt0);
-                    if (q != p) test_triangle<WIDE, false>(S, flt, c, q, pl1, sv1, ev1, mt1);
+                    if (test_triangle<WIDE, false>(S, flt, c, p, pl0, sv0, ev0, mt0)) break;
+                    if (q != p && test_triangle<WIDE, false>(S, flt, c, q, pl1, sv1, ev1, mt1)) break;
                 }
             } else {
                 for (uint32_t p = st; p < end; p++) {
                     if (STATS) ntest++;
-                    test_triangle<WIDE, true>(S, flt, c, p, load_at<WIDE, float4>(c.plane, p, 16u, 0u), zero, zero, make_uint4(0u, 0u, 0u, 0u));
-                    if (S.ref == kDone && flt.done(S.best)) break;
+                    if (test_triangle<WIDE, true>(S, flt, c, p, load_at<WIDE, float4>(c.plane, p, 16u, 0u), zero, zero, make_uint4(0u, 0u, 0u, 0u))) break;
                 }
             }
             if (S.ref < 0) { S.leaf = S.ref; S.ref = stk.pop(S.top); }
