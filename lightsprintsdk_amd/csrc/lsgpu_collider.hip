@@ -761,7 +761,8 @@ static int load_from_file(const float* verts, uint32_t nv, const uint32_t* idx, 
     if (st) return st;
     if ((want_leaf && h.leaf != want_leaf) || h.flags != want_flags)
         return fail(LSG_ERR_INVALID, "tree file %s: built with leaf size %u flags %u", path, h.leaf, h.flags);
-    if (!stack_size_for_depth(h.depth) || h.stack_need + 1 > (uint32_t)stack_size_for_depth(h.depth))
+    // (the header is outside the checksum: any value may stand there)
+    if (h.stack_need >= (uint32_t)stack_size_for_depth(h.depth))
         return fail(LSG_ERR_INVALID, "tree file %s: depth %u does not fit the traversal stack", path, h.depth);
     const uint32_t* order = (const uint32_t*)payload.data();
     for (uint32_t i = 0; i < h.nvalid; i++)

@@ -47,9 +47,7 @@ bool device_ready()
 
 int stack_size_for_depth(uint32_t depth)
 {
-    if (depth + 1 <= 32) return 32;
-    if (depth + 1 <= 64) return 64;
-    return 0;
+    return depth <= 31 ? 32 : (depth <= 63 ? 64 : 0);
 }
 
 } // namespace lsg

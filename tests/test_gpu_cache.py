@@ -136,6 +136,32 @@ def test_gpu_cache_walks_the_stored_tree(gpu, tmp_path, what):
         RRCollider.load(V, I, path)
 
 
+@pytest.mark.parametrize("field,value", [("stack_need", 0xFFFFFFFF), ("stack_need", 32), ("stack_need", -1),
+                                         ("depth", 0xFFFFFFFF), ("depth", 64)])
+def test_gpu_cache_stack_claims(gpu, tmp_path, field, value):
+    """The header's depth and stack entries are outside the checksum: a file that states more than
+    the traversal stack holds, however large the number, or fewer entries than its tree needs (-1:
+    one less) is refused before it reaches the GPU."""
+    from lightsprintsdk_amd import native as N
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = S.icosphere(8, seed=2)
+    a = RRCollider.create(V, I)
+    path = str(tmp_path / "t.lsgbvh")
+    a.save(path)
+    info = a.info()
+    a.close()
+    assert info.depth <= 31
+    raw = bytearray(open(path, "rb").read())
+    at = dict(depth=76, stack_need=80)[field]
+    assert int.from_bytes(raw[at:at + 4], "little") == getattr(info, field)
+    if value == -1:
+        value = info.stack_need - 1
+    raw[at:at + 4] = value.to_bytes(4, "little")
+    open(path, "wb").write(raw)
+    with pytest.raises(N.LsgError, match="stack"):
+        RRCollider.load(V, I, path)
+
+
 def test_gpu_cache_small_trees_and_star(gpu, tmp_path):
     from lightsprintsdk_amd.collider import RRCollider
     v = np.float32([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]])
