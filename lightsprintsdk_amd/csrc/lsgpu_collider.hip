@@ -645,7 +645,7 @@ static int load_tree(ColliderImpl& C, const float* verts, uint32_t nv, const uin
 {
     auto t0 = std::chrono::steady_clock::now();
     int st;
-    C.ntri = nt; C.nverts = nv; C.leaf = h.leaf;
+    C.ntri = nt; C.nverts = nv; C.leaf = h.leaf; C.flags = h.flags;
     memcpy(C.bmin, h.bmin, sizeof C.bmin); memcpy(C.bmax, h.bmax, sizeof C.bmax); C.margin = h.margin;
     if ((st = dalloc(&C.d_verts, 3 * (size_t)nv, &C.bytes))) return st;
     if ((st = dalloc(&C.d_idx, 3 * (size_t)nt, &C.bytes))) return st;

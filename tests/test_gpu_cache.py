@@ -162,6 +162,23 @@ def test_gpu_cache_stack_claims(gpu, tmp_path, field, value):
         RRCollider.load(V, I, path)
 
 
+@pytest.mark.parametrize("lbvh_only", [False, True])
+def test_gpu_cache_saves_a_loaded_tree(gpu, tmp_path, lbvh_only):
+    """A loaded tree saved again is the file it came from, byte for byte, whichever tree it is."""
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = S.icosphere(16, seed=3)
+    a = RRCollider.create(V, I, lbvh_only=lbvh_only)
+    p, q = str(tmp_path / "a.lsgbvh"), str(tmp_path / "b.lsgbvh")
+    a.save(p)
+    b = RRCollider.load(V, I, p)
+    b.save(q)
+    assert open(p, "rb").read() == open(q, "rb").read()
+    c = RRCollider.load(V, I, q)
+    _same_tree(a, c, S.random_rays(V, 5_000, seed=8))
+    for col in (a, b, c):
+        col.close()
+
+
 def test_gpu_cache_small_trees_and_star(gpu, tmp_path):
     from lightsprintsdk_amd.collider import RRCollider
     v = np.float32([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]])
