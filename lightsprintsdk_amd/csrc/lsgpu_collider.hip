@@ -440,7 +440,7 @@ static void launch_trace(const ColliderImpl& C, int stack, const float4* ro, con
         k_trace_closest<64><<<nb, 256, 0, s>>>(C.view(), ro, rd, n, hits, front, planes, q, per_wave);
 }
 
-// BVH2 -> BVH4, on the host after the GPU build.  Every BVH4 node starts from one BVH2
+// A built BVH2 becomes a BVH4 (collapse4_device).  Every BVH4 node starts from one BVH2
 // node's two children and opens the inner child of largest surface area, up to four
 // children, while the traversal stack stays bounded: a BVH2 subtree of height H needs
 // at most H stack entries, so with P entries already on the stack a node may take the
@@ -783,15 +783,27 @@ static int save_to_file(const lsg_collider* c, const char* path, uint32_t flags,
     const ColliderImpl& C = c->impl;
     TreeFileHeader h;
     memset(&h, 0, sizeof h);
+    auto bytes = [&](uint32_t nnodes4) { return 4ull * C.nvalid + sizeof(Node) * (uint64_t)C.nnodes + sizeof(Node4) * (uint64_t)nnodes4; };
+    if (sizeof h + bytes(C.nnodes4) < min_bytes) return LSG_OK;    // small trees build faster than a file loads
+    // the file holds the 4-wide tree in binary32: the BVH2 is collapsed again, and the header
+    // states what that gave (a loaded tree may have been collapsed in another way)
+    ColliderImpl again = C;
+    Node4* n4 = nullptr;
+    if (C.nnodes4)
+        if (int st = collapse4_device(again, (uint32_t)stack_size_for_depth(C.depth) - 1, &n4)) return st;
     memcpy(h.magic, kTreeMagic, 8);
     h.version = LSG_TREE_VERSION; h.header_bytes = sizeof h;
     h.nverts = C.nverts; h.ntri = C.ntri; h.leaf = C.leaf; h.flags = flags; h.nvalid = C.nvalid;
-    h.nnodes = C.nnodes; h.nnodes4 = C.nnodes4; h.depth = C.depth; h.stack_need = C.stack_need;
-    h.root = C.root; h.root4 = C.root4;
+    h.nnodes = C.nnodes; h.nnodes4 = again.nnodes4; h.depth = C.depth; h.stack_need = again.stack_need;
+    h.root = C.root; h.root4 = again.root4;
     memcpy(h.bmin, C.bmin, sizeof h.bmin); memcpy(h.bmax, C.bmax, sizeof h.bmax); h.margin = C.margin;
-    h.payload_bytes = 4ull * C.nvalid + sizeof(Node) * (uint64_t)C.nnodes + sizeof(Node4) * (uint64_t)C.nnodes4;
-    if (sizeof h + h.payload_bytes < min_bytes) return LSG_OK;    // small trees build faster than a file loads
+    h.payload_bytes = bytes(h.nnodes4);
     std::vector<uint8_t> payload(h.payload_bytes);
+    if (n4) {
+        const hipError_t e = hipMemcpy(payload.data() + bytes(0), n4, sizeof(Node4) * (size_t)h.nnodes4, hipMemcpyDeviceToHost);
+        dfree(n4);
+        LSG_HIP(e);
+    }
     if (C.nvalid) {
         std::vector<TriRest> m(C.nvalid);
         LSG_HIP(hipMemcpy(m.data(), C.d_rest, sizeof(TriRest) * (size_t)C.nvalid, hipMemcpyDeviceToHost));
@@ -799,18 +811,6 @@ static int save_to_file(const lsg_collider* c, const char* path, uint32_t flags,
         for (uint32_t i = 0; i < C.nvalid; i++) order[i] = m[i].meta.x;
     }
     if (C.nnodes) LSG_HIP(hipMemcpy(payload.data() + 4ull * C.nvalid, C.d_nodes, sizeof(Node) * (size_t)C.nnodes, hipMemcpyDeviceToHost));
-    if (C.nnodes4) {
-        // the file holds the 4-wide tree in binary32, which the collapse gives again
-        ColliderImpl again = C;
-        Node4* n4 = nullptr;
-        if (int st = collapse4_device(again, (uint32_t)stack_size_for_depth(C.depth) - 1, &n4)) return st;
-        const hipError_t e = again.nnodes4 == C.nnodes4
-                                 ? hipMemcpy(payload.data() + 4ull * C.nvalid + sizeof(Node) * (size_t)C.nnodes, n4,
-                                             sizeof(Node4) * (size_t)C.nnodes4, hipMemcpyDeviceToHost)
-                                 : hipErrorUnknown;
-        dfree(n4);
-        if (e != hipSuccess) return hip_fail(e, "4-wide tree", __LINE__);
-    }
     // the mesh hash from the device copy of the mesh
     std::vector<float> v(3 * (size_t)C.nverts);
     std::vector<uint32_t> ix(3 * (size_t)C.ntri);

@@ -179,6 +179,42 @@ def test_gpu_cache_saves_a_loaded_tree(gpu, tmp_path, lbvh_only):
         col.close()
 
 
+def test_gpu_cache_saves_another_collapse(gpu, tmp_path):
+    """A file whose 4-wide tree is a sound one, but not the one this build collapses to (its nodes all of
+    two children: the BVH2 itself), loads, and saving it states the tree that is written."""
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = S.icosphere(8, seed=2)
+    a = RRCollider.create(V, I)
+    p, q = str(tmp_path / "a.lsgbvh"), str(tmp_path / "b.lsgbvh")
+    a.save(p)
+    raw = bytearray(open(p, "rb").read())
+    info, head_bytes = a.info(), int.from_bytes(raw[12:16], "little")
+    n, at = info.num_nodes, head_bytes + 4 * info.num_valid
+    nodes = np.frombuffer(bytes(raw[at:at + 64 * n]), np.float32).reshape(n, 16)
+    wide = np.zeros((n, 8, 4), np.float32)
+    wide[:, :6, 0], wide[:, :6, 1] = nodes[:, :6], nodes[:, 6:12]
+    refs = np.full((n, 4), 0x7FFFFFFE, np.int32)
+    refs[:, :2] = nodes[:, 12:14].view(np.int32)
+    wide[:, 6] = refs.view(np.float32)
+    payload = bytes(raw[head_bytes:at + 64 * n]) + wide.tobytes()
+    raw = raw[:head_bytes] + payload
+    raw[72:76] = n.to_bytes(4, "little")                       # 4-wide nodes
+    raw[80:84] = info.depth.to_bytes(4, "little")              # stack entries: one a level at most
+    raw[40:48] = _payload_sum(payload).to_bytes(8, "little")
+    raw[120:128] = len(payload).to_bytes(8, "little")
+    open(p, "wb").write(raw)
+    b = RRCollider.load(V, I, p)
+    assert b.info().num_nodes4 == n != info.num_nodes4
+    R = S.random_rays(V, 5_000, seed=8)
+    ha, hb = a.intersect_batch(R), b.intersect_batch(R)
+    np.testing.assert_array_equal(ha[0].view(np.uint8), hb[0].view(np.uint8))
+    b.save(q)
+    c = RRCollider.load(V, I, q)
+    _same_tree(a, c, R)
+    for col in (a, b, c):
+        col.close()
+
+
 def test_gpu_cache_small_trees_and_star(gpu, tmp_path):
     from lightsprintsdk_amd.collider import RRCollider
     v = np.float32([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]])
