@@ -752,6 +752,30 @@ static bool tree4_walkable(const Node4* nodes, uint32_t n4, int32_t root4, uint3
     return true;
 }
 
+// whether a stored BVH2 is one that saving it again can collapse: its root and all refs within the
+// tree and the triangles, and no node with two parents or above the root, so that what hangs
+// from the root is a tree.  (The LBVH's order is kept where it was not rebuilt, so parents need not
+// come before their children.  Its height is checked by the collapse.)
+static bool tree2_walkable(const Node* nodes, uint32_t n, int32_t root, uint32_t nvalid)
+{
+    if (root < 0 || (uint32_t)root >= n) return false;
+    std::vector<bool> has_parent(n, false);
+    has_parent[root] = true;
+    for (uint32_t i = 0; i < n; i++) {
+        int32_t r[2];
+        memcpy(r, &nodes[i].q3, sizeof r);
+        for (int32_t c : r) {
+            if (c < 0) {
+                if ((uint64_t)leaf_start(c) + leaf_count(c) > nvalid) return false;
+                continue;
+            }
+            if ((uint32_t)c >= n || has_parent[c]) return false;
+            has_parent[c] = true;
+        }
+    }
+    return true;
+}
+
 static int load_from_file(const float* verts, uint32_t nv, const uint32_t* idx, uint32_t nt, const uint8_t hash[20], const char* path,
                           uint32_t want_leaf, uint32_t want_flags, lsg_collider** out)
 {
@@ -771,6 +795,8 @@ static int load_from_file(const float* verts, uint32_t nv, const uint32_t* idx, 
     const Node4* nodes4 = (const Node4*)(payload.data() + 4ull * h.nvalid + sizeof(Node) * (uint64_t)h.nnodes);
     if (!tree4_walkable(nodes4, h.nnodes4, h.root4, h.nvalid, h.stack_need))
         return fail(LSG_ERR_INVALID, "tree file %s: its 4-wide tree has refs out of range or needs more stack than stated", path);
+    if (h.nnodes4 && !tree2_walkable(nodes, h.nnodes, h.root, h.nvalid))
+        return fail(LSG_ERR_INVALID, "tree file %s: its 2-wide tree has refs out of range or is no tree", path);
     lsg_collider* c = new (std::nothrow) lsg_collider;
     if (!c) return fail(LSG_ERR_OOM, "lsg_collider_load: host allocation failed");
     if ((st = load_tree(c->impl, verts, nv, idx, nt, h, order, nodes, nodes4))) { free_impl(c->impl); delete c; return st; }

@@ -215,6 +215,41 @@ def test_gpu_cache_saves_another_collapse(gpu, tmp_path):
         col.close()
 
 
+@pytest.mark.parametrize("what", ["cycle", "root_ref", "two_parents", "node_past_end", "leaf_past_end", "root", "root_leaf"])
+def test_gpu_cache_checks_the_stored_bvh2(gpu, tmp_path, what):
+    """Saving a loaded tree walks its BVH2 on the GPU: a file with the right checksum whose BVH2 could
+    lead out of its arrays, or is no tree, is refused before it reaches the GPU."""
+    from lightsprintsdk_amd import native as N
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = S.icosphere(8, seed=2)
+    a = RRCollider.create(V, I)
+    path = str(tmp_path / "t.lsgbvh")
+    a.save(path)
+    info = a.info()
+    a.close()
+    raw = bytearray(open(path, "rb").read())
+    head_bytes = int.from_bytes(raw[12:16], "little")
+    n, nodes = info.num_nodes, head_bytes + 4 * info.num_valid
+    assert info.root_ref == 0
+    ref = lambda i, k: nodes + 64 * i + 48 + 4 * k
+
+    def inner(i):                                    # an inner child ref of node i, or None
+        for k in range(2):
+            c = int.from_bytes(raw[ref(i, k):ref(i, k) + 4], "little", signed=True)
+            if c >= 0:
+                return ref(i, k), c
+    deep = next(i for i in range(n - 1, 0, -1) if inner(i))
+    at, child = inner(deep)
+    other = next(inner(i)[1] for i in range(n) if inner(i) and inner(i)[1] != child)
+    where, bad = dict(cycle=(at, deep), root_ref=(at, 0), two_parents=(at, other), node_past_end=(at, n),
+                      leaf_past_end=(at, -(1 << 31) | (len(I) << 4)), root=(84, n), root_leaf=(84, -(1 << 31)))[what]
+    raw[where:where + 4] = int(bad & 0xFFFFFFFF).to_bytes(4, "little")
+    raw[40:48] = _payload_sum(bytes(raw[head_bytes:])).to_bytes(8, "little")
+    open(path, "wb").write(raw)
+    with pytest.raises(N.LsgError, match="2-wide tree"):
+        RRCollider.load(V, I, path)
+
+
 def test_gpu_cache_small_trees_and_star(gpu, tmp_path):
     from lightsprintsdk_amd.collider import RRCollider
     v = np.float32([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]])
