@@ -168,12 +168,12 @@ struct BlurKernels { float4 k[kFuse]; };
 __global__ __launch_bounds__(kBlurThreads) void k_blur_tiles(const FilterMap* __restrict__ maps, uint32_t nmaps, const float4* __restrict__ rgba,
                                                              const float4* __restrict__ src, float4* __restrict__ dst, uint8_t* __restrict__ bf,
                                                              BlurKernels kernels, uint32_t npass, int first, int last,
-                                                             float4* __restrict__ out, uint32_t* __restrict__ mark, int wrap)
+                                                             float4* __restrict__ out, uint32_t* __restrict__ mark, int wrap, uint32_t tile0)
 {
     __shared__ float4 val[kBlurSide * kBlurSide];
     __shared__ uint8_t fl[kBlurSide * kBlurSide];                 // blur flags
     __shared__ uint8_t tf[(kBlurSide + 2) * (kBlurSide + 2)];     // texel flags, one texel further
-    const uint32_t tid = threadIdx.x, t = blockIdx.x;
+    const uint32_t tid = threadIdx.x, t = tile0 + blockIdx.x;
     uint32_t lo = 0, hi = nmaps;
     while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (maps[mid].tfirst <= t) lo = mid; else hi = mid; }
     const FilterMap M = maps[lo];
@@ -802,6 +802,7 @@ __global__ __launch_bounds__(64) void k_seam_pass(const FilterMap* __restrict__ 
 
 static inline unsigned nblk(uint32_t n) { return (n + 255) / 256; }
 
+constexpr uint32_t kBlurTiles = 1u << 22;             // of a launch: its threads stay below 2^32
 constexpr uint32_t kGrowBlocks = 512;                 // two workgroups of k_grow_tiles per CU
 constexpr uint32_t kGrowChunk = 2 * kTileSteps;       // steps between the host's looks
 
@@ -835,7 +836,9 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
             uint32_t npass = 0;
             while (npass < kFuse && sigma2sum > 0) K.k[npass++] = next_kernel();
             last = !(sigma2sum > 0);
-            k_blur_tiles<<<S.tiles, kBlurThreads, 0, s>>>(d_maps, nmaps, rgba, src, dst, S.flags, K, npass, first, last, S.c, mark, fp.wrap);
+            for (uint32_t t = 0; t < S.tiles; t += std::min(kBlurTiles, S.tiles - t))
+                k_blur_tiles<<<std::min(kBlurTiles, S.tiles - t), kBlurThreads, 0, s>>>(d_maps, nmaps, rgba, src, dst, S.flags, K, npass, first, last, S.c,
+                                                                                        mark, fp.wrap, t);
             std::swap(src, dst);
             first = false;
         } while (!last);

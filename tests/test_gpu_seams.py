@@ -166,6 +166,46 @@ def test_gpu_grow_tiles_vs_oracle(gpu, oracle, spread):
         plan.close()
 
 
+def _filter_plan(images, sigma, spread):
+    """The filter chain over maps [n, h, w, 4] of one size, as one plan: (rgba, rgbf)."""
+    import ctypes
+    from lightsprintsdk_amd import bake as B
+    from lightsprintsdk_amd import native as N
+    from lightsprintsdk_amd.collider import DeviceBuffer
+    n, h, w = images.shape[:3]
+    maps = (N.Lightmap * n)()
+    m = np.frombuffer(maps, np.uint32).reshape(n, 4)
+    m[:, 0] = m[:, 3] = np.arange(n) * (h * w)
+    m[:, 1], m[:, 2] = w, h
+    rgba, rgbf = DeviceBuffer.from_array(images), DeviceBuffer(12 * n * h * w)
+    plan = ctypes.c_void_p()
+    N.check(N.lib().lsg_filter_plan_create(maps, n, ctypes.byref(plan)), "lsg_filter_plan_create")
+    fp = B.FilterParams(smoothing_amount=sigma, spread_foreground=spread).c()
+    N.check(N.lib().lsg_filter_plan_run(plan, rgba.ptr, rgbf.ptr, ctypes.byref(fp), None), "lsg_filter_plan_run")
+    N.check(N.lib().lsg_synchronize(), "sync")
+    out = rgba.download(np.float32, images.shape), rgbf.download(np.float32, (n, h, w, 3))
+    N.lib().lsg_filter_plan_destroy(plan)
+    return out
+
+
+def _same_as_oracle(oracle, images, sigma, spread, distinct):
+    """images repeats its first `distinct` maps: the plan's results against the oracle's."""
+    rgba, rgbf = _filter_plan(images, sigma, spread)
+    for k in range(distinct):
+        ra, rf = oracle.filter_lightmap(images[k], sigma=sigma, spread=spread)
+        what = f"map {k} of {images.shape}, sigma {sigma}, spread {spread}"
+        assert (rgba[k::distinct].view(np.uint32) == ra.view(np.uint32)).all(), what
+        assert (rgbf[k::distinct].view(np.uint32) == rf.astype(np.float32).view(np.uint32)).all(), what
+
+
+def test_gpu_filter_more_maps_than_a_launch_holds(gpu, oracle):
+    """2^23 maps and some: a workgroup of 512 threads for each would pass 2^32 threads a launch."""
+    rng = np.random.default_rng(12)
+    images = rng.uniform(0.1, 1.0, (64, 1, 1, 4)).astype(np.float32)
+    images[:, 0, 0, 3] = rng.choice(np.float32([0.0, 0.001, 0.5, 1.0]), 64)
+    _same_as_oracle(oracle, np.tile(images, ((1 << 17) + 1, 1, 1, 1)), 1.0, 1000.0, 64)
+
+
 @pytest.mark.parametrize("wrap", [False, True])
 def test_gpu_seams_vs_oracle(gpu, oracle, wrap):
     rng = np.random.default_rng(7 + wrap)
