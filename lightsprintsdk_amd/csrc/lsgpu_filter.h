@@ -19,9 +19,9 @@ inline uint32_t map_tiles(uint32_t width, uint32_t height) { return ((width + kT
 struct FilterScratch {
     float4* a = nullptr; float4* b = nullptr; float4* c = nullptr;
     uint8_t* flags = nullptr;
-    uint32_t* changed = nullptr;   // [0] last step changed; [1] last step that filled a texel (wrap: [1..3] frontier sizes, [4..19] step log)
-    uint32_t* front[2] = {nullptr, nullptr};   // lightmapGrow: tile states in [0]; with wrap the frontiers (texel indices)
-    uint32_t* mark = nullptr;      // step at which a texel was filled; with wrap step + 1 at which it was queued, 0 = never
+    uint32_t* changed = nullptr;   // [0] last step changed; [1] last step that filled a texel (by frontiers: [1..3] their sizes, [4..19] step log)
+    uint32_t* front[2] = {nullptr, nullptr};   // lightmapGrow: tile states in [0]; or the frontiers (texel indices)
+    uint32_t* mark = nullptr;      // step at which a texel was filled; by frontiers step + 1 at which it was queued, 0 = never
     uint32_t tiles = 0;            // lightmapGrow tiles of the batch (at most one per texel)
     uint32_t* host_log = nullptr;  // pinned: two chunks of step logs read by the host
     hipEvent_t ev[2] = {nullptr, nullptr};

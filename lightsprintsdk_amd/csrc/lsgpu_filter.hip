@@ -389,22 +389,38 @@ __global__ __launch_bounds__(kTileThreads) void k_grow_tiles(const FilterMap* __
                     if (lane == 0) { fill0[r] = f; empty0[r] = e; }
                 }
                 __syncthreads();
-                // values of the filled texels next to an empty one; the others are never read
+                uint64_t filled = fill0[lane];
+                const uint64_t empty = empty0[lane];
+                const uint64_t tile = ((1ull << kTile) - 1ull) << kHalo;
+                const bool row = lane >= kHalo && lane < kHalo + kTile;
+                if (!__any(filled != 0) || !__any(row && (empty & tile))) {
+                    // nothing to fill, or to fill it from (the same in every wave)
+                    const uint64_t hf = __ballot(row && (filled & tile)), he = __ballot(row && (empty & tile));
+                    if (tid == 0) info[t] = (hf ? 1u : 0u) | (he ? 2u : 0u);
+                    __syncthreads();
+                    continue;
+                }
+                // values of the filled texels next to an empty one; the others are never read, nor are rows
+                // outside the map, which are not written (20,000 maps of 12 x 12: 386 -> 321 us)
+                float4 c[kRegion / kTileWaves];
 #pragma unroll
-                for (uint32_t r = wave; r < kRegion; r += kTileWaves) {
+                for (uint32_t j = 0; j < kRegion / kTileWaves; j++) {
+                    const uint32_t r = wave + j * kTileWaves;
                     uint64_t e = empty0[r];
                     if (r > 0) e |= empty0[r - 1];
                     if (r < kRegion - 1) e |= empty0[r + 1];
                     e |= (e << 1) | (e >> 1);
-                    float4 c = make_float4(0.f, 0.f, 0.f, kNever);
+                    c[j] = make_float4(0.f, 0.f, 0.f, kNever);
                     if ((e & fill0[r]) >> lane & 1u) {
-                        c = img[M.first + (uint32_t)(x + (y0 + (int)r) * w)];
-                        c.w = 0.f;
+                        c[j] = img[M.first + (uint32_t)(x + (y0 + (int)r) * w)];
+                        c[j].w = 0.f;
                     }
-                    val[r * kValPitch + lane] = c;
                 }
-                uint64_t filled = fill0[lane];
-                const uint64_t empty = empty0[lane];
+#pragma unroll
+                for (uint32_t j = 0; j < kRegion / kTileWaves; j++) {
+                    const int r = (int)(wave + j * kTileWaves);
+                    if (y0 + r >= 0 && y0 + r < h) val[r * kValPitch + lane] = c[j];
+                }
                 __syncthreads();
                 const uint64_t strip = ((1ull << kStrip) - 1ull) << (wave * kStrip);
                 for (uint32_t s = 1; s <= nsteps; s++) {
@@ -450,6 +466,7 @@ __global__ __launch_bounds__(kTileThreads) void k_grow_tiles(const FilterMap* __
                 // the stores)
                 for (uint32_t i = tid; i < kTile * kTile; i += kTileThreads) {
                     const uint32_t xc = kHalo + i % kTile, yc = kHalo + i / kTile;
+                    if (x0 + (int)xc >= w || y0 + (int)yc >= h) continue;
                     const float4 v = val[yc * kValPitch + xc];
                     if (v.w > 0.f && v.w < kNever) {
                         const uint32_t g = M.first + (uint32_t)((x0 + (int)xc) + (y0 + (int)yc) * w);
@@ -459,8 +476,6 @@ __global__ __launch_bounds__(kTileThreads) void k_grow_tiles(const FilterMap* __
                     }
                 }
                 if (wave == 0) {
-                    const uint64_t tile = ((1ull << kTile) - 1ull) << kHalo;
-                    const bool row = lane >= kHalo && lane < kHalo + kTile;
                     const uint64_t hf = __ballot(row && (filled & tile)), he = __ballot(row && (empty & ~filled & tile));
                     if (lane == 0) info[t] = (hf ? 1u : 0u) | (he ? 2u : 0u);
                 }
@@ -479,7 +494,7 @@ __global__ void k_grow_changed(const uint32_t* __restrict__ last_step, uint32_t 
     if (threadIdx.x == 0) changed[0] = *last_step == n ? 1u : 0u;
 }
 
-// lightmapGrow init (RRBuffer.cpp:889-893), for the wrapped form below
+// lightmapGrow init (RRBuffer.cpp:889-893), for the form by frontiers below
 __global__ __launch_bounds__(256) void k_grow_init(uint32_t total, const float4* __restrict__ img, float4* __restrict__ g)
 {
     const uint32_t t = blockIdx.x * 256 + threadIdx.x;
@@ -489,7 +504,7 @@ __global__ __launch_bounds__(256) void k_grow_init(uint32_t total, const float4*
 }
 
 // lightmapGrow by frontiers, for wrapped maps (their neighbours are flat texel numbers, not a
-// neighbourhood that tiles).  The reference's step (RRBuffer.cpp:897-947) changes exactly
+// neighbourhood that tiles) and maps that fill little of their tiles.  The reference's step (RRBuffer.cpp:897-947) changes exactly
 // the empty texels that have a filled neighbour in the previous state, and those are the
 // still-empty texels that count a texel filled one step earlier among their neighbours.
 // So each step visits only its frontier: every frontier texel's value is computed from
@@ -803,6 +818,16 @@ __global__ __launch_bounds__(64) void k_seam_pass(const FilterMap* __restrict__ 
 static inline unsigned nblk(uint32_t n) { return (n + 255) / 256; }
 
 constexpr uint32_t kBlurTiles = 1u << 22;             // of a launch: its threads stay below 2^32
+// A tile costs a workgroup a few us however few texels of it the map has; launches over texels cost by
+// texels and steps.  So batches of many tiles with few texels in them take the latter:
+// blur passes below kBlurTexels texels a tile, unless all tiles are resident at once (three passes, us,
+// tiles -> passes: 300,000 maps of 1 x 1 2380 -> 64, 20,000 of 8 x 8 248 -> 180, 4,000 of 1 x 512 665 -> 220;
+// but 20,000 of 16 x 16 391 -> 566, 100 of 4 x 4 29 -> 36);
+// lightmapGrow by frontiers below kGrowTexels, unless there are but 32 tiles a workgroup (with 30% of the
+// texels empty, and with 90%, which is where frontiers are slow: 100,000 of 4 x 4 500 -> 232 and 867 -> 829,
+// 4,000 of 1 x 512 669 -> 505 and 2098 -> 1828; but 100,000 of 6 x 6 618 -> 340 and 1242 -> 2445, 20,000 of 2 x 2
+// 141 -> 157).
+constexpr uint32_t kBlurTexels = 128, kFewBlurTiles = 1024, kGrowTexels = 33, kFewGrowTiles = 16384;
 constexpr uint32_t kGrowBlocks = 512;                 // two workgroups of k_grow_tiles per CU
 constexpr uint32_t kGrowChunk = 2 * kTileSteps;       // steps between the host's looks
 
@@ -820,7 +845,10 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
     float sigma = fp.smoothing_amount;
     if (sigma < 0) return fail(LSG_ERR_INVALID, "smoothing_amount < 0");
     uint32_t steps = (uint32_t)(fp.spread_foreground > 0 ? fp.spread_foreground : 0);
-    uint32_t* const mark = steps && !fp.wrap ? S.mark : nullptr;
+    const uint32_t per_tile = total / S.tiles;
+    const bool blur_tiles = !(seams && seams->nwith && sigma > 0) && (per_tile >= kBlurTexels || S.tiles <= kFewBlurTiles);
+    const bool grow_tiles = !fp.wrap && (per_tile >= kGrowTexels || S.tiles <= kFewGrowTiles);
+    uint32_t* const mark = steps && grow_tiles ? S.mark : nullptr;
     if (sigma > 10) sigma = 10;
     float sigma2sum = sigma * sigma;
     auto next_kernel = [&]() {
@@ -828,7 +856,7 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
         sigma2sum -= sigma2;
         return make_float4(1.f, expf(-0.5f / sigma2), expf(-1 / sigma2), expf(-2 / sigma2));
     };
-    if (!(seams && seams->nwith && sigma > 0)) {
+    if (blur_tiles) {
         float4* src = S.a; float4* dst = S.b;
         bool first = true, last;
         do {
@@ -843,23 +871,25 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
             first = false;
         } while (!last);
     } else {
-        // the seams are smoothed over the whole map after every pass
-        k_smooth_prepare<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, S.a, S.flags, fp.wrap);
-        float4* src = S.a; float4* dst = S.b;
-        while (sigma2sum > 0) {
-            const float4 kernel = next_kernel();
-            k_smooth_pass<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, src, dst, S.flags, kernel);
-            k_seam_pass<<<seams->nwith, 64, 0, s>>>(d_maps, *seams, dst);
-            std::swap(src, dst);
+        // a launch per pass (the seams are smoothed over the whole map after every one)
+        if (sigma > 0) {
+            k_smooth_prepare<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, S.a, S.flags, fp.wrap);
+            float4* src = S.a; float4* dst = S.b;
+            while (sigma2sum > 0) {
+                const float4 kernel = next_kernel();
+                k_smooth_pass<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, src, dst, S.flags, kernel);
+                if (seams && seams->nwith) k_seam_pass<<<seams->nwith, 64, 0, s>>>(d_maps, *seams, dst);
+                std::swap(src, dst);
+            }
+            k_smooth_finish<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, src);
         }
-        k_smooth_finish<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, src);
         // lightmapGrowForBilinearInterpolation
         k_grow_bilinear<<<nblk(total), 256, 0, s>>>(d_maps, nmaps, total, rgba, S.c, mark, fp.wrap);
     }
     // lightmapGrow(spread)
     const float4* g = nullptr;
     if (steps_used) *steps_used = 0;
-    if (steps && !fp.wrap) {
+    if (steps && grow_tiles) {
         // launches of 16 steps over the tiles, in place in S.c; S.changed[1] = the last step
         // that filled a texel.  A launch whose last step filled nothing is the end: the
         // reference stops at the first step that changes nothing (RRBuffer.cpp:948-949).
@@ -919,10 +949,10 @@ int filter_run(const FilterMap* d_maps, uint32_t nmaps, uint32_t total, float4* 
         };
         if (fixed_steps >= 0) {
             // graph-capturable form: a fixed number of steps, no host synchronisation,
-            // S.changed[0] = whether a frontier is still left after the last one
+            // S.changed[0] = whether a frontier is still left after the last one, and may be filled
             const uint32_t n = std::min<uint32_t>((uint32_t)fixed_steps, steps);
             for (uint32_t q = 0; q < n; q++) step(q);
-            k_front_changed<<<1, 64, 0, s>>>(S.changed + 1 + n % 3u, S.changed);
+            if (n < steps) k_front_changed<<<1, 64, 0, s>>>(S.changed + 1 + n % 3u, S.changed);
             if (steps_used) *steps_used = n;
         } else if (!S.host_log) {
             // scratch without pinned memory or events (the allocation-free entry point):

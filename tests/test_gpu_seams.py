@@ -206,6 +206,18 @@ def test_gpu_filter_more_maps_than_a_launch_holds(gpu, oracle):
     _same_as_oracle(oracle, np.tile(images, ((1 << 17) + 1, 1, 1, 1)), 1.0, 1000.0, 64)
 
 
+@pytest.mark.parametrize("sigma,spread", [(1.0, 1000.0), (0.0, 3.0), (1.0, 0.0), (2.5, 16.0)])
+@pytest.mark.parametrize("n,h,w", [(1024, 2, 3), (1025, 2, 3), (1100, 9, 14), (1100, 8, 16), (16384, 4, 8), (16385, 4, 8),
+                                   (16385, 3, 11), (4097, 128, 1)])
+def test_gpu_filter_many_small_maps_vs_oracle(gpu, oracle, n, h, w, sigma, spread):
+    """Both sides of the lines between tiles and separate passes: 1024 and 16384 tiles, 32
+    and 128 texels a tile."""
+    rng = np.random.default_rng(n + w)
+    images = np.stack([_random_map(rng, w, h, fill=0.4) for _ in range(7)])
+    print(f"{n} maps of {h} x {w}, sigma {sigma}, spread {spread}", flush=True)
+    _same_as_oracle(oracle, np.concatenate([images] * (n // 7) + [images[:n % 7]]), sigma, spread, 7)
+
+
 @pytest.mark.parametrize("wrap", [False, True])
 def test_gpu_seams_vs_oracle(gpu, oracle, wrap):
     rng = np.random.default_rng(7 + wrap)
