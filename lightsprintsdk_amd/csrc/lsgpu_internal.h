@@ -147,7 +147,7 @@ struct ColliderImpl {
     uint32_t nnodes4 = 0, stack_need = 0;   // BVH4 nodes; worst-case traversal stack entries
     int32_t root4 = 0;
     NodeT* d_nodes4 = nullptr;
-    float scale = 1.f;            // the nodes' power-of-two scale (node_scale)
+    float scale = 1.f;            // the nodes' power-of-two scale (pack4_device)
     int32_t root = 0;
     float bmin[3], bmax[3], margin = 0;
     float* d_verts = nullptr; uint32_t* d_idx = nullptr;

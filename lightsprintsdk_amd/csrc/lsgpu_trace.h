@@ -92,9 +92,13 @@ __device__ inline float vmin(float a, float b) { float r; asm("v_min_f32 %0, %1,
 // = -o * inverse direction: with c = origin * idir + noi per node and axis, a plane's
 // distance along the ray is one fma, distance from the origin * idir + c.  That differs from
 // (plane - o) * inverse direction by a few ulp of |o * inverse direction|, i.e. |o| * 2e-7 in
-// distance, while every child box is inflated by DELTA_BSP = max|coordinate| * 1e-5; culling
-// stays conservative and the hit, decided only by the triangle test, is unchanged.  near:
-// byte offsets of the axes' near planes in a node, a byte each.
+// distance, while every child box is inflated by DELTA_BSP = max|coordinate| * 1e-5: for origins up
+// to 50 times the largest coordinate away culling is conservative, and the hit, decided only by
+// the triangle test, is unchanged.  From farther away a ray that grazes a box may lose it, as it may with
+// binary32 planes; their outward rounding makes that rarer.  55,000 to 44,000 hits at edges and
+// corners of 600 triangles within [-1, 1]^3, lost from 1000 / 3000 / 10,000 away: binary32 planes
+// 12 / 33 / 83, these 0 / 9 / 64, and none from 5 to 400.  near: byte offsets of the axes' near planes in a
+// node, a byte each.
 struct RayBox { float3 idir, noi; uint32_t near; };
 
 __device__ inline float3 safe_inv(float3 d)
@@ -129,7 +133,8 @@ __device__ inline RayBox ray_box(const float3 o, const float3 d, float unscale)
 // texels), seven binary32 loads a visit -> these five binary16 ones: time 84.9 -> 71.0 ms, VALU
 // 78% -> 94% of issue, L1 tag lookups (one per distinct node and load) 46.7e9 -> 35.1e9, TA
 // busy 86% -> 79%; sun-and-sky bake over 132k triangles 24.2 -> 22.3 ms.  1M random rays
-// against 100k triangles, bound by latency at 20% active lanes, stay at 0.638 ms.
+// against 100k triangles, bound by latency at 20% active lanes, stayed at 0.638 ms (0.49 now, by their
+// launch shape).
 // Straight-line tests, pairs sorted as doubles, branch-free pushes and 32-bit offsets had
 // taken the gather's wave instructions from 49.7e9 to 39.7e9 (89.6 -> 84.9 ms).
 template <bool WIDE, bool ORDERED>

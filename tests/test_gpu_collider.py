@@ -319,6 +319,30 @@ def test_gpu_node_boxes_at_any_scale(gpu, oracle, scale, offset):
     _same_hits(g, gf, o, o)
 
 
+@pytest.mark.parametrize("away", [10.0, 45.0])
+def test_gpu_rays_from_far_away(gpu, oracle, away):
+    """Origins up to 45 times the largest coordinate away, aimed at edges and corners: the box tests'
+    rounding (|o| * 2e-7) stays within the boxes' inflation (1e-5 of the largest coordinate)."""
+    from lightsprintsdk_amd.collider import RRCollider
+    V, I = scenes.icosphere(14, seed=6)
+    rng = np.random.default_rng(int(away))
+    n = 9000
+    w = rng.uniform(size=(n, 3))
+    w[:3000, 0] = 1e-4                               # near an edge
+    w[3000:6000, :2] = 1e-4                          # near a corner
+    w /= w.sum(1, keepdims=True)
+    at = (V[I[rng.integers(0, len(I), n)]].astype(np.float64) * w[:, :, None]).sum(1)
+    d = rng.normal(size=(n, 3))
+    d[::3, 0] *= 1e-3
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    R = np.zeros((n, 8), np.float32)
+    R[:, 0:3], R[:, 4:7], R[:, 7] = at - away * np.abs(V).max() * d, d, np.inf
+    g, gf = RRCollider.create(V, I).intersect_batch(R)
+    o = oracle.intersect_linear_srlnp(V, I, R)
+    assert (o["tri"] >= 0).mean() > 0.9
+    _same_hits(g, gf, o, o)
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 63, 257, 16385, 16389, 262145, 400_001])
 def test_gpu_batch_sizes(gpu, oracle, n):
     """Every launch shape of a device batch (rays spread over few lanes of many waves, full waves,
@@ -340,4 +364,5 @@ def test_gpu_batch_sizes(gpu, oracle, n):
     np.testing.assert_array_equal(g["tri"][:n], ref["tri"])
     m = ref["tri"] >= 0
     np.testing.assert_array_equal(g["t"][:n][m], ref["t"][m])
+    np.testing.assert_array_equal(gf[:n][m].astype(np.int32), ref["front"][m])
     np.testing.assert_array_equal(g.view(np.int32).reshape(-1, 4)[n:], 7)
