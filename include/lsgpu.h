@@ -639,8 +639,8 @@ int  lsg_mlp_forward(lsg_mlp* mlp, const float* x, uint32_t n, float* y, void* s
  * only computes gradients (lsg_mlp_get_grads); *loss (host, optional) = mean loss */
 int  lsg_mlp_train_step(lsg_mlp* mlp, const float* x, const float* t, uint32_t n, float lambda, float lr,
                         float* loss, void* stream);
-/* C[MxN] = A[MxK] B[KxN] on the device through the MLP's MFMA GEMM (bf16 inputs,
- * row-major; M, N, K multiples of 16) -- exposed to verify the kernel */
+/* C[MxN] = A[MxK] B[KxN] on the device by the MFMA tiles that the MLP's kernels are made of (bf16
+ * inputs, row-major; M, N, K multiples of 16) -- exposed to verify their lane layout by itself */
 int  lsg_mlp_gemm_test(const uint16_t* a, const uint16_t* b, float* c, uint32_t m, uint32_t n, uint32_t k);
 
 /* the gather with its hemisphere and light parts written separately: parts =

@@ -35,13 +35,12 @@ __host__ __device__ inline uint16_t f2bf(float f)
 }
 __host__ __device__ inline float bf2f(uint16_t b) { uint32_t u = (uint32_t)b << 16; float f; memcpy(&f, &u, 4); return f; }
 
-// C[M x N] (fp32, row-major ldc) = sum_k A(m,k) B(k,n); A(m,k) = A[m*sAm + k*sAk],
-// B(k,n) = B[k*sBk + n*sBn] (bf16).  One wave per 16x16 tile, four waves per block.
-// Lane l feeds A row l%16 / B column l%16 with k = 4*(l/16)..+3 and receives
-// C rows 4*(l/16)..+3 of column l%16 (the 16x16x16 MFMA lane layout).
-__global__ __launch_bounds__(256) void k_gemm_bf16(const uint16_t* __restrict__ A, int sAm, int sAk,
-                                                   const uint16_t* __restrict__ B, int sBk, int sBn,
-                                                   float* __restrict__ C, int ldc, int M, int N, int K, int accumulate)
+// C[M x N] (fp32) = A[M x K] B[K x N] (bf16), all row-major: not on the network's path, but the same
+// MFMA calls in the lane layout and the K order that k_mlp_infer and k_mlp_train build on, by
+// themselves (lsg_mlp_gemm_test).  One wave per 16x16 tile, four waves per block.  Lane l feeds
+// A row l%16 / B column l%16 with k = 4*(l/16)..+3 and receives C rows 4*(l/16)..+3 of column l%16.
+__global__ __launch_bounds__(256) void k_gemm_bf16(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, float* __restrict__ C,
+                                                   int M, int N, int K)
 {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int tilesN = N / 16;
@@ -50,20 +49,17 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(const uint16_t* __restrict__ 
     const int tm = tile / tilesN, tn = tile % tilesN;
     const int r = lane & 15, kq = (lane >> 4) * 4;
     v4f acc = {0.f, 0.f, 0.f, 0.f};
-    const uint16_t* Ar = A + (size_t)(tm * 16 + r) * sAm;
-    const uint16_t* Bc = B + (size_t)(tn * 16 + r) * sBn;
+    const uint16_t* Ar = A + (size_t)(tm * 16 + r) * K;
+    const uint16_t* Bc = B + tn * 16 + r;
     for (int k0 = 0; k0 < K; k0 += 16) {
         v4s a, b;
         for (int i = 0; i < 4; i++) {
-            a[i] = (short)Ar[(size_t)(k0 + kq + i) * sAk];
-            b[i] = (short)Bc[(size_t)(k0 + kq + i) * sBk];
+            a[i] = (short)Ar[k0 + kq + i];
+            b[i] = (short)Bc[(size_t)(k0 + kq + i) * N];
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
     }
-    for (int i = 0; i < 4; i++) {
-        float* c = C + (size_t)(tm * 16 + kq + i) * ldc + tn * 16 + r;
-        *c = accumulate ? *c + acc[i] : acc[i];
-    }
+    for (int i = 0; i < 4; i++) C[(size_t)(tm * 16 + kq + i) * N + tn * 16 + r] = acc[i];
 }
 
 __global__ void k_to_bf16(const float* __restrict__ x, uint16_t* __restrict__ y, uint32_t n)
@@ -421,14 +417,6 @@ struct MlpImpl {
     }
 };
 
-static int gemm(const uint16_t* A, int sAm, int sAk, const uint16_t* B, int sBk, int sBn, float* C, int ldc, int M, int N, int K,
-                int acc, hipStream_t s)
-{
-    const int tiles = (M / 16) * (N / 16);
-    k_gemm_bf16<<<(tiles + 3) / 4, 256, 0, s>>>(A, sAm, sAk, B, sBk, sBn, C, ldc, M, N, K, acc);
-    return LSG_OK;
-}
-
 } // namespace lsg
 
 struct lsg_mlp { lsg::MlpImpl impl; };
@@ -552,12 +540,12 @@ int lsg_mlp_get_grads(const lsg_mlp* m, float* grads)
     return LSG_OK;
 }
 
-// debugging/verification hook: C[MxN] = A[MxK] B[KxN] with bf16 row-major inputs on
-// the device, through the same MFMA kernel (M, N, K multiples of 16)
+// verification hook: C[MxN] = A[MxK] B[KxN] with bf16 row-major inputs on the device, by
+// k_gemm_bf16 (M, N, K multiples of 16)
 int lsg_mlp_gemm_test(const uint16_t* A, const uint16_t* B, float* C, uint32_t M, uint32_t N, uint32_t K)
 {
     if (!A || !B || !C || !M || !N || !K || M % 16 || N % 16 || K % 16) return fail(LSG_ERR_INVALID, "gemm_test: bad shape");
-    gemm(A, (int)K, 1, B, (int)N, 1, C, (int)N, (int)M, (int)N, (int)K, 0, nullptr);
+    k_gemm_bf16<<<(unsigned)((uint64_t)(M / 16) * (N / 16) + 3) / 4, 256>>>(A, B, C, (int)M, (int)N, (int)K);
     LSG_HIP(hipGetLastError());
     LSG_HIP(hipDeviceSynchronize());
     return LSG_OK;
